@@ -170,19 +170,19 @@ int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
  * token-major activations as stored.  r, when not NULL, is the residual of a
  * fused add: one fp32 rounding of the accumulated product plus r.  Any
  * shape; bf16 / fp16 (fp32 accumulation) or fp32; every tensor shares
- * `dtype`; pointers aligned to the element size.  Shapes on the 256 x 256
- * grid of 2-byte types (zk_gemm_path) run the MFMA pipeline, the rest a
- * masked 128 x 128 kernel. */
+ * `dtype`; pointers aligned to the element size.  2-byte products run the
+ * MFMA tile (256 x 256 down to 64 x 64) with the least estimated time; fp32
+ * and operands that are not 16-byte aligned run a masked 128 x 128 kernel. */
 int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
             int b_kmajor, void* c, int64_t ldc, const void* r, int64_t ldr, int64_t M,
             int64_t N, int64_t K, int dtype, zk_stream_t stream);
 
-/* Which kernel zk_gemm runs for a launch with 16-byte aligned pointers
- * (host-only, no GPU call): ZK_GEMM_TILED -- 2-byte type, M and N multiples
+/* Whether a launch with 16-byte aligned pointers lies on the grid of the
+ * 256 x 256 MFMA pipeline (host-only, no GPU call): ZK_GEMM_TILED -- 2-byte type, M and N multiples
  * of 256, K a multiple of 128 and at least 256, leading dimensions multiples
  * of 8, and each operand's tile within one buffer resource (lda / ldb below
  * 2^22 elements for a [rows, K] operand, 2^24 for a K-major one); otherwise
- * ZK_GEMM_GENERAL.  ldr < 0: no residual. */
+ * ZK_GEMM_GENERAL, a kernel with masked edges.  ldr < 0: no residual. */
 enum zk_gemm_kernel { ZK_GEMM_GENERAL = 0, ZK_GEMM_TILED = 1 };
 int zk_gemm_path(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor, int64_t ldb,
                  int b_kmajor, int64_t ldc, int64_t ldr, int dtype);
@@ -225,9 +225,9 @@ int zk_rope(void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh, void* k,
  * models/llama_simple.py:206-221 followed by apply_rotary_pos_emb
  * (models/llama_simple.py:27-58) or apply_rotary_emb (models/llama_v2.py:
  * 151-177).  Rows are tokens b S + s (M a multiple of S); positions, tables
- * and pairing as for zk_rope.  bf16 / fp16 products on the 256 x 256 grid
- * with head_dim 64 / 128, rot_cols a multiple of 128, S in [128, 2^30) and
- * fewer than 2^24 table positions rotate in the GEMM's epilogue; other
+ * and pairing as for zk_rope.  bf16 / fp16 products with head_dim 64 / 128
+ * rotate in the GEMM's epilogue where the product's tile holds whole heads
+ * (the 256-wide tile: rot_cols a multiple of 128 and S >= 128); other
  * launches run zk_gemm then zk_rope (same result). */
 int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                  int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t S,

@@ -45,8 +45,10 @@ HIPCC_FLAGS = [
 # live ranges in reverse order, which keeps the 256 accumulators in place
 # through the loop (with the default order the both-K-major form moved ~80
 # of them between AGPRs per pass; the NT forms do better with the default).
+_KMAJOR = ["-Wno-inline-asm", "-mllvm", "-greedy-reverse-local-assignment=1"]
 FILE_FLAGS = {"rope.hip": ["-fno-slp-vectorize"], "gemm.hip": ["-Wno-inline-asm"],
-              "gemm_kmajor.hip": ["-Wno-inline-asm", "-mllvm", "-greedy-reverse-local-assignment=1"]}
+              "gemm_ring.hip": ["-Wno-inline-asm"], "gemm_kmajor.hip": _KMAJOR,
+              "gemm_ring_kmajor.hip": _KMAJOR}
 
 
 def _hipcc() -> str:

@@ -1,6 +1,8 @@
-// Projection GEMM entry points (zk_gemm, zk_gemm_nt, the SwiGLU-epilogue
-// launch); the kernels and their design are in gemm_kernels.h.  The tiled
-// forms with a K-major operand are launched from gemm_kmajor.hip.
+// Projection GEMM entry points (zk_gemm, zk_gemm_nt, zk_gemm_rope,
+// zk_gemm_swiglu) and the rule that names a product's tile; the kernels and
+// their design are in gemm_kernels.h and gemm_ring.h.  The tiled forms with a
+// K-major operand are launched from gemm_kmajor.hip, the small tiles from
+// gemm_ring.hip and gemm_ring_kmajor.hip.
 #include <type_traits>
 
 #include "gemm_kernels.h"
@@ -24,6 +26,79 @@ static bool tiled_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km, 
   return lda < lim_a && ldb < lim_b;
 }
 
+// Whether the MFMA kernels whose edges are masked (the RAG form of the 256 x
+// 256 pipeline, gemm_ring.h) take a launch: 2-byte type, every 8-element run
+// of an operand whole and 16-byte aligned -- N a multiple of 8 (stores), K of
+// 8 for an operand along K, M of 8 for a K-major A, leading dimensions of 8
+// -- and tiles within one buffer resource, as above.  Pointer alignment is
+// checked by the caller.
+static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km, int64_t ldb,
+                         int b_km, int64_t ldc, int64_t ldr, int dtype) {
+  if (dtype != ZK_BF16 && dtype != ZK_F16) return false;
+  if (M <= 0 || N <= 0 || K <= 0 || N % 8 || (a_km ? M : K) % 8 || (!b_km && K % 8)) return false;
+  if (lda % 8 || ldb % 8 || ldc % 8 || ldr % 8 || M >= 0x7fffffffLL) return false;
+  const int64_t lim_a = int64_t(1) << (a_km ? 24 : 22), lim_b = int64_t(1) << (b_km ? 24 : 22);
+  return lda < lim_a && ldb < lim_b &&
+         gemm::tile_count(gemm::k64, M, N) < 0x7fffffffLL;
+}
+
+// The tile a 2-byte product runs on: the one with the least estimated time
+//   launch + (full rounds + part) (edge + steps * step),
+// rounds of the tiles the CUs hold at once (cap workgroups each), `part` the
+// share of a round's time that a partly filled last round takes.  Constants
+// in us, fitted to 372 products timed on an MI355X in every tile (32 to 4095
+// tokens by the widths of the layers and heads from 1536 to 49152, forward,
+// input- and weight-gradient layouts, weights not in any cache): over those
+// products the choice is on average 0.3 % and at most 15 % slower than the
+// best tile.  Examples, us on 256 / 128 / 128x2 / 64 / 64x128 tiles:
+//   128 x 2048 x 2048 NT       42 / 26 / 21 / 11.5 / 16      (64)
+//   512 x 4096 x 11008 dX     198 / 121 / 100 / 104 / 76     (64x128)
+//   2048 x 2048 x 5632 NT     105 / 67 / 57 / 85 / 81        (128x2)
+//   1527 x 4096 x 4096 NT      82 / 56 / 80 / 80 / 109       (128)
+//   4095 x 4096 x 32000 dX    731 / 1015 / 1323 / 2839 / -   (256)
+// The K-split tiles are for grids of at most one workgroup per CU, and not
+// built for weight gradients, whose reduction (the tokens) is the short side.
+static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_km) {
+  struct Cost {
+    gemm::Tile t;
+    int per_cu;
+    double launch, edge, step, part;
+  };
+  static constexpr Cost kAlongK[] = {{gemm::k256, 1, 0.5, 9.5, 1.29, 0.82},
+                                     {gemm::k128, 2, 4.7, 0.8, 0.926, 0.73},
+                                     {gemm::k128x2, 1, 0.0, 5.7, 0.59, 0.82},
+                                     {gemm::k64, 2, 4.4, 0.0, 0.48, 0.60},
+                                     {gemm::k64x128, 1, 0.0, 5.1, 0.45, 0.92}};
+  static constexpr Cost kKMajor[] = {{gemm::k256, 1, 4.0, 10.4, 1.31, 0.73},
+                                     {gemm::k128, 2, 4.0, 3.0, 0.79, 0.59},
+                                     {gemm::k64, 2, 2.9, 1.9, 0.36, 0.59}};
+  if (a_km && !b_km) return gemm::k128;  // no layer product: one tile is built
+  const Cost* c = a_km ? kKMajor : kAlongK;
+  const int nc = a_km ? 3 : 5;
+  const int64_t cus = device_cus(), steps = (K + gemm::BK - 1) / gemm::BK;
+  gemm::Tile best = gemm::k256;
+  double best_us = 0;
+  for (int i = 0; i < nc; ++i) {
+    const int64_t n = gemm::tile_count(c[i].t, M, N), cap = cus * c[i].per_cu;
+    if ((c[i].t == gemm::k128x2 || c[i].t == gemm::k64x128) && n > cus) continue;
+    const int64_t full = n / cap, rem = n % cap;
+    double part = 0;  // two per CU: a lone workgroup runs faster than a pair
+    if (rem > 0)
+      part = c[i].per_cu == 2 ? (rem <= cus ? c[i].part : 1.0)
+                              : c[i].part + (1 - c[i].part) * static_cast<double>(rem) / cap;
+    double us = c[i].launch + (c[i].edge + steps * c[i].step) * (full + part);
+    // a K-major A is a weight gradient, which runs beside the input-gradient
+    // chain: the share of the chip it holds counts more than its own time
+    // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone)
+    if (a_km && n < cus) us *= 0.15 + 0.85 * static_cast<double>(n) / cus;
+    if (i == 0 || us < best_us) {
+      best = c[i].t;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 }  // namespace zk
 
 using namespace zk;
@@ -44,41 +119,45 @@ extern "C" int zk_gemm_path(int64_t M, int64_t N, int64_t K, int64_t lda, int a_
 
 namespace {
 
-template <typename T, bool AKM, bool BKM>
-void launch_gemm(bool tiled, const gemm::GemmArgs& ga, hipStream_t s) {
-  if constexpr (sizeof(T) == 2) {
-    if (tiled) {
-      if constexpr (AKM || BKM) {
-        gemm::launch_tiled_kmajor(std::is_same<T, bf16>::value, AKM, BKM, ga, s);
-      } else {
-        const int64_t nwg = (ga.M / gemm::BM) * (ga.N / gemm::BN);
-        if (gemm::half_tiles(nwg))
-          hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, 0, false, false, 4>),
-                             dim3(static_cast<unsigned>(2 * nwg)), dim3(256), 0, s, ga);
-        else
-          hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, 0, false, false>),
-                             dim3(static_cast<unsigned>(nwg)), dim3(256), 0, s, ga);
-      }
-      return;
-    }
-  }
-  {
-    const int64_t nwg = ((ga.M + gemm::GBM - 1) / gemm::GBM) * ((ga.N + gemm::GBM - 1) / gemm::GBM);
-    hipLaunchKernelGGL((gemm::gemm_gen_kernel<T, AKM, BKM>), dim3(static_cast<unsigned>(nwg)),
-                       dim3(256), 0, s, ga);
-  }
+// A 2-byte product on tile t; on_grid: tiled_takes.
+template <typename T, int EPI>
+void launch_256(bool on_grid, const gemm::GemmArgs& ga, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(gemm::tile_count(gemm::k256, ga.M, ga.N)));
+  if (on_grid)
+    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, EPI, false, false>), grid, dim3(256), 0, s, ga);
+  else
+    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, EPI, false, false, true>), grid, dim3(256), 0, s,
+                       ga);
+}
+
+template <int EPI>
+void launch_mfma(bool bf, gemm::Tile t, bool on_grid, int a_km, int b_km, const gemm::GemmArgs& ga,
+                 hipStream_t s) {
+  if (t != gemm::k256)
+    gemm::launch_ring(bf, EPI, a_km, b_km, t, ga, s);
+  else if (a_km || b_km)
+    gemm::launch_tiled_kmajor(bf, a_km, b_km, !on_grid, ga, s);
+  else if (bf)
+    launch_256<bf16, EPI>(on_grid, ga, s);
+  else
+    launch_256<f16, EPI>(on_grid, ga, s);
 }
 
 template <typename T>
-void launch_layout(bool tiled, int a_km, int b_km, const gemm::GemmArgs& ga, hipStream_t s) {
+void launch_general(int a_km, int b_km, const gemm::GemmArgs& ga, hipStream_t s) {
+  const int64_t nwg = ((ga.M + gemm::GBM - 1) / gemm::GBM) * ((ga.N + gemm::GBM - 1) / gemm::GBM);
+  const dim3 grid(static_cast<unsigned>(nwg));
+#define ZK_GEN(A, B) \
+  hipLaunchKernelGGL((gemm::gemm_gen_kernel<T, A, B>), grid, dim3(256), 0, s, ga)
   if (!a_km && !b_km)
-    launch_gemm<T, false, false>(tiled, ga, s);
-  else if (!a_km && b_km)
-    launch_gemm<T, false, true>(tiled, ga, s);
-  else if (a_km && b_km)
-    launch_gemm<T, true, true>(tiled, ga, s);
+    ZK_GEN(false, false);
+  else if (!a_km)
+    ZK_GEN(false, true);
+  else if (b_km)
+    ZK_GEN(true, true);
   else
-    launch_gemm<T, true, false>(tiled, ga, s);
+    ZK_GEN(true, false);
+#undef ZK_GEN
 }
 
 }  // namespace
@@ -107,10 +186,10 @@ extern "C" int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, 
                  (r == nullptr || ldr < (int64_t(1) << 40)) && rows_a < (int64_t(1) << 40) &&
                  rows_b < (int64_t(1) << 40) && M < (int64_t(1) << 40),
              ZK_EINVAL, "zk_gemm: sizes out of range");
-  bool tiled = tiled_takes(M, N, K, lda, a_km, ldb, b_km, ldc, r ? ldr : 8, dtype);
-  for (const void* p : ptrs) tiled = tiled && (p == nullptr || aligned(p, 16));
-  const int64_t nwg = tiled ? (M / gemm::BM) * (N / gemm::BN)
-                            : ((M + gemm::GBM - 1) / gemm::GBM) * ((N + gemm::GBM - 1) / gemm::GBM);
+  const bool on_grid = tiled_takes(M, N, K, lda, a_km, ldb, b_km, ldc, r ? ldr : 8, dtype);
+  bool mfma = on_grid || masked_takes(M, N, K, lda, a_km, ldb, b_km, ldc, r ? ldr : 8, dtype);
+  for (const void* p : ptrs) mfma = mfma && (p == nullptr || aligned(p, 16));
+  const int64_t nwg = ((M + gemm::GBM - 1) / gemm::GBM) * ((N + gemm::GBM - 1) / gemm::GBM);
   ZK_REQUIRE(nwg < 0x7fffffffLL, ZK_EINVAL, "zk_gemm: grid too large");
   gemm::GemmArgs ga{};
   ga.a = a;
@@ -125,12 +204,15 @@ extern "C" int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, 
   ga.N = N;
   ga.K = K;
   hipStream_t s = as_stream(stream);
-  if (dtype == ZK_BF16)
-    launch_layout<bf16>(tiled, a_km, b_km, ga, s);
+  if (mfma)
+    launch_mfma<0>(dtype == ZK_BF16, a_km && !b_km && on_grid ? gemm::k256 : pick_tile(M, N, K, a_km, b_km),
+                   on_grid, a_km, b_km, ga, s);
+  else if (dtype == ZK_BF16)
+    launch_general<bf16>(a_km, b_km, ga, s);
   else if (dtype == ZK_F16)
-    launch_layout<f16>(tiled, a_km, b_km, ga, s);
+    launch_general<f16>(a_km, b_km, ga, s);
   else
-    launch_layout<float>(false, a_km, b_km, ga, s);
+    launch_general<float>(a_km, b_km, ga, s);
   return launch_status("zk_gemm");
 }
 
@@ -141,8 +223,10 @@ extern "C" int zk_gemm_nt(const void* a, int64_t lda, const void* b, int64_t ldb
 }
 
 // The q|k|v projection with the rotary embedding applied in the GEMM's
-// epilogue (EPI 2) when the 256 x 256 pipeline takes the launch; otherwise
-// zk_gemm followed by zk_rope on the rotated columns, which rounds the same.
+// epilogue (EPI 2) when an MFMA kernel takes the launch and its tile holds
+// whole heads; otherwise zk_gemm followed by zk_rope on the rotated columns,
+// which rounds the same (both run the tile pick_tile names, so the product
+// before the rotation is the same too).
 extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                             int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t S,
                             int64_t rot_cols, int64_t head_dim, const float* cos,
@@ -169,11 +253,16 @@ extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t l
   if (M == 0 || N == 0) return ZK_OK;
   ZK_REQUIRE(c != nullptr && (K == 0 || (a != nullptr && b != nullptr)), ZK_EINVAL,
              "zk_gemm_rope: null pointer");
-  const bool epi = tiled_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype) && aligned(a, 16) &&
-                   aligned(b, 16) && aligned(c, 16) && (head_dim == 64 || head_dim == 128) &&
-                   rot_cols % 128 == 0 && aligned(cos, 16) && aligned(sin, 16) &&
-                   S >= 128 && S < (int64_t(1) << 30) && n_pos < (int64_t(1) << 24) &&
-                   (M / gemm::BM) * (N / gemm::BN) < 0x7fffffffLL;
+  const bool on_grid = tiled_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype);
+  bool epi = (on_grid || masked_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype)) && aligned(a, 16) &&
+             aligned(b, 16) && aligned(c, 16) && (head_dim == 64 || head_dim == 128) &&
+             aligned(cos, 16) && aligned(sin, 16) && S < (int64_t(1) << 30) &&
+             n_pos < (int64_t(1) << 24);
+  const gemm::Tile tile = epi ? pick_tile(M, N, K, false, false) : gemm::k256;
+  // the 256-wide tile rotates whole 128-column blocks of sequences of at least
+  // 128 tokens; a 64-wide one holds heads of 64 only
+  if (tile == gemm::k256) epi = epi && rot_cols % 128 == 0 && S >= 128;
+  if (tile == gemm::k64) epi = epi && head_dim == 64;
   if (!epi) {
     const int rc = zk_gemm(a, lda, 0, b, ldb, 0, c, ldc, nullptr, 0, M, N, K, dtype, stream);
     if (rc != ZK_OK || rot_cols == 0) return rc;
@@ -199,29 +288,52 @@ extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t l
   ga.rcols = rot_cols;
   ga.rhalf = static_cast<int>(head_dim / 2);
   ga.rpair = pairing;
-  const dim3 grid(static_cast<unsigned>((M / gemm::BM) * (N / gemm::BN)));
-  hipStream_t s = as_stream(stream);
-  if (dtype == ZK_BF16)
-    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<bf16, 2, false, false>), grid, dim3(256), 0, s, ga);
-  else
-    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<f16, 2, false, false>), grid, dim3(256), 0, s, ga);
+  launch_mfma<2>(dtype == ZK_BF16, tile, on_grid, 0, 0, ga, as_stream(stream));
   return launch_status("zk_gemm_rope");
 }
 
-namespace zk {
-
-// The gate|up projection with the SwiGLU epilogue on the 256 x 256 pipeline
-// (zk_gemm_swiglu routes the shapes it takes here: M a multiple of 256, F of
-// 128, K of 128 and at least 256, ld_x and ld_w below 2^22).  Arguments as
-// zk_gemm_swiglu, already validated.
-int zk_gemm_swiglu_tiled_supported(int64_t M, int64_t F, int64_t K) {
-  return zk_gemm_nt_supported(M, 2 * F, K);
-}
-
-int zk_gemm_swiglu_tiled(const void* x, int64_t ld_x, const void* w_gate, const void* w_up,
-                         int64_t ld_w, void* g_out, void* u_out, int64_t ld_gu, void* z,
-                         int64_t ld_z, void* zt, int64_t ld_zt, int64_t M, int64_t F, int64_t K,
-                         int dtype, zk_stream_t stream) {
+// The gate|up projection with the SwiGLU epilogue (EPI 1): replaces the two
+// nn.Linear products and the activation.  K steps are whole (K % 64 == 0).
+extern "C" int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
+                              const void* w_up, int64_t ld_w, void* g_out, void* u_out,
+                              int64_t ld_gu, void* z, int64_t ld_z, void* zt, int64_t ld_zt,
+                              int64_t M, int64_t F, int64_t K, int dtype, zk_stream_t stream) {
+  ZK_REQUIRE(dtype == ZK_BF16 || dtype == ZK_F16, ZK_EDTYPE,
+             "zk_gemm_swiglu: 2-byte dtypes only (got %d)", dtype);
+  ZK_REQUIRE(M >= 0 && F >= 0 && K >= 0, ZK_EINVAL, "zk_gemm_swiglu: bad shape");
+  ZK_REQUIRE(ld_x >= K && ld_w >= K && ld_gu >= F && ld_z >= F && (zt == nullptr || ld_zt >= M),
+             ZK_EINVAL, "zk_gemm_swiglu: bad leading dimension");
+  if (M == 0 || F == 0) return ZK_OK;
+  ZK_REQUIRE(K > 0 && K % gemm::BK == 0, ZK_EUNSUPPORTED,
+             "zk_gemm_swiglu: K must be a positive multiple of %d (got %lld)", gemm::BK,
+             (long long)K);
+  ZK_REQUIRE(M % 8 == 0 && F % 8 == 0, ZK_EUNSUPPORTED,
+             "zk_gemm_swiglu: M and F must be multiples of 8 (got %lld, %lld)", (long long)M,
+             (long long)F);
+  const int64_t lds[] = {ld_x, ld_w, ld_gu, ld_z, zt ? ld_zt : 8};
+  for (int64_t ld : lds)
+    ZK_REQUIRE(ld % 8 == 0, ZK_EALIGN, "zk_gemm_swiglu: leading dimensions must be multiples of 8");
+  const void* ptrs[] = {x, w_gate, w_up, g_out, u_out, z};
+  for (const void* p : ptrs) {
+    ZK_REQUIRE(p != nullptr, ZK_EINVAL, "zk_gemm_swiglu: null pointer");
+    ZK_REQUIRE(aligned(p, 16), ZK_EALIGN, "zk_gemm_swiglu: operands must be 16-byte aligned");
+  }
+  ZK_REQUIRE(zt == nullptr || aligned(zt, 16), ZK_EALIGN,
+             "zk_gemm_swiglu: operands must be 16-byte aligned");
+  ZK_REQUIRE(ld_x < (int64_t(1) << 26) && ld_w < (int64_t(1) << 26), ZK_EUNSUPPORTED,
+             "zk_gemm_swiglu: leading dimension out of range");
+  ZK_REQUIRE(((M + 127) / 128) * ((F + 63) / 64) < 0x7fffffffLL, ZK_EINVAL,
+             "zk_gemm_swiglu: grid too large");
+  if (!masked_takes(M, 2 * F, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype)) {
+    // rows too far apart for a tile's buffer resource: the two products and the
+    // activation as separate launches
+    int rc = zk_gemm(x, ld_x, 0, w_gate, ld_w, 0, g_out, ld_gu, nullptr, 0, M, F, K, dtype, stream);
+    if (rc != ZK_OK) return rc;
+    rc = zk_gemm(x, ld_x, 0, w_up, ld_w, 0, u_out, ld_gu, nullptr, 0, M, F, K, dtype, stream);
+    if (rc != ZK_OK) return rc;
+    return zt != nullptr ? zk_swiglu_fwd_t(g_out, u_out, ld_gu, z, ld_z, zt, ld_zt, M, F, dtype, stream)
+                         : zk_swiglu_fwd(g_out, u_out, ld_gu, z, ld_z, M, F, dtype, stream);
+  }
   gemm::GemmArgs ga{};
   ga.a = x;
   ga.lda = ld_x;
@@ -238,15 +350,8 @@ int zk_gemm_swiglu_tiled(const void* x, int64_t ld_x, const void* w_gate, const 
   ga.M = M;
   ga.N = 2 * F;
   ga.K = K;
-  const int64_t nwg = (M / gemm::BM) * (2 * F / gemm::BN);
-  hipStream_t s = as_stream(stream);
-  if (dtype == ZK_BF16)
-    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<bf16, 1, false, false>),
-                       dim3(static_cast<unsigned>(nwg)), dim3(256), 0, s, ga);
-  else
-    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<f16, 1, false, false>),
-                       dim3(static_cast<unsigned>(nwg)), dim3(256), 0, s, ga);
+  const bool on_grid = tiled_takes(M, 2 * F, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype);
+  launch_mfma<1>(dtype == ZK_BF16, pick_tile(M, 2 * F, K, false, false), on_grid, 0, 0, ga,
+                 as_stream(stream));
   return launch_status("zk_gemm_swiglu");
 }
-
-}  // namespace zk

@@ -40,9 +40,11 @@
 // round-robins XCDs) take consecutive tiles, ordered in groups of four M
 // tiles, so each XCD's L2 serves a 4 x 8 block of tiles.
 //
-// Shapes off that grid, fp32 operands, and leading dimensions past the
-// buffer-resource range go to gemm_gen_kernel: 128 x 128 tiles staged
-// through registers with masked loads and stores (any M, N, K).
+// Shapes off that grid take the same kernel with its edges masked (RAG) or the
+// small-tile kernel of gemm_ring.h, whichever gemm.hip's cost rule names.
+// fp32 operands, layouts that are not 16-byte aligned and leading dimensions
+// past the buffer-resource range go to gemm_gen_kernel: 128 x 128 tiles
+// staged through registers with masked loads and stores (any M, N, K).
 //
 // This header holds the kernels; gemm.hip launches the NT forms (the
 // forward products and the SwiGLU-epilogue instance) and the general kernel,
@@ -75,6 +77,23 @@ __device__ __forceinline__ v4i rsrc_words(const void* base) {
   r[2] = 0x7fffffff;
   r[3] = 0x00020000;
   return r;
+}
+
+// The same with the resource ending `left` bytes past base (at most 2 GiB, and
+// empty for left <= 0): an LDS load's lanes at or past the end write zeros
+// (checked per 4 bytes; a scalar offset past the end counts as past it).
+__device__ __forceinline__ v4i rsrc_left(const void* base, int64_t left) {
+  v4i r = rsrc_words(base);
+  const int64_t n = left < 0 ? 0 : left > 0x7fffffff ? 0x7fffffff : left;
+  r[2] = __builtin_amdgcn_readfirstlane(static_cast<int>(n));
+  return r;
+}
+
+// Tile index of workgroup `bid` of `n`: the dispatch order round-robins the
+// eight XCDs, so XCD x gets the x-th eighth of the tile order.
+__device__ __forceinline__ int64_t xcd_order(int64_t bid, int64_t n) {
+  const int64_t x = bid & 7, q = n >> 3, r = n & 7;
+  return x * q + (x < r ? x : r) + (bid >> 3);
 }
 
 template <typename T>
@@ -150,6 +169,15 @@ __device__ __forceinline__ int nt_off(int r, int col) {
 // An NT tile: ROWS x 64 (128-byte rows, chunks swizzled by nt_sw) in eight
 // instructions of 32 rows; instruction i of wave w fills LDS chunks
 // 256 i + 64 w .. +63, lane l the chunk of row 32 i + (64 w + l) / 8.
+// RAG: the lane offset `off` of K step k of an NT tile, or an offset past any
+// resource when this lane's 16-byte chunk (column 8 ((tid % 8) ^ nt_sw(row)),
+// row tid / 8 modulo 16) lies at or past K.
+__device__ __forceinline__ uint32_t ld_past(uint32_t off, int64_t k, int64_t K) {
+  const int tid = threadIdx.x;
+  const int col = 8 * ((tid & 7) ^ nt_sw(tid >> 3));
+  return k * BK + col < K ? off : 0x80000000u;
+}
+
 template <typename T>
 struct TileDma {
   static constexpr int D = BK, NT = 256, RSTEP = NT / (D / 8);
@@ -169,6 +197,16 @@ struct TileDma {
   __device__ __forceinline__ void issue_wave_rows(T* tile, const T* src, uint32_t soff,
                                                   int i) const {
     dma16(rsrc_words(src), lane_off8, soff, lds_addr(tile + wave_el) + i * NT * 16);
+  }
+  // issue_wave_rows and issue from a given resource and lane offset
+  __device__ __forceinline__ void issue_wave_rows_in(T* tile, v4i r, uint32_t voff, uint32_t soff,
+                                                     int i) const {
+    dma16(r, voff, soff, lds_addr(tile + wave_el) + i * NT * 16);
+  }
+  __device__ __forceinline__ void issue_in(T* tile, v4i r, uint32_t voff, int64_t ld, int i) const {
+    const uint32_t soff =
+        static_cast<uint32_t>(static_cast<int64_t>(i) * RSTEP * ld * static_cast<int64_t>(sizeof(T)));
+    dma16(r, voff, soff, lds_addr(tile + wave_el) + i * NT * 16);
   }
   // piece i (rows 32 i .. 32 i + 31) of the tile whose first row is `gbase`
   __device__ __forceinline__ void issue(T* tile, const T* gbase, int64_t ld, int i) const {
@@ -205,9 +243,12 @@ struct TileDmaK {
   }
   // piece i of the tile whose first row (k) and column are at `gbase`
   __device__ __forceinline__ void issue(T* tile, const T* gbase, int64_t ld, int i) const {
+    issue_in(tile, rsrc_words(gbase), ld, i);
+  }
+  __device__ __forceinline__ void issue_in(T* tile, v4i r, int64_t ld, int i) const {
     const int ri = 4 * (i & 1) + 16 * (i >> 1);
     const uint32_t soff = static_cast<uint32_t>(ri * ld * static_cast<int64_t>(sizeof(T)));
-    dma16(rsrc_words(gbase), lane_off, soff, lds_addr(tile + (wave_row + ri) * 256));
+    dma16(r, lane_off, soff, lds_addr(tile + (wave_row + ri) * 256));
   }
 };
 
@@ -251,34 +292,21 @@ __device__ __forceinline__ float silu_fast(float g) {
 
 // AKM / BKM: operand A / B is K-major (see the top of the file).  EPI 1
 // takes NT operands only.
-// Products with A along the reduction whose 256 x 256 tiles would occupy at
-// most half the CUs (e.g. a 4096 x 2048 product: 128 tiles on 256 CUs) run on
-// 128 x 256 tiles instead, twice the workgroups with half the work each and
-// every output summed in the same order.
-inline bool half_tiles(int64_t nwg) { return nwg > 0 && 2 * nwg <= device_cus(); }
+// Operand-read order of a set (see mm_ld): A0, B0 .. B7, A1 .. A7, with A
+// pieces numbered 0 .. 7 and B pieces 8 .. 15.
+__device__ constexpr int kReadOrder[16] = {0, 8, 9, 10, 11, 12, 13, 14, 15, 1, 2, 3, 4, 5, 6, 7};
 
-// Operand-read order of a set (see mm_ld): A0, B0 .. B7, A1 .. A(MB-1), with
-// A pieces numbered 0 .. MB-1 and B pieces MB .. MB+7.
-struct ReadOrder {
-  int v[16];
-};
-template <int MB>
-constexpr ReadOrder read_order() {
-  ReadOrder r{};
-  r.v[0] = 0;
-  for (int i = 1; i <= 8; ++i) r.v[i] = MB + i - 1;
-  for (int i = 9; i < MB + 8; ++i) r.v[i] = i - 8;
-  return r;
-}
-
-// MB: 16-row MFMA blocks per wave along M -- 8 (the 256 x 256 tile) or 4 (a
-// 128 x 256 tile: for a product whose 256 x 256 tiles would occupy at most
-// half the CUs, twice the workgroups with half the work each).
-template <typename T, int EPI, bool AKM, bool BKM, int MB = 8>
+// RAG: M, N, K off the grid (M and N multiples of 8 where an operand is
+// contiguous along them, K of 8 for an NT operand).  The buffer resources end
+// with the operands, so that loads past an edge write zeros to LDS; the
+// columns of an NT tile past K are sent out of range lane by lane, K is
+// padded to an even number of steps (at least four) that way, and stores are
+// masked per 8-column chunk.  The SwiGLU epilogue takes silu in the IEEE form.
+template <typename T, int EPI, bool AKM, bool BKM, bool RAG = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_tiled_kernel(GemmArgs args) {
   static_assert(EPI == 0 || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
-  static_assert(MB == 8 || (MB == 4 && EPI == 0 && !AKM), "128-row tiles: plain epilogue, A along K");
+  constexpr int MB = 8;         // 16-row MFMA blocks per wave along M
   constexpr int TBM = 32 * MB;  // tile rows
   constexpr int WR = 16 * MB;   // rows per wave
   const T* __restrict__ A = static_cast<const T*>(args.a);
@@ -294,9 +322,13 @@ void gemm_tiled_kernel(GemmArgs args) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, q4 = lane >> 4;
   const int wm = wave >> 1, wn = wave & 1;
-  const int64_t n_m = M / TBM, n_n = N / BN, nwg = n_m * n_n;
+  const int64_t n_m = RAG ? (M + TBM - 1) / TBM : M / TBM;
+  const int64_t n_n = RAG ? (N + BN - 1) / BN : N / BN, nwg = n_m * n_n;
   int64_t pid = blockIdx.x;
-  if ((nwg & 7) == 0) pid = (pid & 7) * (nwg >> 3) + (pid >> 3);
+  if constexpr (RAG)
+    pid = xcd_order(pid, nwg);
+  else if ((nwg & 7) == 0)
+    pid = (pid & 7) * (nwg >> 3) + (pid >> 3);
   const int64_t per_group = static_cast<int64_t>(GROUP_M) * n_n;
   const int64_t grp = pid / per_group;
   const int64_t mf = grp * GROUP_M;
@@ -373,14 +405,39 @@ void gemm_tiled_kernel(GemmArgs args) {
         xb[q][r - MB] = *reinterpret_cast<const V8*>(&t[ntB[s] + 1024 * (r - MB)]);
     }
   };
+  // RAG: elements from the tile's first one (K step 0) to the operand's end
+  const int64_t b_rows = EPI == 1 ? N / 2 : N;
+  const int64_t a_left = AKM ? (K - 1) * lda + M - m0 : (M - 1 - m0) * lda + K;
+  const int64_t b_left = EPI == 1 ? (b_rows - 1 - f0 - 8 * (wv & 1)) * ldb + K
+                         : BKM    ? (K - 1) * ldb + N - n0
+                                  : (N - 1 - n0) * ldb + K;
   auto loadA = [&](int sa, int64_t k, int p) __attribute__((always_inline)) {
-    if constexpr (AKM)
+    if constexpr (RAG) {
+      const v4i r = rsrc_left(Ab + k * a_step, 2 * (a_left - k * a_step));
+      if constexpr (AKM)
+        admak.issue_in(&As[sa * (TBM * BK)], r, lda, p);
+      else
+        adma.issue_in(&As[sa * (TBM * BK)], r, ld_past(adma.lane_off, k, K), lda, p);
+    } else if constexpr (AKM) {
       admak.issue(&As[sa * (TBM * BK)], Ab + k * a_step, lda, p);
-    else
+    } else {
       adma.issue(&As[sa * (TBM * BK)], Ab + k * a_step, lda, p);
+    }
   };
   auto loadB = [&](int sb, int64_t k, int p) __attribute__((always_inline)) {
-    if constexpr (EPI != 1) {
+    if constexpr (RAG) {
+      if constexpr (EPI == 1) {
+        const v4i r = rsrc_left(bwave + k * BK, 2 * (b_left - k * BK));
+        bdma.issue_wave_rows_in(Bs(sb), r, ld_past(bdma.lane_off8, k, K),
+                                static_cast<uint32_t>(32 * p * ldb), p);
+      } else {
+        const v4i r = rsrc_left(Bb + k * b_step, 2 * (b_left - k * b_step));
+        if constexpr (BKM)
+          bdmak.issue_in(Bs(sb), r, ldb, p);
+        else
+          bdma.issue_in(Bs(sb), r, ld_past(bdma.lane_off, k, K), ldb, p);
+      }
+    } else if constexpr (EPI != 1) {
       if constexpr (BKM)
         bdmak.issue(Bs(sb), Bb + k * b_step, ldb, p);
       else
@@ -390,17 +447,14 @@ void gemm_tiled_kernel(GemmArgs args) {
                            static_cast<uint32_t>(16 * p * ldb * static_cast<int64_t>(sizeof(T))), p);
     }
   };
-  // The 8 MB MFMAs of set q in rows of eight.  After row c: A piece c (LK 1:
-  // of step k into ring stage lst) or 8 / MB B pieces (LK 2: into B stage
-  // lst), and, when RD, (MB + 8) / MB operand pieces of substep s0 of stages
-  // (ra, rb) into set q0, in the order the next set's MFMAs use them: its
-  // first row needs A piece 0 and all eight B pieces, row c A piece c, so the
-  // reads go A0, B0 .. B7, A1 .. A(MB-1) (for MB = 8, B7 is in flight from
-  // row 4, three rows before it is needed; read last, it stalled the next
-  // set's first MFMA for the LDS latency at every substep).  The fences keep
-  // this order.
-  constexpr ReadOrder kRO = read_order<MB>();
-  constexpr int RPR = (MB + 8) / MB, BPR = 8 / MB;
+  // The 64 MFMAs of set q in rows of eight.  After row c: A piece c (LK 1: of
+  // step k into ring stage lst) or B piece c (LK 2: into B stage lst), and,
+  // when RD, two operand pieces of substep s0 of stages (ra, rb) into set q0,
+  // in the order the next set's MFMAs use them: its first row needs A piece 0
+  // and all eight B pieces, row c A piece c, so the reads go A0, B0 .. B7, A1
+  // .. A7 (B7 is in flight from row 4, three rows before it is needed; read
+  // last, it stalled the next set's first MFMA for the LDS latency at every
+  // substep).  The fences keep this order.
   auto mm_ld = [&](int q, int lk, int lst, int64_t k, bool rd, int ra, int rb, int s0,
                    int q0) __attribute__((always_inline)) {
 #pragma unroll
@@ -408,19 +462,17 @@ void gemm_tiled_kernel(GemmArgs args) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[c][j] = Mm::mma16(xa[q][c], xb[q][j], acc[c][j]);
       if (rd) {
-#pragma unroll
-        for (int u = 0; u < RPR; ++u) rd_piece(ra, rb, s0, q0, kRO.v[RPR * c + u]);
+        rd_piece(ra, rb, s0, q0, kReadOrder[2 * c]);
+        rd_piece(ra, rb, s0, q0, kReadOrder[2 * c + 1]);
       }
       if (lk == 1) loadA(lst, k, c);
-      if (lk == 2) {
-#pragma unroll
-        for (int u = 0; u < BPR; ++u) loadB(lst, k, BPR * c + u);
-      }
+      if (lk == 2) loadB(lst, k, c);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  const int64_t n_k = K / BK;  // even, >= 4
+  // even, >= 4
+  const int64_t n_k = RAG ? (K > 2 * BK ? (K + 2 * BK - 1) / (2 * BK) * 2 : 4) : K / BK;
   // prologue: steps 0 and 1 of A and B
 #pragma unroll
   for (int p = 0; p < MB; ++p) loadA(0, 0, p);
@@ -491,18 +543,13 @@ void gemm_tiled_kernel(GemmArgs args) {
   // wave's own LDS region (pitch 132 floats), then 16-byte row stores.
   // Accumulator layout: acc[i][j][e] is row 16 i + 4 (l / 16) + e, column
   // 16 j + l % 16 of the wave's block.
+  if constexpr (RAG) wait_vmcnt<0>();
   __syncthreads();
   int el = lane;
   asm volatile("" : "+v"(el));  // keep the epilogue's index math after the loop
   // each wave's 16 x 132-float staging area (and for EPI 1 the z tile after
-  // it): a 32 KB A stage each for 256-row tiles (Bs0 for wave 3); for 128-row
-  // tiles (EPI 0 only) two in the 48 KB A ring, Bs0 and Bs1
-  float* ws;
-  if constexpr (MB == 8)
-    ws = reinterpret_cast<float*>(wave < 3 ? &As[wave * (TBM * BK)] : Bs0);
-  else
-    ws = wave < 2 ? reinterpret_cast<float*>(As) + wave * (16 * 132)
-                  : reinterpret_cast<float*>(wave == 2 ? Bs0 : Bs1);
+  // it) in a 32 KB A stage each (Bs0 for wave 3)
+  float* ws = reinterpret_cast<float*>(wave < 3 ? &As[wave * (TBM * BK)] : Bs0);
   const int e16 = el & 15, eq = el >> 4;
   typedef T T8 __attribute__((ext_vector_type(8)));
   // EPI 2: the wave's 128 columns hold whole heads (head dim 2 rhalf = 64 or
@@ -571,8 +618,10 @@ void gemm_tiled_kernel(GemmArgs args) {
           o2[e] = static_cast<T>(y2);
         }
         const int64_t gcol = n0 + wn * 128;
-        *reinterpret_cast<T8*>(C + grow * args.ldc + gcol + 8 * ca) = o1;
-        *reinterpret_cast<T8*>(C + grow * args.ldc + gcol + 8 * cb) = o2;
+        if (!RAG || grow < M) {
+          *reinterpret_cast<T8*>(C + grow * args.ldc + gcol + 8 * ca) = o1;
+          *reinterpret_cast<T8*>(C + grow * args.ldc + gcol + 8 * cb) = o2;
+        }
       }
     } else if (EPI == 2 && rot) {
       // interleaved pairs (2 i, 2 i + 1) inside each chunk: 16 rows x 16 chunks
@@ -597,7 +646,8 @@ void gemm_tiled_kernel(GemmArgs args) {
           o[2 * j] = static_cast<T>(y1);
           o[2 * j + 1] = static_cast<T>(y2);
         }
-        *reinterpret_cast<T8*>(C + grow * args.ldc + n0 + wn * 128 + 8 * ch) = o;
+        if (!RAG || grow < M)
+          *reinterpret_cast<T8*>(C + grow * args.ldc + n0 + wn * 128 + 8 * ch) = o;
       }
     } else if constexpr (EPI != 1) {
       // c = acc (+ r), one rounding; 16 rows x 16 chunks of 8 columns
@@ -612,6 +662,7 @@ void gemm_tiled_kernel(GemmArgs args) {
         float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         const int64_t grow = row0 + rr;
         const int64_t gcol = n0 + wn * 128 + 8 * ch;
+        if (RAG && (grow >= M || gcol >= N)) continue;
         if (R != nullptr) {
           const T8 rv = *reinterpret_cast<const T8*>(R + grow * args.ldr + gcol);
 #pragma unroll
@@ -648,14 +699,18 @@ void gemm_tiled_kernel(GemmArgs args) {
         for (int e = 0; e < 8; ++e) {
           go[e] = static_cast<T>(gv[e]);
           uo[e] = static_cast<T>(uv[e]);
-          zo[e] = static_cast<T>(round_to<T>(silu_fast(to_f32(go[e]))) * to_f32(uo[e]));
+          const float gr = to_f32(go[e]);
+          const float sv = RAG ? gr / (1.0f + expf(-gr)) : silu_fast(gr);
+          zo[e] = static_cast<T>(round_to<T>(sv) * to_f32(uo[e]));
           zs[(16 * jp + 8 * h + e) * 136 + 16 * i + rr] = zo[e];
         }
         const int64_t grow = row0 + rr;
         const int64_t f = f0 + wn * 64 + 16 * jp + 8 * h;
-        *reinterpret_cast<T8*>(G + grow * args.ldc + f) = go;
-        *reinterpret_cast<T8*>(U + grow * args.ldc + f) = uo;
-        *reinterpret_cast<T8*>(Z + grow * args.ldz + f) = zo;
+        if (!RAG || (grow < M && f < b_rows)) {
+          *reinterpret_cast<T8*>(G + grow * args.ldc + f) = go;
+          *reinterpret_cast<T8*>(U + grow * args.ldc + f) = uo;
+          *reinterpret_cast<T8*>(Z + grow * args.ldz + f) = zo;
+        }
       }
     }
   }
@@ -670,7 +725,8 @@ void gemm_tiled_kernel(GemmArgs args) {
         const int ch = q * 64 + el;
         const int fr = ch >> 4, tc = ch & 15;
         const T8 v = *reinterpret_cast<const T8*>(&zs[fr * 136 + 8 * tc]);
-        *reinterpret_cast<T8*>(ZT + (fw0 + fr) * args.ldzt + t0 + 8 * tc) = v;
+        if (!RAG || (fw0 + fr < b_rows && t0 + 8 * tc < M))
+          *reinterpret_cast<T8*>(ZT + (fw0 + fr) * args.ldzt + t0 + 8 * tc) = v;
       }
     }
   }
@@ -683,8 +739,9 @@ void gemm_tiled_kernel(GemmArgs args) {
 // (out-of-range elements are zero), written to LDS as [128 rows][32 k] (k
 // contiguous, padded rows), and consumed by v_mfma_f32_16x16x32 (2-byte
 // types) or v_mfma_f32_16x16x4f32 (fp32, full fp32 products).  Stores are
-// masked per element.  This is the path for token counts off the 256 grid
-// and for fp32 layers; it needs no alignment beyond the element's.
+// masked per element.  This is the path for fp32 layers and for 2-byte
+// operands the DMA kernels cannot load (16-byte alignment); it needs no
+// alignment beyond the element's.
 constexpr int GBM = 128, GBK = 32;
 
 template <typename T>
@@ -797,10 +854,28 @@ __global__ __launch_bounds__(256) void gemm_gen_kernel(GemmArgs args) {
       }
 }
 
-// The tiled kernel with A and / or B K-major (gemm_kmajor.hip), bf16 or fp16,
-// on a launch tiled_takes accepted.
-void launch_tiled_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, const GemmArgs& ga,
+// The tiled kernel with A and / or B K-major (gemm_kmajor.hip), bf16 or fp16;
+// ragged: off the grid (RAG), not for A K-major with B along K.
+void launch_tiled_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, bool ragged, const GemmArgs& ga,
                          hipStream_t s);
+
+// Tiles of the 2-byte MFMA kernels: the 256 x 256 pipeline above, and the
+// small-tile kernel of gemm_ring.h with 4 waves (k128: 128 x 128, k64: 64 x
+// 64, two workgroups per CU) or 8 waves split over K (k128x2: 128 x 128,
+// k64x128: 64 x 128, one workgroup per CU).
+enum Tile { k256, k128, k128x2, k64, k64x128 };
+inline int tile_rows(Tile t) { return t == k256 ? 256 : t == k64 || t == k64x128 ? 64 : 128; }
+inline int tile_cols(Tile t) { return t == k256 ? 256 : t == k64 ? 64 : 128; }
+inline int64_t tile_count(Tile t, int64_t M, int64_t N) {
+  return ((M + tile_rows(t) - 1) / tile_rows(t)) * ((N + tile_cols(t) - 1) / tile_cols(t));
+}
+
+// The small-tile kernel; epi as for gemm_tiled_kernel, 1 and 2 on NT operands
+// only (gemm_ring.hip; gemm_ring_kmajor.hip for the K-major forms).
+void launch_ring(bool bf16, int epi, bool a_kmajor, bool b_kmajor, Tile t, const GemmArgs& ga,
+                 hipStream_t s);
+void launch_ring_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, Tile t, const GemmArgs& ga,
+                        hipStream_t s);
 
 }  // namespace gemm
 

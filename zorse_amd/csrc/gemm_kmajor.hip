@@ -9,26 +9,27 @@ namespace gemm {
 
 namespace {
 template <typename T>
-void launch_t(bool akm, bool bkm, const GemmArgs& ga, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>((ga.M / BM) * (ga.N / BN)));
-  if (akm && bkm)
-    hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, true, true>), grid, dim3(256), 0, s, ga);
-  else if (akm)
-    hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, true, false>), grid, dim3(256), 0, s, ga);
-  else if (half_tiles(grid.x))
-    hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, false, true, 4>), dim3(2 * grid.x), dim3(256), 0,
-                       s, ga);
-  else
-    hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, false, true>), grid, dim3(256), 0, s, ga);
+void launch_t(bool akm, bool bkm, bool ragged, const GemmArgs& ga, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(((ga.M + BM - 1) / BM) * ((ga.N + BN - 1) / BN)));
+#define ZK_TILED(A, B, R) \
+  hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, A, B, R>), grid, dim3(256), 0, s, ga)
+  if (akm && bkm) {
+    if (ragged) ZK_TILED(true, true, true); else ZK_TILED(true, true, false);
+  } else if (akm) {
+    ZK_TILED(true, false, false);
+  } else {
+    if (ragged) ZK_TILED(false, true, true); else ZK_TILED(false, true, false);
+  }
+#undef ZK_TILED
 }
 }  // namespace
 
-void launch_tiled_kmajor(bool bf16_, bool a_kmajor, bool b_kmajor, const GemmArgs& ga,
+void launch_tiled_kmajor(bool bf16_, bool a_kmajor, bool b_kmajor, bool ragged, const GemmArgs& ga,
                          hipStream_t s) {
   if (bf16_)
-    launch_t<bf16>(a_kmajor, b_kmajor, ga, s);
+    launch_t<bf16>(a_kmajor, b_kmajor, ragged, ga, s);
   else
-    launch_t<f16>(a_kmajor, b_kmajor, ga, s);
+    launch_t<f16>(a_kmajor, b_kmajor, ragged, ga, s);
 }
 
 }  // namespace gemm
