@@ -1,0 +1,97 @@
+"""The fp32 matrix-core kernels (csrc/attn_f32.hip, the fp32 tiles of
+csrc/gemm_ring.h) at the edges of their tiles, against float64.
+
+Bounds: fp32 sums of n products are off by at most n 2^-24 times the sum of
+the absolute products; attention results by assert_close's 1e-4 of the
+largest value."""
+import pytest
+import torch
+
+from oracle import decoder as O
+from tests._tol import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(shape, seed, dev):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dev)
+
+
+# 64 x 64 tiles (fewer 128 x 128 tiles than CUs) and 128 x 128 tiles; K a few
+# elements into a step, one row, weight gradients over odd token counts
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (65, 72, 40), (256, 688, 256), (2056, 2200, 40)])
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, True), (True, False)],
+                         ids=["X_Wt", "dY_W", "dYt_X", "At_B"])
+def test_gemm_fp32_tiles(dev, M, N, K, layout):
+    from zorse_amd import kernels as K_
+    a_km, b_km = layout
+    if a_km:
+        M, K = -(-M // 8) * 8, K if not b_km else K + 3
+    print(f"gemm fp32 {M}x{N}x{K} {layout}", flush=True)
+    pad = torch.full(((K if a_km else M) + 1, (M if a_km else K) + 8), float("nan"), device=dev)
+    a = pad[:-1, :-8]
+    a.copy_(_randn(a.shape, 1, dev))
+    bpad = torch.full(((K if b_km else N) + 1, (N if b_km else K) + 8), float("nan"), device=dev)
+    b = bpad[:-1, :-8]
+    b.copy_(_randn(b.shape, 2, dev))
+    r = _randn((M, N), 3, dev)
+    out = torch.full((M + 1, N + 8), 7.0, device=dev)
+    K_.gemm(a, b, a_kmajor=a_km, b_kmajor=b_km, residual=r, out=out[:M, :N])
+    am = (a.t() if a_km else a).double().contiguous()
+    bm = (b if b_km else b.t()).double().contiguous()
+    ref = torch.mm(am, bm) + r.double()
+    bound = (K + 2) * 2.0 ** -24 * (torch.mm(am.abs(), bm.abs()) + r.double().abs())
+    assert bool(((out[:M, :N].double() - ref).abs() <= bound).all())
+    assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+
+
+# B, Sq, Skv, Hq, Hkv, d, causal, window: one row, tile edges at 32 and 64,
+# head dims off 4, GQA, cross lengths, windows
+CASES = [(1, 1, 1, 1, 1, 16, True, 0), (2, 31, 31, 2, 1, 64, True, 0),
+         (1, 65, 65, 4, 2, 50, True, 33), (1, 130, 130, 2, 2, 128, True, 0),
+         (1, 33, 97, 4, 4, 100, False, 0), (1, 97, 32, 2, 1, 66, False, 0),
+         (2, 128, 128, 4, 4, 64, True, 0), (1, 64, 64, 3, 1, 110, True, 1)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c))
+def test_attention_fp32(dev, case):
+    from zorse_amd import kernels as K
+    B, Sq, Skv, Hq, Hkv, d, causal, window = case
+    print(f"attention fp32 {case}", flush=True)
+    q, do = _randn((B, Sq, Hq, d), 10, "cpu"), _randn((B, Sq, Hq, d), 11, "cpu")
+    k, v = _randn((B, Skv, Hkv, d), 12, "cpu"), _randn((B, Skv, Hkv, d), 13, "cpu")
+    dq_, dk_, dv_ = (t.to(dev) for t in (q, k, v))
+    o, lse = K.attn_fwd(dq_, dk_, dv_, causal=causal, window=window)
+    ro, rlse = O.attention(q.double(), k.double(), v.double(), causal, window)
+    assert_close(o, ro, torch.float32, "o")
+    assert_close(lse, rlse, torch.float32, "lse")
+    got = K.attn_bwd(dq_, dk_, dv_, o, do.to(dev), lse, causal=causal, window=window)
+    ref = O.attention_bwd(q.double(), k.double(), v.double(), do.double(), causal, window)
+    # dS = P (dP - delta) cancels (wholly for a query with one visible key):
+    # dP and delta are sums of d products, each off by up to (d + 2) 2^-24 of
+    # their absolute products, carried into dq / dk by k / q and the scale
+    big = [t.abs().max().item() for t in (do, v, q, k)]
+    floor = (d + 2) * 2.0 ** -24 * d * big[0] * big[1] * max(big[2:]) / d ** 0.5
+    for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+        diff = (g.double().cpu() - r).abs().max().item()
+        assert diff <= 1e-4 * r.abs().max().item() + (floor if name != "dv" else 0), (name, diff)
+
+
+def test_attention_fp32_masked_values_do_not_leak(dev):
+    """An infinity or NaN in a position a row does not see leaves the row's
+    result as it was, bit for bit within the sums' rounding: the last 9 tokens
+    hold infinities, the other rows match a run on the shorter sequence."""
+    from zorse_amd import kernels as K
+    S, keep, H, d = 70, 61, 2, 48
+    q, k, v, do = (_randn((2, S, H, d), 20 + i, dev) for i in range(4))
+    for t in (q, k, v, do):
+        t[:, keep:] = float("inf")
+        t[:, keep + 3] = float("nan")
+    o, lse = K.attn_fwd(q, k, v, causal=True)
+    short = [t[:, :keep].contiguous() for t in (q, k, v, do)]
+    so, slse = K.attn_fwd(*short[:3], causal=True)
+    assert_close(o[:, :keep], so.double(), torch.float32, "o")
+    assert_close(lse[..., :keep], slse.double(), torch.float32, "lse")
+    dq, _, _ = K.attn_bwd(q, k, v, o, do, lse, causal=True)
+    sdq, _, _ = K.attn_bwd(*short[:3], so, short[3], slse, causal=True)
+    assert_close(dq[:, :keep], sdq.double(), torch.float32, "dq")

@@ -37,39 +37,6 @@ namespace zk {
 int check_attn_desc(const zk_attn_desc* d, const char* who, bool bwd);
 void fill_args(AttnArgs& a, const zk_attn_desc* d);
 
-// ----------------------------------------------------------------- prep ----
-// fp32 path: 8 lanes per (b, q, h) row; each lane covers d/8 elements.
-// Writes delta = rowsum(dO o O) and lse2 = lse * log2(e) (+inf for an empty
-// row, so that exp2(s - lse2) = 0), both fp32 [B, Hq, Sq].  (The MFMA path
-// forms both inside attn_bwd_dq.)
-template <typename T>
-__global__ __launch_bounds__(256) void attn_bwd_prep(AttnArgs a) {
-  const int64_t rows = a.B * a.Sq * a.Hq;
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t row = gid >> 3;
-  const int sub = threadIdx.x & 7;
-  float acc = 0.f;
-  int64_t b = 0, q = 0, h = 0;
-  if (row < rows) {
-    h = row % a.Hq;
-    const int64_t bq = row / a.Hq;
-    q = bq % a.Sq;
-    b = bq / a.Sq;
-    const T* Or = static_cast<const T*>(a.o) + b * a.o_sb + q * a.o_ss + h * a.o_sh;
-    const T* Dr = static_cast<const T*>(a.dout) + b * a.o_sb + q * a.o_ss + h * a.o_sh;
-    for (int64_t e = sub; e < a.d; e += 8) acc = fmaf(to_f32(Or[e]), to_f32(Dr[e]), acc);
-  }
-  acc += __shfl_xor(acc, 1, 64);
-  acc += __shfl_xor(acc, 2, 64);
-  acc += __shfl_xor(acc, 4, 64);
-  if (row < rows && sub == 0) {
-    const int64_t i = (b * a.Hq + h) * a.Sq + q;
-    a.delta[i] = acc;
-    const float l = a.lse[i];
-    a.lse2[i] = l == -INFINITY ? INFINITY : l * kLog2e;
-  }
-}
-
 // ------------------------------------------------------------- dK / dV -----
 template <int D>
 struct DkdvCfg {
@@ -615,98 +582,6 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
   }
 }
 
-// ------------------------------------------------------------- fp32 path ---
-// Simple per-row kernels for fp32 layers (small shapes, no MFMA).
-
-// The inverse RoPE rotation of one row x[0 .. d) at sequence position `row`
-// (the same pairings and formula as rope_inverse_regs).
-__device__ __forceinline__ void rope_inverse_row(float* x, const AttnArgs& a, int64_t row) {
-  int64_t pos = a.rope_pos != nullptr ? a.rope_pos[row] : row;
-  if (pos < 0) pos = 0;
-  if (pos > a.rope_npos - 1) pos = a.rope_npos - 1;
-  const int64_t half = a.d / 2;
-  const float* ct = a.rope_cos + pos * half;
-  const float* st = a.rope_sin + pos * half;
-  for (int64_t i = 0; i < half; ++i) {
-    const int64_t ia = a.rope_interleaved ? 2 * i : i;
-    const int64_t ib = a.rope_interleaved ? 2 * i + 1 : i + half;
-    const float u = x[ia], w = x[ib];
-    x[ia] = fmaf(u, ct[i], w * st[i]);
-    x[ib] = fmaf(w, ct[i], -u * st[i]);
-  }
-}
-template <int D>
-__global__ __launch_bounds__(64) void attn_bwd_dq_f32(AttnArgs a) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
-  if (row >= a.B * a.Hq * a.Sq) return;
-  const int64_t qi = row % a.Sq, bh = row / a.Sq;
-  const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
-  const float* Q = static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh + qi * a.q_ss;
-  const float* dO = static_cast<const float*>(a.dout) + b * a.o_sb + hq * a.o_sh + qi * a.o_ss;
-  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
-  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
-  const float lse = a.lse[(b * a.Hq + hq) * a.Sq + qi];
-  const float del = a.delta[(b * a.Hq + hq) * a.Sq + qi];
-  float acc[D];
-  for (int e = 0; e < a.d; ++e) acc[e] = 0.f;
-  for (int64_t j = 0; j < a.Skv; ++j) {
-    if (!attn_visible(qi, j, a.Skv, a.causal, a.window)) continue;
-    const float* kr = K + j * a.k_ss;
-    const float* vr = V + j * a.v_ss;
-    float s = 0.f, dp = 0.f;
-    for (int e = 0; e < a.d; ++e) {
-      s = fmaf(Q[e], kr[e], s);
-      dp = fmaf(dO[e], vr[e], dp);
-    }
-    const float p = expf(s * a.scale - lse);
-    const float ds = p * (dp - del) * a.scale;
-    for (int e = 0; e < a.d; ++e) acc[e] = fmaf(ds, kr[e], acc[e]);
-  }
-  if (a.rope_cos != nullptr) rope_inverse_row(acc, a, qi);
-  float* dq = static_cast<float*>(a.dq) + b * a.dq_sb + hq * a.dq_sh + qi * a.dq_ss;
-  for (int e = 0; e < a.d; ++e) dq[e] = acc[e];
-}
-
-template <int D>
-__global__ __launch_bounds__(64) void attn_bwd_dkv_f32(AttnArgs a) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
-  if (row >= a.B * a.Hkv * a.Skv) return;
-  const int64_t kj = row % a.Skv, bh = row / a.Skv;
-  const int64_t b = bh / a.Hkv, hk = bh % a.Hkv;
-  const int64_t n_rep = a.Hq / a.Hkv;
-  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh + kj * a.k_ss;
-  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh + kj * a.v_ss;
-  float dk[D], dv[D];
-  for (int e = 0; e < a.d; ++e) { dk[e] = 0.f; dv[e] = 0.f; }
-  for (int64_t r = 0; r < n_rep; ++r) {
-    const int64_t hq = hk * n_rep + r;
-    const float* Q = static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh;
-    const float* dO = static_cast<const float*>(a.dout) + b * a.o_sb + hq * a.o_sh;
-    for (int64_t qi = 0; qi < a.Sq; ++qi) {
-      if (!attn_visible(qi, kj, a.Skv, a.causal, a.window)) continue;
-      const float* qr = Q + qi * a.q_ss;
-      const float* dr = dO + qi * a.o_ss;
-      float s = 0.f, dp = 0.f;
-      for (int e = 0; e < a.d; ++e) {
-        s = fmaf(qr[e], K[e], s);
-        dp = fmaf(dr[e], V[e], dp);
-      }
-      const float lse = a.lse[(b * a.Hq + hq) * a.Sq + qi];
-      const float del = a.delta[(b * a.Hq + hq) * a.Sq + qi];
-      const float p = expf(s * a.scale - lse);
-      const float ds = p * (dp - del) * a.scale;
-      for (int e = 0; e < a.d; ++e) {
-        dv[e] = fmaf(p, dr[e], dv[e]);
-        dk[e] = fmaf(ds, qr[e], dk[e]);
-      }
-    }
-  }
-  if (a.rope_cos != nullptr) rope_inverse_row(dk, a, kj);
-  float* dkp = static_cast<float*>(a.dk) + b * a.dk_sb + hk * a.dk_sh + kj * a.dk_ss;
-  float* dvp = static_cast<float*>(a.dv) + b * a.dv_sb + hk * a.dv_sh + kj * a.dv_ss;
-  for (int e = 0; e < a.d; ++e) { dkp[e] = dk[e]; dvp[e] = dv[e]; }
-}
-
 }  // namespace zk
 
 using namespace zk;
@@ -849,19 +724,8 @@ static int attn_bwd_impl(const char* who, const zk_attn_desc* desc, const void* 
   a.lse2 = a.delta + ((desc->B * desc->Hq * desc->Sq + 63) & ~int64_t(63));
   hipStream_t s = as_stream(stream);
 
-  const int64_t rows = desc->B * desc->Sq * desc->Hq;
-  const dim3 pgrid(static_cast<unsigned>((rows * 8 + 255) / 256));
   if (desc->dtype == ZK_F32) {
-    if (rows > 0) hipLaunchKernelGGL(attn_bwd_prep<float>, pgrid, dim3(256), 0, s, a);
-    const int64_t qrows = desc->B * desc->Hq * desc->Sq;
-    const int64_t krows = desc->B * desc->Hkv * desc->Skv;
-    if (desc->d <= 64) {
-      if (qrows > 0) hipLaunchKernelGGL(attn_bwd_dq_f32<64>, dim3((qrows + 63) / 64), dim3(64), 0, s, a);
-      if (krows > 0) hipLaunchKernelGGL(attn_bwd_dkv_f32<64>, dim3((krows + 63) / 64), dim3(64), 0, s, a);
-    } else {
-      if (qrows > 0) hipLaunchKernelGGL(attn_bwd_dq_f32<128>, dim3((qrows + 63) / 64), dim3(64), 0, s, a);
-      if (krows > 0) hipLaunchKernelGGL(attn_bwd_dkv_f32<128>, dim3((krows + 63) / 64), dim3(64), 0, s, a);
-    }
+    launch_attn_bwd_f32(a, s);
     return launch_status(who);
   }
   ZK_REQUIRE(aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(o, 16) &&

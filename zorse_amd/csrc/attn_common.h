@@ -52,6 +52,11 @@ struct AttnArgs {
   int64_t t_ld;
 };
 
+// fp32 attention (attn_f32.hip): the forward, and the backward's two kernels
+// (its workspace's delta and lse2 hold rowsum(dO o O) and the natural LSE).
+void launch_attn_fwd_f32(const AttnArgs& a, hipStream_t s);
+void launch_attn_bwd_f32(const AttnArgs& a, hipStream_t s);
+
 // Transposed store of a workgroup's rows (of O or a gradient): lane l of wave w holds
 // x[nt][j] = element 32 nt + 8 (j / 4) + 4 g + j % 4 (g = l / 32) of row
 // 32 w + l % 32 (the MFMA accumulator layout), NCOL = 32 x (waves) rows in

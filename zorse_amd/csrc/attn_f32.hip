@@ -1,0 +1,504 @@
+// Attention for fp32 layers, forward and backward, on the fp32 matrix cores
+// (v_mfma_f32_16x16x4f32: full fp32 products and sums), any head dim up to
+// 128 (zero-padded to D = 64 or 128 in registers and LDS).
+//
+// Workgroup = 4 waves, 16 queries (forward, dQ) or 16 keys (dK / dV) per
+// wave; the other side streams through LDS in tiles of 32 rows, the next
+// tile's global loads in flight in registers during the current one's math.
+// The arrangement is the 16-bit kernels' (attn_fwd.hip, attn_bwd.hip): scores
+// transposed in the forward and dQ (a lane owns one query and 4 keys of each
+// 16-key block, so the softmax is per lane plus two exchanges), probabilities
+// straight from the accumulators into the next product's operand, dQ by its
+// own pass, nothing accumulated through memory.
+//
+// Operands.  The MFMA takes one float per lane: row (or column) l % 16 and k
+// index l / 16.  Both operands of a product may permute k alike, so a 16-byte
+// LDS read of elements 16 c + 4 (l / 16) .. + 3 serves four MFMAs; and the
+// accumulator's rows 4 (l / 16) + e make operand e of the product that
+// consumes them, whose other operand reads those rows' elements.  LDS rows
+// are padded to D + 4 floats: both read patterns spread over the banks.
+//
+// Bound by latency at the sizes fp32 layers have (the parity layer's shape, 2
+// sequences x 4 heads x 128 x 64, is 16 workgroups).  There a thread per row
+// took 1770 us forward, 1955 us for dQ and 1976 us for dK / dV; these kernels
+// take 16, 26 and 31 us.
+#include "attn_common.h"
+#include "vec.h"
+
+namespace zk {
+
+namespace {
+
+constexpr int kTile = 32;  // rows per LDS tile
+
+// Rows r0 .. r0 + 31 (of `rows`) of a [.., d] tensor, D / 8 floats per
+// thread: load() issues the global loads, store() writes the LDS tile.
+template <int D, bool kVec>
+struct TileReg {
+  static constexpr int NC = kTile * D / 4 / 256;  // 4-float chunks per thread
+  float4 v[NC];
+  __device__ __forceinline__ void load(const float* base, int64_t ld, int64_t r0, int64_t rows, int d) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int id = i * 256 + static_cast<int>(threadIdx.x);
+      const int r = id / (D / 4), c = 4 * (id % (D / 4));
+      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (r0 + r < rows && c < d) {
+        const float* p = base + (r0 + r) * ld + c;
+        if (kVec) {
+          x = *reinterpret_cast<const float4*>(p);
+        } else {
+          x.x = p[0];
+          if (c + 1 < d) x.y = p[1];
+          if (c + 2 < d) x.z = p[2];
+          if (c + 3 < d) x.w = p[3];
+        }
+      }
+      v[i] = x;
+    }
+  }
+  // returns whether one of this thread's values is an infinity or NaN
+  __device__ __forceinline__ int store(float* tile) const {
+    float z = 0.f;  // stays 0 for finite values, else NaN
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int id = i * 256 + static_cast<int>(threadIdx.x);
+      *reinterpret_cast<float4*>(&tile[(id / (D / 4)) * (D + 4) + 4 * (id % (D / 4))]) = v[i];
+      z += 0.f * v[i].x + 0.f * v[i].y + 0.f * v[i].z + 0.f * v[i].w;
+    }
+    return z != 0.f;
+  }
+};
+
+// This lane's operand of row `row` (null: zeros): elements 16 c + 4 q4 .. + 3.
+template <int D, bool kVec>
+__device__ __forceinline__ void load_row(float4 (&x)[D / 16], const float* row, int d) {
+  const int q4 = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c) {
+    const int e = 16 * c + 4 * q4;
+    x[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row == nullptr || e >= d) continue;
+    if (kVec) {
+      x[c] = *reinterpret_cast<const float4*>(row + e);
+    } else {
+      x[c].x = row[e];
+      if (e + 1 < d) x[c].y = row[e + 1];
+      if (e + 2 < d) x[c].z = row[e + 2];
+      if (e + 3 < d) x[c].w = row[e + 3];
+    }
+  }
+}
+
+__device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// X Y^T over d of the LDS rows row0 .. + 15 (X) and this lane's operand y.
+template <int D>
+__device__ __forceinline__ f32x4 dot_rows(const float* tile, int row0, const float4 (&y)[D / 16]) {
+  const int l16 = threadIdx.x & 15, q4 = (threadIdx.x & 63) >> 4;
+  const float* p = tile + (row0 + l16) * (D + 4) + 4 * q4;
+  f32x4 s{};
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c) {
+    const float4 x = *reinterpret_cast<const float4*>(p + 16 * c);
+    s = mma4(x.x, y[c].x, s);
+    s = mma4(x.y, y[c].y, s);
+    s = mma4(x.z, y[c].z, s);
+    s = mma4(x.w, y[c].w, s);
+  }
+  return s;
+}
+
+// acc^T += X^T w over the 16 LDS rows row0 ..: w[e] belongs to row 4 q4 + e.
+template <int D>
+__device__ __forceinline__ void add_rows(f32x4 (&acc)[D / 16], const float* tile, int row0,
+                                         const f32x4& w) {
+  const int l16 = threadIdx.x & 15, q4 = (threadIdx.x & 63) >> 4;
+  const float* p = tile + (row0 + 4 * q4) * (D + 4) + l16;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int nt = 0; nt < D / 16; ++nt)
+      acc[nt] = mma4(p[e * (D + 4) + 16 * nt], w[e], acc[nt]);
+}
+
+// The same for a tile that holds an infinity or NaN, where a product with the
+// zero weight of a masked row would be NaN: row by row, masked rows left out.
+template <int D, typename Vis>
+__device__ __forceinline__ void add_rows_visible(f32x4 (&acc)[D / 16], const float* tile, int row0,
+                                              const f32x4& w, Vis visible) {
+  const int l16 = threadIdx.x & 15, q4 = (threadIdx.x & 63) >> 4;
+  for (int r = 0; r < 16; ++r) {
+    float wr = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wr = (r & 3) == e ? w[e] : wr;
+    wr = __shfl(wr, (r >> 2) * 16 + l16, 64);
+    if (!visible(row0 + r)) continue;
+#pragma unroll
+    for (int nt = 0; nt < D / 16; ++nt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[nt][e] = fmaf(wr, tile[(row0 + r) * (D + 4) + 16 * nt + 4 * q4 + e], acc[nt][e]);
+  }
+}
+
+// sum / max over the four lane groups that share a column
+__device__ __forceinline__ float group_sum(float x) {
+  x += __shfl_xor(x, 16, 64);
+  return x + __shfl_xor(x, 32, 64);
+}
+__device__ __forceinline__ float group_max(float x) {
+  x = fmaxf(x, __shfl_xor(x, 16, 64));
+  return fmaxf(x, __shfl_xor(x, 32, 64));
+}
+
+// This lane's accumulators (elements 16 nt + 4 q4 + e of its row), scaled, to
+// the row at dst.
+template <int D, bool kVec>
+__device__ __forceinline__ void store_row(float* dst, const f32x4 (&x)[D / 16], float scale, int d) {
+  const int q4 = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int nt = 0; nt < D / 16; ++nt) {
+    const int e0 = 16 * nt + 4 * q4;
+    if (kVec) {
+      if (e0 < d)
+        *reinterpret_cast<float4*>(dst + e0) = make_float4(x[nt][0] * scale, x[nt][1] * scale,
+                                                           x[nt][2] * scale, x[nt][3] * scale);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e0 + e < d) dst[e0 + e] = x[nt][e] * scale;
+    }
+  }
+}
+
+// The transpose of the RoPE rotation on one row of a tensor just stored
+// (gradients of queries / keys the forward rotated), by the 16-lane column's
+// four lanes after a barrier: pairs (i, i + d / 2) or (2 i, 2 i + 1), the
+// formula of rope_inverse_regs.
+__device__ __forceinline__ void rope_inverse_row(float* x, const AttnArgs& a, int64_t row, int q4) {
+  int64_t pos = a.rope_pos != nullptr ? a.rope_pos[row] : row;
+  if (pos < 0) pos = 0;
+  if (pos > a.rope_npos - 1) pos = a.rope_npos - 1;
+  const int half = static_cast<int>(a.d / 2);
+  const float* ct = a.rope_cos + pos * half;
+  const float* st = a.rope_sin + pos * half;
+  for (int i = q4; i < half; i += 4) {
+    const int ia = a.rope_interleaved ? 2 * i : i;
+    const int ib = a.rope_interleaved ? 2 * i + 1 : i + half;
+    const float u = x[ia], w = x[ib];
+    x[ia] = fmaf(u, ct[i], w * st[i]);
+    x[ib] = fmaf(w, ct[i], -u * st[i]);
+  }
+}
+
+// Rows of the other side that rows r0 .. r0 + n - 1 of one side meet, as a
+// tile range [lo, hi): keys for queries (kKeys) or queries for keys.
+template <bool kKeys>
+__device__ __forceinline__ void tile_range(const AttnArgs& a, int64_t r0, int64_t n, int64_t& lo,
+                                           int64_t& hi) {
+  lo = 0;
+  hi = kKeys ? a.Skv : a.Sq;
+  if (kKeys) {
+    if (a.causal && hi > r0 + n) hi = r0 + n;
+    if (a.window > 0 && r0 - a.window + 1 > lo) lo = r0 - a.window + 1;
+  } else {
+    if (a.causal) lo = r0;
+    if (a.window > 0 && r0 + n - 1 + a.window < hi) hi = r0 + n - 1 + a.window;
+  }
+  lo /= kTile;
+  hi = hi > lo * kTile ? (hi + kTile - 1) / kTile : lo;
+}
+
+template <int D, bool kVec>
+__global__ __launch_bounds__(256) void attn_fwd_f32(AttnArgs a, int64_t n_qt) {
+  __shared__ __attribute__((aligned(16))) float Ks[kTile * (D + 4)], Vs[kTile * (D + 4)];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
+  const int64_t nbh = a.B * a.Hq, qt = n_qt - 1 - blockIdx.x / nbh, bh = blockIdx.x % nbh;
+  const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
+  const int64_t q0 = qt * 64, my_q = q0 + 16 * wave + l16;
+  const int d = static_cast<int>(a.d);
+  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
+  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
+  float4 q[D / 16];
+  load_row<D, kVec>(q, my_q < a.Sq ? static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh +
+                                         my_q * a.q_ss : nullptr, d);
+  f32x4 o[D / 16];
+#pragma unroll
+  for (int nt = 0; nt < D / 16; ++nt) o[nt] = f32x4{};
+  float m = -INFINITY, l = 0.f;
+  int64_t t0, t1;
+  tile_range<true>(a, q0, 64, t0, t1);
+  TileReg<D, kVec> kr, vr;
+  if (t0 < t1) {
+    kr.load(K, a.k_ss, t0 * kTile, a.Skv, d);
+    vr.load(V, a.v_ss, t0 * kTile, a.Skv, d);
+  }
+  for (int64_t t = t0; t < t1; ++t) {
+    __syncthreads();  // the previous tile's reads are done
+    kr.store(Ks);
+    const bool odd = __syncthreads_or(vr.store(Vs));
+    auto visible = [&](int r) __attribute__((always_inline)) {
+      return attn_visible(my_q, t * kTile + r, a.Skv, a.causal, a.window);
+    };
+    if (t + 1 < t1) {
+      kr.load(K, a.k_ss, (t + 1) * kTile, a.Skv, d);
+      vr.load(V, a.v_ss, (t + 1) * kTile, a.Skv, d);
+    }
+    f32x4 s[2];
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[h] = dot_rows<D>(Ks, 16 * h, q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[h][e] = visible(16 * h + 4 * q4 + e) ? s[h][e] * a.scale : -INFINITY;
+        mloc = fmaxf(mloc, s[h][e]);
+      }
+    }
+    const float m_new = fmaxf(m, group_max(mloc));
+    const float ref = m_new == -INFINITY ? 0.f : m_new;  // nothing visible yet
+    const float alpha = expf(m - ref);
+    m = m_new;
+    l *= alpha;
+#pragma unroll
+    for (int nt = 0; nt < D / 16; ++nt) o[nt] *= alpha;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[h][e] = expf(s[h][e] - ref);
+        l += s[h][e];
+      }
+      if (odd)
+        add_rows_visible<D>(o, Vs, 16 * h, s[h], visible);
+      else
+        add_rows<D>(o, Vs, 16 * h, s[h]);
+    }
+  }
+  l = group_sum(l);
+  if (my_q >= a.Sq) return;
+  store_row<D, kVec>(static_cast<float*>(a.out) + b * a.o_sb + hq * a.o_sh + my_q * a.o_ss, o,
+                     l > 0.f ? 1.0f / l : 0.f, d);
+  if (q4 == 0) a.lse_out[(b * a.Hq + hq) * a.Sq + my_q] = l > 0.f ? m + logf(l) : -INFINITY;
+}
+
+// dQ, and delta = rowsum(dO o O) for the dK / dV kernel that follows.
+template <int D, bool kVec>
+__global__ __launch_bounds__(256) void attn_bwd_dq_f32(AttnArgs a, int64_t n_qt) {
+  __shared__ __attribute__((aligned(16))) float Ks[kTile * (D + 4)], Vs[kTile * (D + 4)];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
+  const int64_t nbh = a.B * a.Hq, qt = n_qt - 1 - blockIdx.x / nbh, bh = blockIdx.x % nbh;
+  const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
+  const int64_t q0 = qt * 64, my_q = q0 + 16 * wave + l16;
+  const int d = static_cast<int>(a.d);
+  const bool in = my_q < a.Sq;
+  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
+  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
+  const int64_t orow = b * a.o_sb + hq * a.o_sh + my_q * a.o_ss;
+  float4 q[D / 16], g[D / 16];
+  load_row<D, kVec>(q, in ? static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh + my_q * a.q_ss
+                          : nullptr, d);
+  load_row<D, kVec>(g, in ? static_cast<const float*>(a.dout) + orow : nullptr, d);
+  float lse = INFINITY, del = 0.f;
+  {
+    float4 ov[D / 16];
+    load_row<D, kVec>(ov, in ? static_cast<const float*>(a.o) + orow : nullptr, d);
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      del = fmaf(ov[c].x, g[c].x, del);
+      del = fmaf(ov[c].y, g[c].y, del);
+      del = fmaf(ov[c].z, g[c].z, del);
+      del = fmaf(ov[c].w, g[c].w, del);
+    }
+    del = group_sum(del);
+    if (in) {
+      const int64_t i = (b * a.Hq + hq) * a.Sq + my_q;
+      lse = a.lse[i];
+      if (lse == -INFINITY) lse = INFINITY;  // an empty row: probabilities 0
+      if (q4 == 0) {
+        a.delta[i] = del;
+        a.lse2[i] = lse;
+      }
+    }
+  }
+  f32x4 dq[D / 16];
+#pragma unroll
+  for (int nt = 0; nt < D / 16; ++nt) dq[nt] = f32x4{};
+  int64_t t0, t1;
+  tile_range<true>(a, q0, 64, t0, t1);
+  TileReg<D, kVec> kr, vr;
+  if (t0 < t1) {
+    kr.load(K, a.k_ss, t0 * kTile, a.Skv, d);
+    vr.load(V, a.v_ss, t0 * kTile, a.Skv, d);
+  }
+  for (int64_t t = t0; t < t1; ++t) {
+    __syncthreads();
+    vr.store(Vs);
+    const bool odd = __syncthreads_or(kr.store(Ks));
+    auto visible = [&](int r) __attribute__((always_inline)) {
+      return in && attn_visible(my_q, t * kTile + r, a.Skv, a.causal, a.window);
+    };
+    if (t + 1 < t1) {
+      kr.load(K, a.k_ss, (t + 1) * kTile, a.Skv, d);
+      vr.load(V, a.v_ss, (t + 1) * kTile, a.Skv, d);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4 s = dot_rows<D>(Ks, 16 * h, q);
+      const f32x4 dp = dot_rows<D>(Vs, 16 * h, g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[e] = visible(16 * h + 4 * q4 + e) ? expf(s[e] * a.scale - lse) * (dp[e] - del) : 0.f;
+      }
+      if (odd)
+        add_rows_visible<D>(dq, Ks, 16 * h, s, visible);
+      else
+        add_rows<D>(dq, Ks, 16 * h, s);
+    }
+  }
+  float* out = static_cast<float*>(a.dq) + b * a.dq_sb + hq * a.dq_sh + my_q * a.dq_ss;
+  if (in) store_row<D, kVec>(out, dq, a.scale, d);
+  if (a.rope_cos != nullptr) {
+    __syncthreads();  // the row's four lanes have stored it
+    if (in) rope_inverse_row(out, a, my_q, q4);
+  }
+}
+
+// dK and dV of 64 keys per workgroup, summed over the query heads of the
+// group; after attn_bwd_dq_f32 (delta, lse2).
+template <int D, bool kVec>
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_f32(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) float Qs[kTile * (D + 4)], Gs[kTile * (D + 4)];
+  __shared__ __attribute__((aligned(16))) float ls[kTile], ds[kTile];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
+  const int64_t nbh = a.B * a.Hkv, kt = blockIdx.x / nbh, bh = blockIdx.x % nbh;
+  const int64_t b = bh / a.Hkv, hk = bh % a.Hkv, n_rep = a.Hq / a.Hkv;
+  const int64_t k0 = kt * 64, my_k = k0 + 16 * wave + l16;
+  const int d = static_cast<int>(a.d);
+  const bool in = my_k < a.Skv;
+  float4 k[D / 16], v[D / 16];
+  load_row<D, kVec>(k, in ? static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh + my_k * a.k_ss
+                          : nullptr, d);
+  load_row<D, kVec>(v, in ? static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh + my_k * a.v_ss
+                          : nullptr, d);
+  f32x4 dk[D / 16], dv[D / 16];
+#pragma unroll
+  for (int nt = 0; nt < D / 16; ++nt) {
+    dk[nt] = f32x4{};
+    dv[nt] = f32x4{};
+  }
+  int64_t t0, t1;
+  tile_range<false>(a, k0, 64, t0, t1);
+  const int64_t nt = t1 - t0, n_it = nt * n_rep;
+  TileReg<D, kVec> qr, gr;
+  float lr = 0.f, dr = 0.f;
+  auto load = [&](int64_t it) __attribute__((always_inline)) {
+    const int64_t hq = hk * n_rep + it / nt, r0 = (t0 + it % nt) * kTile;
+    qr.load(static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh, a.q_ss, r0, a.Sq, d);
+    gr.load(static_cast<const float*>(a.dout) + b * a.o_sb + hq * a.o_sh, a.o_ss, r0, a.Sq, d);
+    if (threadIdx.x < kTile) {
+      const int64_t qi = r0 + threadIdx.x, i = (b * a.Hq + hq) * a.Sq + qi;
+      lr = qi < a.Sq ? a.lse2[i] : INFINITY;
+      dr = qi < a.Sq ? a.delta[i] : 0.f;
+    }
+  };
+  if (n_it > 0) load(0);
+  for (int64_t it = 0; it < n_it; ++it) {
+    __syncthreads();
+    const int odd_q = qr.store(Qs), odd_g = gr.store(Gs);
+    if (threadIdx.x < kTile) {
+      ls[threadIdx.x] = lr;
+      ds[threadIdx.x] = dr;
+    }
+    const bool odd = __syncthreads_or(odd_q | odd_g);
+    if (it + 1 < n_it) load(it + 1);
+    const int64_t r0 = (t0 + it % nt) * kTile;
+    auto visible = [&](int r) __attribute__((always_inline)) {
+      return in && r0 + r < a.Sq && attn_visible(r0 + r, my_k, a.Skv, a.causal, a.window);
+    };
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 s = dot_rows<D>(Qs, 16 * h, k);
+      const f32x4 dp = dot_rows<D>(Gs, 16 * h, v);
+      f32x4 p, w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 16 * h + 4 * q4 + e;
+        const bool vis = visible(r);
+        p[e] = vis ? expf(s[e] * a.scale - ls[r]) : 0.f;
+        w[e] = vis ? p[e] * (dp[e] - ds[r]) : 0.f;
+      }
+      if (odd) {
+        add_rows_visible<D>(dv, Gs, 16 * h, p, visible);
+        add_rows_visible<D>(dk, Qs, 16 * h, w, visible);
+      } else {
+        add_rows<D>(dv, Gs, 16 * h, p);
+        add_rows<D>(dk, Qs, 16 * h, w);
+      }
+    }
+  }
+  float* dkp = static_cast<float*>(a.dk) + b * a.dk_sb + hk * a.dk_sh + my_k * a.dk_ss;
+  if (in) {
+    store_row<D, kVec>(dkp, dk, a.scale, d);
+    store_row<D, kVec>(static_cast<float*>(a.dv) + b * a.dv_sb + hk * a.dv_sh + my_k * a.dv_ss, dv,
+                       1.f, d);
+  }
+  if (a.rope_cos != nullptr) {
+    __syncthreads();
+    if (in) rope_inverse_row(dkp, a, my_k, q4);
+  }
+}
+
+// float4 accesses: head dim and strides multiples of 4, pointers of 16 bytes
+bool vec4_ok(int64_t d, std::initializer_list<int64_t> strides,
+             std::initializer_list<const void*> ptrs) {
+  if (d % 4 != 0) return false;
+  for (int64_t s : strides)
+    if (s % 4 != 0) return false;
+  for (const void* p : ptrs)
+    if (!aligned(p, 16)) return false;
+  return true;
+}
+
+}  // namespace
+
+#define ZK_F32_DISPATCH(KERNEL, GRID, ...)                                                   \
+  do {                                                                                       \
+    if (a.d <= 64 && vec)                                                                    \
+      hipLaunchKernelGGL((KERNEL<64, true>), GRID, dim3(256), 0, s, __VA_ARGS__);            \
+    else if (a.d <= 64)                                                                      \
+      hipLaunchKernelGGL((KERNEL<64, false>), GRID, dim3(256), 0, s, __VA_ARGS__);           \
+    else if (vec)                                                                            \
+      hipLaunchKernelGGL((KERNEL<128, true>), GRID, dim3(256), 0, s, __VA_ARGS__);           \
+    else                                                                                     \
+      hipLaunchKernelGGL((KERNEL<128, false>), GRID, dim3(256), 0, s, __VA_ARGS__);          \
+  } while (0)
+
+void launch_attn_fwd_f32(const AttnArgs& a, hipStream_t s) {
+  const bool vec = vec4_ok(a.d, {a.q_sb, a.q_ss, a.q_sh, a.k_sb, a.k_ss, a.k_sh, a.v_sb, a.v_ss,
+                                 a.v_sh, a.o_sb, a.o_ss, a.o_sh}, {a.q, a.k, a.v, a.out});
+  const int64_t n_qt = (a.Sq + 63) / 64;
+  const dim3 grid(static_cast<unsigned>(n_qt * a.B * a.Hq));
+  ZK_F32_DISPATCH(attn_fwd_f32, grid, a, n_qt);
+}
+
+void launch_attn_bwd_f32(const AttnArgs& a, hipStream_t s) {
+  const bool vec = vec4_ok(a.d, {a.q_sb, a.q_ss, a.q_sh, a.k_sb, a.k_ss, a.k_sh, a.v_sb, a.v_ss,
+                                 a.v_sh, a.o_sb, a.o_ss, a.o_sh, a.dq_sb, a.dq_ss, a.dq_sh, a.dk_sb,
+                                 a.dk_ss, a.dk_sh, a.dv_sb, a.dv_ss, a.dv_sh},
+                           {a.q, a.k, a.v, a.o, a.dout, a.dq, a.dk, a.dv});
+  const int64_t n_qt = (a.Sq + 63) / 64, n_kt = (a.Skv + 63) / 64;
+  if (n_qt > 0) {
+    const dim3 grid(static_cast<unsigned>(n_qt * a.B * a.Hq));
+    ZK_F32_DISPATCH(attn_bwd_dq_f32, grid, a, n_qt);
+  }
+  if (n_kt > 0) {
+    const dim3 grid(static_cast<unsigned>(n_kt * a.B * a.Hkv));
+    ZK_F32_DISPATCH(attn_bwd_dkdv_f32, grid, a);
+  }
+}
+
+}  // namespace zk

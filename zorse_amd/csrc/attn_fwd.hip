@@ -289,44 +289,6 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
   }
 }
 
-// --------------------------------------------------------------------------
-// fp32 path: one thread per query row, online softmax over all keys with the
-// row kept in registers.  Used for fp32 layers (small shapes); no MFMA.
-template <int D>
-__global__ __launch_bounds__(64) void attn_fwd_f32_kernel(AttnArgs a) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
-  const int64_t total = a.B * a.Hq * a.Sq;
-  if (row >= total) return;
-  const int64_t qi = row % a.Sq;
-  const int64_t bh = row / a.Sq;
-  const int64_t b = bh / a.Hq, hq = bh % a.Hq;
-  const int64_t hk = hq / (a.Hq / a.Hkv);
-  const float* Q = static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh + qi * a.q_ss;
-  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
-  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
-  float q[D], acc[D];
-  for (int e = 0; e < D; ++e) { q[e] = e < a.d ? Q[e] : 0.f; acc[e] = 0.f; }
-  float m = -INFINITY, l = 0.f;
-  for (int64_t j = 0; j < a.Skv; ++j) {
-    if (!attn_visible(qi, j, a.Skv, a.causal, a.window)) continue;
-    const float* kr = K + j * a.k_ss;
-    float s = 0.f;
-    for (int e = 0; e < a.d; ++e) s = fmaf(q[e], kr[e], s);
-    s *= a.scale;
-    const float m_new = fmaxf(m, s);
-    const float alpha = expf(m - m_new);
-    const float p = expf(s - m_new);
-    l = l * alpha + p;
-    const float* vr = V + j * a.v_ss;
-    for (int e = 0; e < a.d; ++e) acc[e] = fmaf(acc[e], alpha, p * vr[e]);
-    m = m_new;
-  }
-  float* O = static_cast<float*>(a.out) + b * a.o_sb + hq * a.o_sh + qi * a.o_ss;
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
-  for (int e = 0; e < a.d; ++e) O[e] = acc[e] * inv;
-  a.lse_out[(b * a.Hq + hq) * a.Sq + qi] = l > 0.f ? m + logf(l) : -INFINITY;
-}
-
 }  // namespace zk
 
 using namespace zk;
@@ -418,12 +380,7 @@ static int attn_fwd_impl(const char* who, const zk_attn_desc* desc, const void* 
   a.t_ld = ld_t;
   hipStream_t s = as_stream(stream);
   if (desc->dtype == ZK_F32) {
-    const int64_t rows = desc->B * desc->Hq * desc->Sq;
-    const dim3 grid(static_cast<unsigned>((rows + 63) / 64));
-    if (desc->d <= 64)
-      hipLaunchKernelGGL(attn_fwd_f32_kernel<64>, grid, dim3(64), 0, s, a);
-    else
-      hipLaunchKernelGGL(attn_fwd_f32_kernel<128>, grid, dim3(64), 0, s, a);
+    launch_attn_fwd_f32(a, s);
     return launch_status(who);
   }
   ZK_REQUIRE(aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(o, 16),
