@@ -27,17 +27,18 @@ static bool tiled_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km, 
 }
 
 // Whether the MFMA kernels whose edges are masked (the RAG form of the 256 x
-// 256 pipeline, gemm_ring.h) take a launch: 2-byte type, every 8-element run
-// of an operand whole and 16-byte aligned -- N a multiple of 8 (stores), K of
-// 8 for an operand along K, M of 8 for a K-major A, leading dimensions of 8
-// -- and tiles within one buffer resource, as above.  Pointer alignment is
-// checked by the caller.
+// 256 pipeline, gemm_ring.h) take a launch: every 8-element run of an operand
+// whole and 16-byte aligned -- N a multiple of 8 (stores), K of 8 for an
+// operand along K, M of 8 for a K-major A, leading dimensions of 8 -- and
+// tiles within one buffer resource (fp32: half the leading dimensions above).
+// Pointer alignment is checked by the caller.
 static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km, int64_t ldb,
                          int b_km, int64_t ldc, int64_t ldr, int dtype) {
-  if (dtype != ZK_BF16 && dtype != ZK_F16) return false;
   if (M <= 0 || N <= 0 || K <= 0 || N % 8 || (a_km ? M : K) % 8 || (!b_km && K % 8)) return false;
   if (lda % 8 || ldb % 8 || ldc % 8 || ldr % 8 || M >= 0x7fffffffLL) return false;
-  const int64_t lim_a = int64_t(1) << (a_km ? 24 : 22), lim_b = int64_t(1) << (b_km ? 24 : 22);
+  const int wide = dtype == ZK_F32 ? 1 : 0;
+  const int64_t lim_a = int64_t(1) << ((a_km ? 24 : 22) - wide),
+                lim_b = int64_t(1) << ((b_km ? 24 : 22) - wide);
   return lda < lim_a && ldb < lim_b &&
          gemm::tile_count(gemm::k64, M, N) < 0x7fffffffLL;
 }
@@ -204,7 +205,9 @@ extern "C" int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, 
   ga.N = N;
   ga.K = K;
   hipStream_t s = as_stream(stream);
-  if (mfma)
+  if (mfma && dtype == ZK_F32)
+    gemm::launch_ring_f32(a_km, b_km, ga, s);
+  else if (mfma)
     launch_mfma<0>(dtype == ZK_BF16, a_km && !b_km && on_grid ? gemm::k256 : pick_tile(M, N, K, a_km, b_km),
                    on_grid, a_km, b_km, ga, s);
   else if (dtype == ZK_BF16)
@@ -254,7 +257,7 @@ extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t l
   ZK_REQUIRE(c != nullptr && (K == 0 || (a != nullptr && b != nullptr)), ZK_EINVAL,
              "zk_gemm_rope: null pointer");
   const bool on_grid = tiled_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype);
-  bool epi = (on_grid || masked_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype)) && aligned(a, 16) &&
+  bool epi = dtype != ZK_F32 && masked_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype) && aligned(a, 16) &&
              aligned(b, 16) && aligned(c, 16) && (head_dim == 64 || head_dim == 128) &&
              aligned(cos, 16) && aligned(sin, 16) && S < (int64_t(1) << 30) &&
              n_pos < (int64_t(1) << 24);

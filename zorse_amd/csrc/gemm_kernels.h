@@ -42,8 +42,8 @@
 //
 // Shapes off that grid take the same kernel with its edges masked (RAG) or the
 // small-tile kernel of gemm_ring.h, whichever gemm.hip's cost rule names.
-// fp32 operands, layouts that are not 16-byte aligned and leading dimensions
-// past the buffer-resource range go to gemm_gen_kernel: 128 x 128 tiles
+// Layouts that are not 16-byte aligned and leading dimensions past the
+// buffer-resource range go to gemm_gen_kernel: 128 x 128 tiles
 // staged through registers with masked loads and stores (any M, N, K).
 //
 // This header holds the kernels; gemm.hip launches the NT forms (the
@@ -739,9 +739,8 @@ void gemm_tiled_kernel(GemmArgs args) {
 // (out-of-range elements are zero), written to LDS as [128 rows][32 k] (k
 // contiguous, padded rows), and consumed by v_mfma_f32_16x16x32 (2-byte
 // types) or v_mfma_f32_16x16x4f32 (fp32, full fp32 products).  Stores are
-// masked per element.  This is the path for fp32 layers and for 2-byte
-// operands the DMA kernels cannot load (16-byte alignment); it needs no
-// alignment beyond the element's.
+// masked per element.  This is the path for operands the DMA kernels cannot
+// load (16-byte alignment); it needs no alignment beyond the element's.
 constexpr int GBM = 128, GBK = 32;
 
 template <typename T>
@@ -876,6 +875,8 @@ void launch_ring(bool bf16, int epi, bool a_kmajor, bool b_kmajor, Tile t, const
                  hipStream_t s);
 void launch_ring_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, Tile t, const GemmArgs& ga,
                         hipStream_t s);
+// fp32 (gemm_f32.hip)
+void launch_ring_f32(bool a_kmajor, bool b_kmajor, const GemmArgs& ga, hipStream_t s);
 
 }  // namespace gemm
 

@@ -1,4 +1,4 @@
-// The small-tile MFMA GEMM for bf16 / fp16, any M, N and K:
+// The small-tile MFMA GEMM for bf16 / fp16 and fp32, any M, N and K:
 //
 //   C[M, N] = op(A) op(B)^T (+ R[M, N])
 //
@@ -7,7 +7,8 @@
 // grid, and products whose large tiles would leave CUs idle.
 //
 // Workgroup = 4 waves in a 2 x 2 arrangement over a tile of 32 MB x 32 NB,
-// each wave MB x NB blocks of v_mfma_f32_16x16x32; K advances by 64.  Tiles
+// each wave MB x NB blocks of v_mfma_f32_16x16x32; K advances by 64 (fp32:
+// v_mfma_f32_16x16x4f32, by 32: the same 128 bytes per tile row).  Tiles
 // reach LDS through buffer_load_dwordx4 ... lds.  B sits in a ring of RB
 // stages and A in one of RB + 1, so loads run RB K steps ahead; operands are
 // double-buffered in registers across the 32-deep substeps, and each K step
@@ -33,28 +34,37 @@
 namespace zk {
 namespace gemm {
 
-// Swizzle of a K-major tile of COLS columns (see kmaj_sw for 256): the eight
-// rows {k0 .. k0 + 3, k0 + 8 .. k0 + 11} that one transposed read of a
+// Elements of one K step of a tile row (128 bytes).
+template <typename T>
+constexpr int kStep = 128 / static_cast<int>(sizeof(T));
+
+// Swizzle of a K-major tile of COLS columns: k-row k's 16-byte chunk c sits at
+// chunk position c ^ sw.  2-byte types (see kmaj_sw for 256 columns): the
+// eight rows {k0 .. k0 + 3, k0 + 8 .. k0 + 11} that one transposed read of a
 // 32-lane half touches go to eight different 32-byte groups of a 256-byte
 // bank row.  128 columns: one row fills a bank row, as for 256.  64 columns:
-// two rows share one (k & 1 picks the half), four chunk pairs remain; 32
-// columns: four rows share one, two pairs remain.
-template <int COLS>
+// two rows share one (k & 1 picks the half), four chunk pairs remain.  fp32:
+// an operand read takes one float of rows 4 (l / 16) + j, which land on four
+// different 64-byte segments.
+template <typename T, int COLS>
 __device__ __forceinline__ int kmaj_sw_n(int k) {
+  if (sizeof(T) == 4) return 4 * ((k >> 2) & 3);
   if (COLS >= 128) return 2 * ((k & 3) | ((k >> 1) & 4));
-  if (COLS == 64) return 2 * (((k >> 1) & 1) | ((k >> 2) & 2));
-  return 2 * ((k >> 3) & 1);
+  return 2 * (((k >> 1) & 1) | ((k >> 2) & 2));
 }
 
-// One operand tile of ROWS outputs x 64 k and its loads by NW waves (4 or 8):
-// ROWS / (8 NW) instructions per wave and K step.
+// One operand tile of ROWS outputs x 128 bytes of k and its loads by NW waves
+// (4, or 8 for 2-byte types): ROWS / (8 NW) instructions per wave and K step.
 template <typename T, int ROWS, bool KM, int NW>
 struct RingTile {
-  static constexpr int EL = ROWS * BK;      // elements of a stage
-  static constexpr int NI = ROWS / 8 / NW;  // load instructions per wave
+  static constexpr int ES = sizeof(T);
+  static constexpr int EL = ROWS * kStep<T>;         // elements of a stage
+  static constexpr int NI = ROWS / 8 / NW;           // load instructions per wave
+  static constexpr int RPI = 1024 / (ROWS * ES);     // K-major: k-rows per instruction
+  static constexpr int LPR = ROWS * ES / 16;         // K-major: lanes per k-row
   uint32_t lane_off;  // bytes from the tile's first element
   int kcol;           // NT: this lane's first k of the tile
-  int wave_el;        // LDS elements before this wave's first instruction
+  int wave_by;        // LDS bytes before this wave's first instruction
   // FOLD: an NT tile whose one instruction loads rows 0 .. 31 of two sources
   // (waves 0 - 3 and 4 - 7)
   template <bool FOLD = false>
@@ -64,50 +74,80 @@ struct RingTile {
     if constexpr (KM) {
       // instruction i of wave w: k-rows kw + ki(i) .., kw from the wave and
       // ki(i) chosen so that a lane's swizzle is the same for every i
-      const int kw = NW == 8 || ROWS == 32 ? (512 / ROWS) * w : 8 * (w & 1) + 16 * (w >> 1);
-      const int row = kw + lane / (ROWS / 8);
-      const int c = (lane % (ROWS / 8)) ^ kmaj_sw_n<ROWS>(row);
-      lane_off = static_cast<uint32_t>(row * ld * 2 + c * 16);
-      wave_el = kw * ROWS;
+      const int kw = ES == 4 ? 4 * w : NW == 8 ? RPI * w : 8 * (w & 1) + 16 * (w >> 1);
+      const int row = kw + lane / LPR;
+      const int c = (lane % LPR) ^ kmaj_sw_n<T, ROWS>(row);
+      lane_off = static_cast<uint32_t>(row * ld * ES + c * 16);
+      wave_by = kw * ROWS * ES;
       kcol = 0;
     } else {
       const int row = tid >> 3;
       const int c = (tid & 7) ^ nt_sw(row);
-      lane_off = static_cast<uint32_t>((FOLD ? row & 31 : row) * ld * 2 + c * 16);
-      kcol = 8 * c;
-      wave_el = w * 512;
+      lane_off = static_cast<uint32_t>((FOLD ? row & 31 : row) * ld * ES + c * 16);
+      kcol = c * (16 / ES);
+      wave_by = w * 1024;
     }
   }
   // first k-row (K-major) of instruction i, less the wave's
   static constexpr int ki(int i) {
+    if (ES == 4) return ROWS == 128 ? 2 * (i & 1) + 16 * (i >> 1) : 16 * i;
     return NW == 4 && ROWS == 128 ? 4 * (i & 1) + 32 * (i >> 1) : 32 * i;
   }
   // instruction i of the stage at `lds` (byte address) from the resource r;
   // voff is lane_off or, past K, an offset out of range
   __device__ __forceinline__ void issue(uint32_t lds, v4i r, uint32_t voff, int64_t ld, int i) const {
     if constexpr (KM)
-      dma16(r, voff, static_cast<uint32_t>(ki(i) * ld * 2), lds + 2 * (wave_el + ki(i) * ROWS));
+      dma16(r, voff, static_cast<uint32_t>(ki(i) * ld * ES), lds + wave_by + ki(i) * ROWS * ES);
     else
-      dma16(r, voff, static_cast<uint32_t>(8 * NW * i * ld * 2), lds + 2 * wave_el + i * (1024 * NW));
+      dma16(r, voff, static_cast<uint32_t>(8 * NW * i * ld * ES), lds + wave_by + i * (1024 * NW));
   }
 };
 
-// LDS element offset of this lane's first transposed read for the 16-column
-// block at colw (see kmaj_base).
-template <int COLS>
+// One lane's operand of a 16-wide block and substep (half a K step): 8
+// elements of consecutive k (2-byte types: one MFMA) or 4 (fp32: four MFMAs,
+// element j at k = 4 (l / 16) + j in both operands).
+template <typename T>
+struct RingOp {
+  typedef typename Mfma<T>::vec8 vec;
+  static __device__ __forceinline__ f32x4 mma(vec a, vec b, f32x4 c) { return Mfma<T>::mma16(a, b, c); }
+};
+template <>
+struct RingOp<float> {
+  typedef f32x4 vec;
+  static __device__ __forceinline__ f32x4 mma(vec a, vec b, f32x4 c) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+    return c;
+  }
+};
+
+// LDS element offset of this lane's first K-major read for the 16-column block
+// at colw (see kmaj_base); block r is at that ^ 16 r, substep 1 half a tile on.
+template <typename T, int COLS>
 __device__ __forceinline__ int kmaj_base_n(int colw) {
   const int lane = threadIdx.x & 63;
-  const int k = 8 * (lane >> 4) + ((lane & 15) >> 2);
-  const int col = colw + 4 * (lane & 3);
-  return k * COLS + (((col >> 3) ^ kmaj_sw_n<COLS>(k)) << 3) + (col & 7);
+  if constexpr (sizeof(T) == 4) {
+    const int k = 4 * (lane >> 4), col = colw + (lane & 15);
+    return k * COLS + (((col >> 2) ^ kmaj_sw_n<T, COLS>(k)) << 2) + (col & 3);
+  } else {
+    const int k = 8 * (lane >> 4) + ((lane & 15) >> 2);
+    const int col = colw + 4 * (lane & 3);
+    return k * COLS + (((col >> 3) ^ kmaj_sw_n<T, COLS>(k)) << 3) + (col & 7);
+  }
 }
 template <typename T, int COLS>
-__device__ __forceinline__ typename Mfma<T>::vec8 kmaj_operand_n(const T* tile, int off) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off));
-  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off + 4 * COLS));
-  return __builtin_bit_cast(typename Mfma<T>::vec8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+__device__ __forceinline__ typename RingOp<T>::vec kmaj_operand_n(const T* tile, int off) {
+  if constexpr (sizeof(T) == 4) {
+    const T* p = tile + off;
+    return f32x4{p[0], p[COLS], p[2 * COLS], p[3 * COLS]};
+  } else {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off));
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off + 4 * COLS));
+    return __builtin_bit_cast(typename RingOp<T>::vec,
+                              __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
 }
 
 // EPI as for gemm_tiled_kernel: 0 plain (+ residual), 1 SwiGLU (the B tile's
@@ -119,15 +159,16 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(WPE, W
 void gemm_ring_kernel(GemmArgs args) {
   static_assert(EPI == 0 || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
   constexpr int TBM = 32 * MB, TBN = 32 * NB, WR = 16 * MB, WC = 16 * NB;
-  typedef Mfma<T> Mm;
-  typedef typename Mm::vec8 V8;
-  constexpr int NT = 256 * KS;
+  typedef RingOp<T> Mm;
+  typedef typename Mm::vec V8;
+  constexpr int NT = 256 * KS, ES = sizeof(T), BK = kStep<T>;
+  static_assert(ES == 2 || (EPI == 0 && KS == 1), "fp32: plain epilogue");
   typedef RingTile<T, TBM, AKM, 4 * KS> TA;
   typedef RingTile<T, TBN, BKM, 4 * KS> TB;
   constexpr int RA = KS == 1 ? RB + 1 : RB;  // A stages
   constexpr int LDS_EL = RA * TA::EL + RB * TB::EL;
   constexpr int EP = TBN + 4;  // pitch of the epilogue's fp32 tile
-  static_assert(TBM * EP * 4 <= LDS_EL * 2, "the epilogue tile lies in the rings");
+  static_assert(TBM * EP * 4 <= LDS_EL * ES, "the epilogue tile lies in the rings");
   __shared__ __attribute__((aligned(16))) T lds[LDS_EL];
   T* const As = lds;
   T* const Bs = lds + RA * TA::EL;
@@ -150,14 +191,14 @@ void gemm_ring_kernel(GemmArgs args) {
 
   // first element of each operand's tile, bytes left from there to the
   // operand's end, and the bytes of one K step
-  const char* Ab = static_cast<const char*>(args.a) + 2 * (AKM ? m0 : m0 * lda);
-  int64_t a_left = 2 * (AKM ? (K - 1) * lda + M - m0 : (M - 1 - m0) * lda + K);
-  const int64_t a_step = AKM ? 2 * BK * lda : 2 * BK;
+  const char* Ab = static_cast<const char*>(args.a) + ES * (AKM ? m0 : m0 * lda);
+  const int64_t a_left = ES * (AKM ? (K - 1) * lda + M - m0 : (M - 1 - m0) * lda + K);
+  const int64_t a_step = AKM ? ES * BK * lda : ES * BK;
   const int64_t b_rows = EPI == 1 ? N / 2 : N, b_r0 = EPI == 1 ? f0 : n0;
-  const char* Bb = static_cast<const char*>(args.b) + 2 * (BKM ? b_r0 : b_r0 * ldb);
-  const char* B2b = EPI == 1 ? static_cast<const char*>(args.b2) + 2 * b_r0 * ldb : nullptr;
-  int64_t b_left = 2 * (BKM ? (K - 1) * ldb + b_rows - b_r0 : (b_rows - 1 - b_r0) * ldb + K);
-  const int64_t b_step = BKM ? 2 * BK * ldb : 2 * BK;
+  const char* Bb = static_cast<const char*>(args.b) + ES * (BKM ? b_r0 : b_r0 * ldb);
+  const char* B2b = EPI == 1 ? static_cast<const char*>(args.b2) + ES * b_r0 * ldb : nullptr;
+  const int64_t b_left = ES * (BKM ? (K - 1) * ldb + b_rows - b_r0 : (b_rows - 1 - b_r0) * ldb + K);
+  const int64_t b_step = BKM ? ES * BK * ldb : ES * BK;
 
   TA ta;
   TB tb;
@@ -174,15 +215,15 @@ void gemm_ring_kernel(GemmArgs args) {
 
   int abase[2], bbase[2];  // operand read bases of the two substeps (elements)
   if constexpr (AKM) {
-    abase[0] = kmaj_base_n<TBM>(wm * WR);
-    abase[1] = abase[0] + 32 * TBM;
+    abase[0] = kmaj_base_n<T, TBM>(wm * WR);
+    abase[1] = abase[0] + BK / 2 * TBM;
   } else {
-    abase[0] = nt_off(wm * WR + l16, 8 * q4);
-    abase[1] = abase[0] ^ 32;
+    abase[0] = nt_off(wm * WR + l16, 8 * q4) * 2 / ES;
+    abase[1] = abase[0] ^ (64 / ES);
   }
   if constexpr (BKM) {
-    bbase[0] = kmaj_base_n<TBN>(wn * WC);
-    bbase[1] = bbase[0] + 32 * TBN;
+    bbase[0] = kmaj_base_n<T, TBN>(wn * WC);
+    bbase[1] = bbase[0] + BK / 2 * TBN;
   } else if constexpr (EPI == 1) {
     // wave half wn: features WC / 2 wn .. of the gate rows, then of the up
     // rows (block j < NB / 2: gate, else up), so that a wave's blocks j and
@@ -190,8 +231,8 @@ void gemm_ring_kernel(GemmArgs args) {
     bbase[0] = nt_off(wn * (WC / 2) + l16, 8 * q4);
     bbase[1] = bbase[0] ^ 32;
   } else {
-    bbase[0] = nt_off(wn * WC + l16, 8 * q4);
-    bbase[1] = bbase[0] ^ 32;
+    bbase[0] = nt_off(wn * WC + l16, 8 * q4) * 2 / ES;
+    bbase[1] = bbase[0] ^ (64 / ES);
   }
   V8 xa[2][MB], xb[2][NB];
   // operand piece r (A row blocks, then B row blocks) of substep s, stages sa / sb
@@ -201,7 +242,7 @@ void gemm_ring_kernel(GemmArgs args) {
       if constexpr (AKM)
         xa[s][r] = kmaj_operand_n<T, TBM>(t, abase[s] ^ (16 * r));
       else
-        xa[s][r] = *reinterpret_cast<const V8*>(t + abase[s] + 1024 * r);
+        xa[s][r] = *reinterpret_cast<const V8*>(t + abase[s] + 16 * BK * r);
     } else {
       const int j = r - MB;
       const T* t = Bs + sb * TB::EL;
@@ -211,7 +252,7 @@ void gemm_ring_kernel(GemmArgs args) {
         xb[s][j] = *reinterpret_cast<const V8*>(
             t + bbase[s] + 1024 * (j % (NB / 2)) + (j / (NB / 2)) * (TBN / 2) * BK);
       else
-        xb[s][j] = *reinterpret_cast<const V8*>(t + bbase[s] + 1024 * j);
+        xb[s][j] = *reinterpret_cast<const V8*>(t + bbase[s] + 16 * BK * j);
     }
   };
   // loads of K step k (k0 = 64 k): resource of the step, lane offset
@@ -234,18 +275,18 @@ void gemm_ring_kernel(GemmArgs args) {
     return s;
   };
   auto load_a = [&](const Src& s, int st, int i) __attribute__((always_inline)) {
-    ta.issue(lds_a + st * (2 * TA::EL), s.r, s.voff, lda, i);
+    ta.issue(lds_a + st * (ES * TA::EL), s.r, s.voff, lda, i);
   };
   auto load_b = [&](const Src& s, int st, int i) __attribute__((always_inline)) {
     if constexpr (EPI == 1 && !kFold) {
       // pieces of the first half: gate rows 32 i .., of the second: up rows
       if (i < TB::NI / 2)
-        tb.issue(lds_b + st * (2 * TB::EL), s.r, s.voff, ldb, i);
+        tb.issue(lds_b + st * (ES * TB::EL), s.r, s.voff, ldb, i);
       else
         dma16(s.r2, s.voff, static_cast<uint32_t>(32 * KS * (i - TB::NI / 2) * ldb * 2),
-              lds_b + st * (2 * TB::EL) + 2 * tb.wave_el + i * (4096 * KS));
+              lds_b + st * (ES * TB::EL) + tb.wave_by + i * (4096 * KS));
     } else {
-      tb.issue(lds_b + st * (2 * TB::EL), s.r, s.voff, ldb, i);
+      tb.issue(lds_b + st * (ES * TB::EL), s.r, s.voff, ldb, i);
     }
   };
   // The MB NB MFMAs of set q, row by row; after row c its share of the loads
@@ -259,7 +300,7 @@ void gemm_ring_kernel(GemmArgs args) {
 #pragma unroll
     for (int c = 0; c < MB; ++c) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) acc[c][j] = Mm::mma16(xa[q][c], xb[q][j], acc[c][j]);
+      for (int j = 0; j < NB; ++j) acc[c][j] = Mm::mma(xa[q][c], xb[q][j], acc[c][j]);
       if (rd) {
 #pragma unroll
         for (int u = c * (MB + NB) / MB; u < (c + 1) * (MB + NB) / MB; ++u)
@@ -331,7 +372,7 @@ void gemm_ring_kernel(GemmArgs args) {
 #pragma unroll
       for (int c = 0; c < MB; ++c) {
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[c][j] = Mm::mma16(xa[q][c], xb[q][j], acc[c][j]);
+        for (int j = 0; j < NB; ++j) acc[c][j] = Mm::mma(xa[q][c], xb[q][j], acc[c][j]);
 #pragma unroll
         for (int u = c * (MB + NB) / MB; u < (c + 1) * (MB + NB) / MB; ++u)
           rd_piece(st1, st1, q ^ 1, u == 0 ? 0 : u <= NB ? MB + u - 1 : u - NB);
@@ -446,10 +487,9 @@ void gemm_ring_kernel(GemmArgs args) {
       const int id = it * NT + tid, row = id / CPR, ch = id % CPR;
       const int64_t gr = m0 + row, gc = n0 + 8 * ch;
       if (gr >= M || gc >= N) continue;
-      T8 o;
       float v[8];
       chunk(row, 8 * ch, v);
-      if (EPI == 2 && gc < args.rcols) {
+      if constexpr (EPI == 2) if (gc < args.rcols) {
         // this chunk rotated: its pair is the chunk rhalf columns away in the
         // same head (half-split) or inside the chunk (interleaved); the
         // product is rounded to T first, as the RoPE pass would read it
@@ -477,6 +517,7 @@ void gemm_ring_kernel(GemmArgs args) {
           const float4 c4 = *reinterpret_cast<const float4*>(cp + hc / 2);
           const float4 s4 = *reinterpret_cast<const float4*>(sp + hc / 2);
           const float cs[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
+          T8 o;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float x1 = round_to<T>(v[2 * e]), x2 = round_to<T>(v[2 * e + 1]);
@@ -492,13 +533,12 @@ void gemm_ring_kernel(GemmArgs args) {
         }
       }
       if (EPI == 0 && R != nullptr) {
-        const T8 rv = *reinterpret_cast<const T8*>(R + gr * args.ldr + gc);
+        float rv[8];
+        Vec8<T>::load(R + gr * args.ldr + gc, rv);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += to_f32(rv[e]);
+        for (int e = 0; e < 8; ++e) v[e] += rv[e];
       }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = static_cast<T>(v[e]);
-      *reinterpret_cast<T8*>(C + gr * args.ldc + gc) = o;
+      Vec8<T>::store(C + gr * args.ldc + gc, v);
     }
   }
 }
