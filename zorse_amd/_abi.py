@@ -174,8 +174,15 @@ def dtype_code(dtype: torch.dtype) -> int:
     raise TypeError(f"unsupported dtype {dtype} (float32, float16, bfloat16)")
 
 
+# The raw handle of the current stream without a torch.cuda.Stream object: 0.06
+# us a call where building the object takes 2 us, half of a launch.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device: torch.device | None = None) -> int:
     """hipStream_t of torch's current stream on ``device``."""
+    if _raw_stream is not None and device is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

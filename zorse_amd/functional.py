@@ -27,7 +27,7 @@ def rope_tables(seq: int, head_dim: int, theta: float, dtype: torch.dtype,
                 device: torch.device, interleaved: bool = False):
     """fp32 cos / sin tables [seq, head_dim/2] holding exactly the values the
     reference multiplies by (rounded to ``dtype`` for the half-split form)."""
-    key = (seq, head_dim, float(theta), dtype, str(device), interleaved)
+    key = (seq, head_dim, float(theta), dtype, device, interleaved)
     with _rope_lock:
         hit = _rope_cache.get(key)
     if hit is not None:

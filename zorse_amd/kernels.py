@@ -205,9 +205,13 @@ def _gemm_operand(name: str, t: torch.Tensor):
     if t.dim() != 2:
         raise ValueError(f"gemm: {name} must be 2-D, got shape {tuple(t.shape)}")
     rows, cols = t.shape
-    if t.stride(1) != 1 and cols > 1:
+    ld, unit = t.stride()
+    if unit == 1 and rows > 1 and ld >= cols > 0:
+        return rows, cols, ld
+    if unit != 1 and cols > 1:
         raise ValueError(f"gemm: {name} needs unit column stride")
-    ld = t.stride(0) if rows > 1 else max(cols, 1)
+    if rows <= 1:
+        ld = max(cols, 1)
     if ld < cols:
         raise ValueError(f"gemm: {name} has overlapping rows (row stride {ld} < {cols})")
     return rows, cols, max(ld, 1)
@@ -466,23 +470,13 @@ def _attn_desc(q, k, v, o, scale, causal, window, dq=None, dk=None, dv=None):
             raise ValueError(f"{name} dtype {t.dtype} != q dtype {q.dtype}")
     if (causal or window) and Sq != Skv:
         raise ValueError("causal / windowed attention needs Sq == Skv")
-    desc = _abi.AttnDesc()
-    desc.B, desc.Sq, desc.Skv, desc.Hq, desc.Hkv, desc.d = B, Sq, Skv, Hq, Hkv, d
-    desc.q_sb, desc.q_ss, desc.q_sh = q.stride(0), q.stride(1), q.stride(2)
-    desc.k_sb, desc.k_ss, desc.k_sh = k.stride(0), k.stride(1), k.stride(2)
-    desc.v_sb, desc.v_ss, desc.v_sh = v.stride(0), v.stride(1), v.stride(2)
-    if o is not None:
-        desc.o_sb, desc.o_ss, desc.o_sh = o.stride(0), o.stride(1), o.stride(2)
-    for pre, t in (("dq", dq), ("dk", dk), ("dv", dv)):
-        if t is not None:
-            setattr(desc, pre + "_sb", t.stride(0))
-            setattr(desc, pre + "_ss", t.stride(1))
-            setattr(desc, pre + "_sh", t.stride(2))
-    desc.scale = float(scale)
-    desc.causal = int(bool(causal))
-    desc.window = int(window or 0)
-    desc.dtype = dtype_code(q.dtype)
-    return desc
+    def st(t):
+        return t.stride()[:3] if t is not None else (0, 0, 0)
+
+    # one constructor call, fields in the order of zk_attn_desc
+    return _abi.AttnDesc(B, Sq, Skv, Hq, Hkv, d, *st(q), *st(k), *st(v), *st(o), *st(dq),
+                         *st(dk), *st(dv), float(scale), int(bool(causal)), int(window or 0),
+                         dtype_code(q.dtype))
 
 
 def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool = True,

@@ -15,9 +15,11 @@ are single GEMMs into adjacent slices: no concatenation, no gradient copies.
 """
 from __future__ import annotations
 
+import contextlib
 import math
 import os
 from dataclasses import dataclass
+from functools import cached_property
 
 import torch
 
@@ -72,27 +74,34 @@ class LayerSpec:
             off += n
         return out
 
-    @property
+    @cached_property
     def numel(self) -> int:
         return sum(math.prod(s) for s in self.shapes().values())
+
+    @cached_property
+    def view_specs(self) -> tuple:
+        """(name, shape, strides, offset) of the views FlatViews takes."""
+        o, h, F = self.offsets(), self.hidden, self.ffn
+        mats = (("qkv", (self.qkv_dim, h), o["q"][0]), ("o", (h, self.q_dim), o["o"][0]),
+                ("gu", (2 * F, h), o["gate"][0]), ("down", (h, F), o["down"][0]))
+        return (*((n, s, (s[1], 1), a) for n, s, a in mats),
+                ("ln1", (h,), (1,), o["ln1"][0]), ("ln2", (h,), (1,), o["ln2"][0]))
 
 
 class FlatViews:
     """Named views of a flat buffer laid out as LayerSpec.offsets()."""
 
+    __slots__ = ("qkv", "o", "gu", "down", "ln1", "ln2")
+
     def __init__(self, spec: LayerSpec, flat: torch.Tensor):
-        o = spec.offsets()
-        h, F = spec.hidden, spec.ffn
-
-        def v(a, b, shp):
-            return flat[a:b].view(shp)
-
-        self.qkv = v(o["q"][0], o["v"][1], (spec.qkv_dim, h))
-        self.o = v(*o["o"], (h, spec.q_dim))
-        self.gu = v(o["gate"][0], o["up"][1], (2 * F, h))
-        self.down = v(*o["down"], (h, F))
-        self.ln1 = flat[o["ln1"][0]:o["ln1"][1]]
-        self.ln2 = flat[o["ln2"][0]:o["ln2"][1]]
+        if flat.dim() == 1 and flat.numel() >= spec.numel and flat.stride(0) == 1:
+            # six host calls of 0.8 us where slice + view take 2.7 us each
+            base = flat.storage_offset()
+            for name, shape, strides, off in spec.view_specs:
+                setattr(self, name, flat.as_strided(shape, strides, base + off))
+        else:  # strided, or too short for its layer: view and the kernels' checks say so
+            for name, shape, _, off in spec.view_specs:
+                setattr(self, name, flat[off:off + math.prod(shape)].view(shape))
 
 
 # Every projection product runs on the hand-written GEMMs (zk_gemm) with the
@@ -175,6 +184,15 @@ def _transposed_outputs(t):
 _wgrad_side = os.environ.get("ZORSE_WGRAD_STREAM", "1") != "0"
 _side_streams: dict = {}
 
+# A layer backward with less work than this keeps them in order too: its
+# kernels are shorter than the host takes to enqueue them, and the three
+# cross-stream waits cost the host 15 us each.  Forward + backward, side
+# stream / in order: tiny shape at 256 tokens (0.5e11) 620 / 470 us, at 512
+# (1.0e11) 460 / 397, at 1024 (2.1e11) 647 / 623, at 2048 (4.2e11) 935 / 994;
+# 1B grouped-query at 512 (1.2e11) 620 / 485, at 1024 (2.5e11) 744 / 772; 7B at
+# 128 (1.0e11) 653 / 650, at 512 (4.1e11) 1004 / 1047.
+SIDE_STREAM_FLOPS = 2.2e11
+
 
 def set_wgrad_stream(enable: bool) -> bool:
     """Run the weight-gradient GEMMs on a side stream (True) or in order on the
@@ -189,10 +207,10 @@ class _WeightGrads:
     side stream (after the compute stream's work so far) or, when disabled,
     on the compute stream; join() makes the compute stream wait for them."""
 
-    def __init__(self, device, grad_flat):
-        self.main = torch.cuda.current_stream(device)
+    def __init__(self, device, grad_flat, flops):
         self.side = None
-        if _wgrad_side:
+        if _wgrad_side and flops >= SIDE_STREAM_FLOPS:
+            self.main = torch.cuda.current_stream(device)
             self.side = _side_streams.get(device)
             if self.side is None:
                 self.side = _side_streams[device] = torch.cuda.Stream(device=device)
@@ -276,6 +294,19 @@ def _rope_for(S, spec, dtype, device, positions):
                        spec.interleaved_rope)
 
 
+def _heads(qkv, spec, B, S):
+    """The q, k, v [B, S, heads, d] views of a [B S, qkv_dim] q|k|v buffer."""
+    if qkv.shape != (B * S, spec.qkv_dim):
+        raise ValueError(f"q|k|v buffer {tuple(qkv.shape)} != {(B * S, spec.qkv_dim)}")
+    ld, u = qkv.stride()
+    d, off = spec.head_dim, qkv.storage_offset()
+    st = (S * ld, ld, d * u, u)
+    kv = (B, S, spec.kv_heads, d)
+    return (qkv.as_strided((B, S, spec.heads, d), st, off),
+            qkv.as_strided(kv, st, off + u * spec.q_dim),
+            qkv.as_strided(kv, st, off + u * (spec.q_dim + spec.kv_dim)))
+
+
 def layer_forward(x: torch.Tensor, w: FlatViews, spec: LayerSpec, attn_cache=None,
                   positions: torch.Tensor | None = None):
     """Forward on compute-dtype tensors; returns (out, saved tuple).
@@ -297,9 +328,7 @@ def layer_forward(x: torch.Tensor, w: FlatViews, spec: LayerSpec, attn_cache=Non
     cos, sin = _rope_for(S, spec, x.dtype, x.device, positions)
     qkv = K.gemm_rope(n1, w.qkv, seq_len=S, rot_cols=spec.q_dim + spec.kv_dim, head_dim=d,
                       cos=cos, sin=sin, positions=positions, interleaved=spec.interleaved_rope)
-    q = qkv[:, :spec.q_dim].view(B, S, Hq, d)
-    k = qkv[:, spec.q_dim:spec.q_dim + spec.kv_dim].view(B, S, Hkv, d)
-    v = qkv[:, spec.q_dim + spec.kv_dim:].view(B, S, Hkv, d)
+    q, k, v = _heads(qkv, spec, B, S)
     hit = attn_cache.take() if attn_cache is not None else None
     if hit is not None:
         o, lse = hit
@@ -349,7 +378,8 @@ def layer_backward(dout: torch.Tensor, saved, w: FlatViews, spec: LayerSpec,
     d, Hq, Hkv, F = spec.head_dim, spec.heads, spec.kv_heads, spec.ffn
     g = FlatViews(spec, grad_flat)
     dout2 = dout.reshape(T, h)
-    wgrad = _WeightGrads(dout.device, grad_flat)
+    # the backward's products: two of the forward's size per weight
+    wgrad = _WeightGrads(dout.device, grad_flat, 4.0 * T * spec.numel)
 
     # MLP: out = hdn + z W_down^T
     wgrad(dout2, z, g.down)
@@ -372,13 +402,9 @@ def layer_backward(dout: torch.Tensor, saved, w: FlatViews, spec: LayerSpec,
     # attention: hdn = x + o W_o^T
     wgrad(dh, o2, g.o)
     do2 = _dgrad(dh, w.o)                            # [T, Hq d]
-    q = qkv[:, :spec.q_dim].view(B, S, Hq, d)
-    k = qkv[:, spec.q_dim:spec.q_dim + spec.kv_dim].view(B, S, Hkv, d)
-    v = qkv[:, spec.q_dim + spec.kv_dim:].view(B, S, Hkv, d)
+    q, k, v = _heads(qkv, spec, B, S)
     dqkv = torch.empty_like(qkv)
-    dq = dqkv[:, :spec.q_dim].view(B, S, Hq, d)
-    dk = dqkv[:, spec.q_dim:spec.q_dim + spec.kv_dim].view(B, S, Hkv, d)
-    dv = dqkv[:, spec.q_dim + spec.kv_dim:].view(B, S, Hkv, d)
+    dq, dk, dv = _heads(dqkv, spec, B, S)
     for fn in list(BEFORE_ATTENTION_BACKWARD):
         fn()
     cos, sin = _rope_for(S, spec, dout.dtype, dout.device, positions)
@@ -471,6 +497,13 @@ class AttentionCache:
         self._entries[self._key] = (self._storage, o, lse)
 
 
+def _no_autocast():
+    """Autocast off for a block: nothing to do where it is off already."""
+    if torch.is_autocast_enabled("cuda"):
+        return torch.autocast("cuda", enabled=False)
+    return contextlib.nullcontext()
+
+
 class DecoderLayerFunction(torch.autograd.Function):
     """autograd node of one decoder layer: inputs (x, flat_param)."""
 
@@ -480,7 +513,7 @@ class DecoderLayerFunction(torch.autograd.Function):
         w = FlatViews(spec, w_flat)
         if attn_cache is not None:
             attn_cache.bind(x, flat_param, w_flat)
-        with torch.autocast("cuda", enabled=False):
+        with _no_autocast():
             out, saved = layer_forward(x.contiguous(), w, spec, attn_cache, positions)
         ctx.spec = spec
         ctx.param_dtype = flat_param.dtype
@@ -496,7 +529,7 @@ class DecoderLayerFunction(torch.autograd.Function):
         w = FlatViews(spec, w_flat)
         dout = dout.to(w_flat.dtype).contiguous()
         grad_flat = torch.empty(spec.numel, device=dout.device, dtype=w_flat.dtype)
-        with torch.autocast("cuda", enabled=False):
+        with _no_autocast():
             dx = layer_backward(dout, saved, w, spec, grad_flat)
         if ctx.param_dtype != grad_flat.dtype:
             grad_flat = grad_flat.to(ctx.param_dtype)
