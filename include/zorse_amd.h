@@ -274,6 +274,17 @@ int zk_attn_fwd_t(const zk_attn_desc* desc, const void* q, const void* k,
                   const void* v, void* o, float* lse, void* o_t, int64_t ld_t,
                   zk_stream_t stream);
 
+/* zk_attn_fwd / zk_attn_bwd (same reference lines, same masks) for the other
+ * head dims of 2-byte types: even, 34 .. 62 and 66 .. 126, rows as they are
+ * stored (no padding).  Strides multiples of 2 elements, pointers 4-byte
+ * aligned, row strides below 2^23 elements. */
+int zk_attn_fwd_ragged(const zk_attn_desc* desc, const void* q, const void* k,
+                       const void* v, void* o, float* lse, zk_stream_t stream);
+int zk_attn_bwd_ragged(const zk_attn_desc* desc, const void* q, const void* k,
+                       const void* v, const void* o, const void* dout,
+                       const float* lse, void* dq, void* dk, void* dv,
+                       void* workspace, int64_t workspace_bytes, zk_stream_t stream);
+
 /* Bytes of workspace zk_attn_bwd needs: the fp32 row deltas rowsum(dO o O)
  * and the log2-domain LSE, [B, Hq, Sq] each. */
 int64_t zk_attn_bwd_workspace(const zk_attn_desc* desc);

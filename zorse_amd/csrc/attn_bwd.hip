@@ -34,7 +34,7 @@
 
 namespace zk {
 
-int check_attn_desc(const zk_attn_desc* d, const char* who, bool bwd);
+int check_attn_desc(const zk_attn_desc* d, const char* who, bool bwd, bool ragged);
 void fill_args(AttnArgs& a, const zk_attn_desc* d);
 
 // ------------------------------------------------------------- dK / dV -----
@@ -48,12 +48,15 @@ struct DkdvCfg {
 };
 
 // kFull: Sq is a multiple of the query block, so no block runs past the end.
-template <typename T, int D, bool kFull>
+// KR: as in the forward, 0 for a head dim of D, else ceil(a.d / 16).
+template <typename T, int D, bool kFull, int KR = 0>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
   typedef DkdvCfg<D> C;
   typedef Mfma<T> M;
   typedef typename M::vec8 V8;
   constexpr int BK = C::BK, MQ = C::MQ;
+  constexpr int KS = KR ? KR : D / 16, NB = (KS + 1) / 2;
+  const int hd = KR ? static_cast<int>(a.d) : D;
   // Q / dO tiles double-buffered (swizzled rows); each wave keeps its own copy
   // of the block's lse2 / delta vectors so every wave issues the same loads.
   // Q / dO tiles of the two stages, each its own array: the compiler then sees
@@ -99,12 +102,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
   // B operands of S = Q K^T and dP = dO V^T: lane holds row my_key.  K stays
   // in registers; V goes to this wave's LDS rows (read back per step), which
   // keeps the kernel within 256 registers (two waves per SIMD).
-  V8 kreg[D / 16];
+  V8 kreg[KS];
   T* Vme = Vw[wave];
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
+  for (int ks = 0; ks < KS; ++ks) {
     V8 vv;
-    if (my_key < a.Skv) {
+    if (my_key < a.Skv && KR) {
+      kreg[ks] = load_cols8<T>(Kp + my_key * a.k_ss, 16 * ks + 8 * g, hd);
+      vv = load_cols8<T>(Vp + my_key * a.v_ss, 16 * ks + 8 * g, hd);
+    } else if (my_key < a.Skv) {
       kreg[ks] = *reinterpret_cast<const V8*>(Kp + my_key * a.k_ss + 16 * ks + 8 * g);
       vv = *reinterpret_cast<const V8*>(Vp + my_key * a.v_ss + 16 * ks + 8 * g);
     } else {
@@ -114,9 +120,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
     *reinterpret_cast<V8*>(&Vme[tile_off<D>(l32, 16 * ks + 8 * g)]) = vv;
   }
 
-  f32x16 dk[D / 32], dv[D / 32];
+  f32x16 dk[NB], dv[NB];
 #pragma unroll
-  for (int nt = 0; nt < D / 32; ++nt) {
+  for (int nt = 0; nt < NB; ++nt) {
     dk[nt] = f32x16{};
     dv[nt] = f32x16{};
   }
@@ -141,9 +147,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
   const int64_t nqb = qb_hi - qb_lo;
   const int64_t n_iter = nqb * n_rep;
 
-  TileLoader<T, D, MQ> qload, dload;
-  qload.init(a.q_ss);
-  dload.init(a.o_ss);
+  std::conditional_t<KR != 0, RaggedLoader<T, D, MQ>, TileLoader<T, D, MQ>> qload, dload;
+  if constexpr (KR != 0) {
+    qload.init(a.q_ss, hd);
+    dload.init(a.o_ss, hd);
+  } else {
+    qload.init(a.q_ss);
+    dload.init(a.o_ss);
+  }
   // iteration it covers query block qb_lo + it % nqb of q-head hk * n_rep +
   // it / nqb; (qbi, hr) below track that pair without dividing
   auto issue = [&](int64_t qbi, int64_t hr, int st) {
@@ -211,13 +222,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
       // step it follows (the fences keep the compiler from sinking it)
       V8 qa = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(Qt) + rb);
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
+      for (int ks = 0; ks < KS; ++ks) {
         const int ro = rb ^ (ks << 5);
-        const V8 da = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(dOt) + ro);
+        V8 da = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(dOt) + ro);
         const V8 vb = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(Vme) + ro);
         V8 qn = qa;
-        if (ks + 1 < D / 16)
+        if (ks + 1 < KS)
           qn = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(Qt) + (rb ^ ((ks + 1) << 5)));
+        if (KR && ks == KS - 1) {
+          qa = mask_cols<T>(qa, 16 * ks + 8 * g, hd);
+          da = mask_cols<T>(da, 16 * ks + 8 * g, hd);
+        }
         __builtin_amdgcn_sched_barrier(0);
         sv = M::mma(qa, kreg[ks], sv);
         dpv = M::mma(da, vb, dpv);
@@ -255,7 +270,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
       for (int h = 0; h < 2; ++h) {
         const int kk = 2 * mb + h;
 #pragma unroll
-        for (int nt = 0; nt < D / 32; ++nt) {
+        for (int nt = 0; nt < NB; ++nt) {
           const V8 dA = tr_at(dOt, tb ^ (nt << 6), kk);
           dv[nt] = M::mma(dA, pb[h], dv[nt]);
           const V8 qA = tr_at(Qt, tb ^ (nt << 6), kk);
@@ -303,12 +318,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
   // dK = scale (Q^T dS)^T, dV = (dO^T P)^T: lane holds key my_key and
   // d rows 32 nt + 8 a4 + 4 g + 0..3 (4 consecutive elements).
   if (my_key < a.Skv) {
-    if (a.rope_cos != nullptr) rope_inverse_regs<D>(dk, a, my_key, g);
+    if constexpr (KR == 0) {
+      if (a.rope_cos != nullptr) rope_inverse_regs<D>(dk, a, my_key, g);
+    }
     typedef T T4 __attribute__((ext_vector_type(4)));
     T* dkp = static_cast<T*>(a.dk) + b * a.dk_sb + hk * a.dk_sh + my_key * a.dk_ss;
     T* dvp = static_cast<T*>(a.dv) + b * a.dv_sb + hk * a.dv_sh + my_key * a.dv_ss;
 #pragma unroll
-    for (int nt = 0; nt < D / 32; ++nt)
+    for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
       for (int a4 = 0; a4 < 4; ++a4) {
         const int d0 = 32 * nt + 8 * a4 + 4 * g;
@@ -318,8 +335,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
           wk[e] = static_cast<T>(dk[nt][4 * a4 + e] * a.scale);
           wv[e] = static_cast<T>(dv[nt][4 * a4 + e]);
         }
-        *reinterpret_cast<T4*>(dkp + d0) = wk;
-        *reinterpret_cast<T4*>(dvp + d0) = wv;
+        if constexpr (KR != 0) {
+          store_cols4(dkp, d0, hd, wk);
+          store_cols4(dvp, d0, hd, wv);
+        } else {
+          *reinterpret_cast<T4*>(dkp + d0) = wk;
+          *reinterpret_cast<T4*>(dvp + d0) = wv;
+        }
       }
   }
   if (a.dk_t != nullptr) {
@@ -328,12 +350,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
     __syncthreads();
     const int64_t left = a.Skv - k0;
     const int nc = static_cast<int>(left < BK ? left : BK);
-    const int64_t off = hk * D * a.t_ld + b * a.Skv + k0;
+    const int64_t off = hk * hd * a.t_ld + b * a.Skv + k0;
     T* tile = &Vw[0][0];  // all D rows in one array (the other pointers are unused)
-    store_rows_transposed<T, D, BK, D>(dk, a.scale, tile, tile, tile, tile,
-                                       static_cast<T*>(a.dk_t) + off, a.t_ld, nc);
-    store_rows_transposed<T, D, BK, D>(dv, 1.f, tile, tile, tile, tile,
-                                       static_cast<T*>(a.dv_t) + off, a.t_ld, nc);
+    store_rows_transposed<T, D, BK, D, KR>(dk, a.scale, tile, tile, tile, tile,
+                                       static_cast<T*>(a.dk_t) + off, a.t_ld, nc, hd);
+    store_rows_transposed<T, D, BK, D, KR>(dv, 1.f, tile, tile, tile, tile,
+                                       static_cast<T*>(a.dv_t) + off, a.t_ld, nc, hd);
   }
 }
 
@@ -350,12 +372,14 @@ struct DqCfg {
 };
 
 // kFull: Skv is a multiple of the key tile, so no tile runs past the end.
-template <typename T, int D, bool kFull>
+template <typename T, int D, bool kFull, int KR = 0>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) {
   typedef DqCfg<D> C;
   typedef Mfma<T> M;
   typedef typename M::vec8 V8;
   constexpr int BM = C::BM, BN = C::BN, NT = C::NT;
+  constexpr int KS = KR ? KR : D / 16, NB = (KS + 1) / 2;
+  const int hd = KR ? static_cast<int>(a.d) : D;
   // swizzled rows; each stage its own array, so the compiler sees that the
   // next tile's asynchronous loads do not alias this tile's reads
   __shared__ __attribute__((aligned(16))) T K0[BN * D], K1[BN * D], V0[BN * D], V1[BN * D];
@@ -393,10 +417,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
   const T* Vp = static_cast<const T*>(a.v) + b * a.v_sb + hk * a.v_sh;
 
   // B operands of S^T = K Q^T and dP^T = V dO^T: lane holds query my_q.
-  V8 qreg[D / 16], dreg[D / 16];
+  V8 qreg[KS], dreg[KS];
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    if (my_q < a.Sq) {
+  for (int ks = 0; ks < KS; ++ks) {
+    if (my_q < a.Sq && KR) {
+      qreg[ks] = load_cols8<T>(Qp + my_q * a.q_ss, 16 * ks + 8 * g, hd);
+      dreg[ks] = load_cols8<T>(Dp + my_q * a.o_ss, 16 * ks + 8 * g, hd);
+    } else if (my_q < a.Sq) {
       qreg[ks] = *reinterpret_cast<const V8*>(Qp + my_q * a.q_ss + 16 * ks + 8 * g);
       dreg[ks] = *reinterpret_cast<const V8*>(Dp + my_q * a.o_ss + 16 * ks + 8 * g);
     } else {
@@ -413,8 +440,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
     float part = 0.f;
     if (my_q < a.Sq) {
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
-        const V8 ov = *reinterpret_cast<const V8*>(Op + my_q * a.o_ss + 16 * ks + 8 * g);
+      for (int ks = 0; ks < KS; ++ks) {
+        V8 ov;
+        if constexpr (KR != 0)
+          ov = load_cols8<T>(Op + my_q * a.o_ss, 16 * ks + 8 * g, hd);
+        else
+          ov = *reinterpret_cast<const V8*>(Op + my_q * a.o_ss + 16 * ks + 8 * g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) part = fmaf(to_f32(ov[e]), to_f32(dreg[ks][e]), part);
       }
@@ -437,9 +468,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
   const int64_t t_lo = kv_lo / BN;
   const int64_t t_hi = kv_hi > kv_lo ? (kv_hi + BN - 1) / BN : t_lo;
 
-  TileLoader<T, D, BN, NT> kload, vload;
-  kload.init(a.k_ss);
-  vload.init(a.v_ss);
+  std::conditional_t<KR != 0, RaggedLoader<T, D, BN, NT>, TileLoader<T, D, BN, NT>> kload, vload;
+  if constexpr (KR != 0) {
+    kload.init(a.k_ss, hd);
+    vload.init(a.v_ss, hd);
+  } else {
+    kload.init(a.k_ss);
+    vload.init(a.v_ss);
+  }
   auto issue = [&](int64_t kb0, int st) {
     kload.issue(st ? K1 : K0, Kp, a.k_ss, kb0, a.Skv, kFull);
     vload.issue(st ? V1 : V0, Vp, a.v_ss, kb0, a.Skv, kFull);
@@ -451,9 +487,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
   const int rbase = 2 * tile_off<D>(l32, 8 * g);
   const int tbase = 2 * tile_off<D>(4 * g + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
 
-  f32x16 dq[D / 32];
+  f32x16 dq[NB];
 #pragma unroll
-  for (int nt = 0; nt < D / 32; ++nt) dq[nt] = f32x16{};
+  for (int nt = 0; nt < NB; ++nt) dq[nt] = f32x16{};
 
   // One pipeline step on LDS stage ST (compile-time: immediate LDS offsets).
   auto step = [&](auto stage_tag, int64_t t) {
@@ -498,10 +534,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
         vq[i] = rowread(Vt, i);
       }
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
+      for (int ks = 0; ks < KS; ++ks) {
         __builtin_amdgcn_sched_barrier(0);
-        const V8 kA = kq[ks % PF], vA = vq[ks % PF];
-        if (ks + PF < D / 16) {
+        V8 kA = kq[ks % PF], vA = vq[ks % PF];
+        if (KR && ks == KS - 1) {
+          kA = mask_cols<T>(kA, 16 * ks + 8 * g, hd);
+          vA = mask_cols<T>(vA, 16 * ks + 8 * g, hd);
+        }
+        if (ks + PF < KS) {
           kq[ks % PF] = rowread(Kt, ks + PF);
           vq[ks % PF] = rowread(Vt, ks + PF);
         }
@@ -526,7 +566,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
         typedef short s16x4 __attribute__((ext_vector_type(4)));
         typedef short s16x8 __attribute__((ext_vector_type(8)));
         typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-        const int kk = 2 * tt + m / (D / 32), nt = m % (D / 32);
+        const int kk = 2 * tt + m / NB, nt = m % NB;
         const char* kb = reinterpret_cast<const char*>(Kt) + kk * 16 * D * 2;
         const int off = tb ^ (nt << 6);
         const s16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(kb + off));
@@ -535,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
         const s16x8 w = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
         return __builtin_bit_cast(V8, w);
       };
-      constexpr int NM = 2 * (D / 32);
+      constexpr int NM = 2 * NB;
       V8 tq[PF];
 #pragma unroll
       for (int i = 0; i < PF; ++i) tq[i] = trread(i);
@@ -544,7 +584,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
         __builtin_amdgcn_sched_barrier(0);
         const V8 w = tq[m % PF];
         if (m + PF < NM) tq[m % PF] = trread(m + PF);
-        dq[m % (D / 32)] = M::mma(w, sb[m / (D / 32)], dq[m % (D / 32)]);
+        dq[m % NB] = M::mma(w, sb[m / NB], dq[m % NB]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -557,18 +597,23 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
   }
 
   if (my_q < a.Sq) {
-    if (a.rope_cos != nullptr) rope_inverse_regs<D>(dq, a, my_q, g);
+    if constexpr (KR == 0) {
+      if (a.rope_cos != nullptr) rope_inverse_regs<D>(dq, a, my_q, g);
+    }
     typedef T T4 __attribute__((ext_vector_type(4)));
     T* dqp = static_cast<T*>(a.dq) + b * a.dq_sb + hq * a.dq_sh + my_q * a.dq_ss;
 #pragma unroll
-    for (int nt = 0; nt < D / 32; ++nt)
+    for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
       for (int a4 = 0; a4 < 4; ++a4) {
         const int d0 = 32 * nt + 8 * a4 + 4 * g;
         T4 w;
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = static_cast<T>(dq[nt][4 * a4 + e] * a.scale);
-        *reinterpret_cast<T4*>(dqp + d0) = w;
+        if constexpr (KR != 0)
+          store_cols4(dqp, d0, hd, w);
+        else
+          *reinterpret_cast<T4*>(dqp + d0) = w;
       }
   }
   if (a.dq_t != nullptr) {
@@ -576,9 +621,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
     // hold the tile once every wave is past its last step
     __syncthreads();
     const int64_t left = a.Sq - q0;
-    store_rows_transposed<T, D, BM, BN * D / BM>(
-        dq, a.scale, K0, K1, V0, V1, static_cast<T*>(a.dq_t) + hq * D * a.t_ld + b * a.Sq + q0,
-        a.t_ld, static_cast<int>(left < BM ? left : BM));
+    store_rows_transposed<T, D, BM, BN * D / BM, KR>(
+        dq, a.scale, K0, K1, V0, V1, static_cast<T*>(a.dq_t) + hq * hd * a.t_ld + b * a.Sq + q0,
+        a.t_ld, static_cast<int>(left < BM ? left : BM), hd);
   }
 }
 
@@ -612,7 +657,7 @@ static int attn_bwd_impl(const char* who, const zk_attn_desc* desc, const void* 
                          const void* k, const void* v, const void* o, const void* dout,
                          const float* lse, void* dq, void* dk, void* dv, void* workspace,
                          int64_t workspace_bytes, const RopeInv* rope,
-                         const TransposedOut* tout, zk_stream_t stream);
+                         const TransposedOut* tout, bool ragged, zk_stream_t stream);
 }  // namespace zk
 
 extern "C" int zk_attn_bwd(const zk_attn_desc* desc, const void* q,
@@ -621,7 +666,18 @@ extern "C" int zk_attn_bwd(const zk_attn_desc* desc, const void* q,
                            void* dk, void* dv, void* workspace,
                            int64_t workspace_bytes, zk_stream_t stream) {
   return attn_bwd_impl("zk_attn_bwd", desc, q, k, v, o, dout, lse, dq, dk, dv, workspace,
-                       workspace_bytes, nullptr, nullptr, stream);
+                       workspace_bytes, nullptr, nullptr, false, stream);
+}
+
+extern "C" int zk_attn_bwd_ragged(const zk_attn_desc* desc, const void* q, const void* k,
+                                  const void* v, const void* o, const void* dout,
+                                  const float* lse, void* dq, void* dk, void* dv,
+                                  void* workspace, int64_t workspace_bytes, zk_stream_t stream) {
+  const char* who = "zk_attn_bwd_ragged";
+  ZK_REQUIRE(desc == nullptr || desc->dtype != ZK_F32, ZK_EUNSUPPORTED,
+             "%s: 2-byte dtypes only", who);
+  return attn_bwd_impl(who, desc, q, k, v, o, dout, lse, dq, dk, dv, workspace,
+                       workspace_bytes, nullptr, nullptr, true, stream);
 }
 
 namespace zk {
@@ -656,7 +712,7 @@ extern "C" int zk_attn_bwd_rope_t(const zk_attn_desc* desc, const void* q, const
   }
   const TransposedOut t = {dq_t, dk_t, dv_t, ld_t};
   return attn_bwd_impl(who, desc, q, k, v, o, dout, lse, dq, dk, dv, workspace,
-                       workspace_bytes, cos != nullptr ? &r : nullptr, &t, stream);
+                       workspace_bytes, cos != nullptr ? &r : nullptr, &t, false, stream);
 }
 
 extern "C" int zk_attn_bwd_rope(const zk_attn_desc* desc, const void* q, const void* k,
@@ -670,7 +726,7 @@ extern "C" int zk_attn_bwd_rope(const zk_attn_desc* desc, const void* q, const v
   if (rc != ZK_OK) return rc;
   const RopeInv r = {cos, sin, n_pos, positions, pairing};
   return attn_bwd_impl(who, desc, q, k, v, o, dout, lse, dq, dk, dv, workspace,
-                       workspace_bytes, &r, nullptr, stream);
+                       workspace_bytes, &r, nullptr, false, stream);
 }
 
 namespace zk {
@@ -678,8 +734,8 @@ static int attn_bwd_impl(const char* who, const zk_attn_desc* desc, const void* 
                          const void* k, const void* v, const void* o, const void* dout,
                          const float* lse, void* dq, void* dk, void* dv, void* workspace,
                          int64_t workspace_bytes, const RopeInv* rope,
-                         const TransposedOut* tout, zk_stream_t stream) {
-  int rc = check_attn_desc(desc, who, true);
+                         const TransposedOut* tout, bool ragged, zk_stream_t stream) {
+  int rc = check_attn_desc(desc, who, true, ragged);
   if (rc != ZK_OK) return rc;
   if (tout != nullptr) {
     ZK_REQUIRE(tout->dq_t && tout->dk_t && tout->dv_t, ZK_EINVAL,
@@ -728,9 +784,10 @@ static int attn_bwd_impl(const char* who, const zk_attn_desc* desc, const void* 
     launch_attn_bwd_f32(a, s);
     return launch_status(who);
   }
-  ZK_REQUIRE(aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(o, 16) &&
-                 aligned(dout, 16) && aligned(dq, 8) && aligned(dk, 8) && aligned(dv, 8),
-             ZK_EALIGN, "%s: tensors must be 16-byte aligned", who);
+  const int al = ragged ? 4 : 16, gal = ragged ? 4 : 8;
+  ZK_REQUIRE(aligned(q, al) && aligned(k, al) && aligned(v, al) && aligned(o, al) &&
+                 aligned(dout, al) && aligned(dq, gal) && aligned(dk, gal) && aligned(dv, gal),
+             ZK_EALIGN, "%s: tensors must be %d-byte aligned", who, al);
   const int64_t n_kt = (desc->Skv + DkdvCfg<128>::BK - 1) / DkdvCfg<128>::BK;
   const dim3 kgrid(static_cast<unsigned>(n_kt * desc->B * desc->Hkv));
   const bool q_full = desc->Sq % DkdvCfg<128>::MQ == 0;
@@ -753,6 +810,35 @@ static int attn_bwd_impl(const char* who, const zk_attn_desc* desc, const void* 
         hipLaunchKernelGGL((attn_bwd_dkdv<T, D, false>), kgrid, dim3(256), 0, s, a);        \
     }                                                                                       \
   } while (0)
+  if (ragged) {
+#define ZK_BWD_R(T, D, KR)                                                                   \
+  do {                                                                                       \
+    const int64_t n_qt = (desc->Sq + DqCfg<D>::BM - 1) / DqCfg<D>::BM;                       \
+    if (n_qt > 0)                                                                            \
+      hipLaunchKernelGGL((attn_bwd_dq<T, D, false, KR>),                                     \
+                         dim3(static_cast<unsigned>(n_qt * desc->B * desc->Hq)),             \
+                         dim3(DqCfg<D>::NT), 0, s, a, n_qt);                                 \
+    if (n_kt > 0)                                                                            \
+      hipLaunchKernelGGL((attn_bwd_dkdv<T, D, false, KR>), kgrid, dim3(256), 0, s, a);       \
+  } while (0)
+#define ZK_BWD_RT(T)                              \
+  switch ((desc->d + 15) / 16) {                  \
+    case 3: ZK_BWD_R(T, 64, 3); break;            \
+    case 4: ZK_BWD_R(T, 64, 4); break;            \
+    case 5: ZK_BWD_R(T, 128, 5); break;           \
+    case 6: ZK_BWD_R(T, 128, 6); break;           \
+    case 7: ZK_BWD_R(T, 128, 7); break;           \
+    default: ZK_BWD_R(T, 128, 8); break;          \
+  }
+    if (desc->dtype == ZK_BF16) {
+      ZK_BWD_RT(bf16)
+    } else {
+      ZK_BWD_RT(f16)
+    }
+#undef ZK_BWD_RT
+#undef ZK_BWD_R
+    return launch_status(who);
+  }
   if (desc->dtype == ZK_BF16) {
     if (desc->d == 128) ZK_BWD(bf16, 128); else ZK_BWD(bf16, 64);
   } else {

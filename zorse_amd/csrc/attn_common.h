@@ -65,11 +65,13 @@ void launch_attn_bwd_f32(const AttnArgs& a, hipStream_t s);
 // values pass through an LDS tile [D][NCOL] held by up to four arrays the
 // caller no longer needs, RP feature rows each (p0 first); every wave must be
 // done with them on entry.  16-byte stores, NCOL / 8 lanes per feature row.
-// Ends with a barrier, so the arrays may be reused at once.
-template <typename T, int D, int NCOL, int RP>
-__device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[D / 32], float scale,
+// Ends with a barrier, so the arrays may be reused at once.  NB: the 32-row
+// blocks x holds; KR > 0 (a ragged head dim): only the first `d` feature rows
+// are stored.
+template <typename T, int D, int NCOL, int RP, int KR, int NB>
+__device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[NB], float scale,
                                                       T* p0, T* p1, T* p2, T* p3, T* dst,
-                                                      int64_t ld, int ncols) {
+                                                      int64_t ld, int ncols, int d) {
   static_assert(RP % 32 == 0 && D <= 4 * RP, "feature rows per array");
   constexpr int NT = 2 * NCOL;  // threads: 64 per 32 columns
   const int tid = threadIdx.x, l32 = tid & 31, g = (tid >> 5) & 1, wave = tid >> 6;
@@ -79,7 +81,7 @@ __device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[D / 32],
     return p + (r % RP) * NCOL;
   };
 #pragma unroll
-  for (int nt = 0; nt < D / 32; ++nt)
+  for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const int r = 32 * nt + 8 * (j >> 2) + 4 * g + (j & 3);
@@ -89,10 +91,10 @@ __device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[D / 32],
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   constexpr int CPR = NCOL / 8;  // 16-byte chunks per feature row
 #pragma unroll
-  for (int i = 0; i < D * CPR / NT; ++i) {
+  for (int i = 0; i < 32 * NB * CPR / NT; ++i) {
     const int id = NT * i + tid;
     const int r = id / CPR, col = 8 * (id % CPR);
-    if (col < ncols)
+    if (col < ncols && (KR == 0 || r < d))
       *reinterpret_cast<u32x4*>(dst + r * ld + col) = *reinterpret_cast<const u32x4*>(row_ptr(r) + col);
   }
   __syncthreads();
@@ -344,9 +346,90 @@ struct TileLoader {
   }
 };
 
-// Number of vector-memory instructions tile_load_async issues per wave.
-template <int D, int ROWS>
-constexpr int tile_load_insts() { return ROWS * D / 8 / 256; }
+// The tile load for an even head dim d < D (a head row may start at any 4-byte
+// address): chunks past the row read nothing (their offset lies
+// past the resource's end, which writes zeros), the chunk that straddles the
+// row's end also holds up to 6 elements of whatever follows (mask_cols below
+// takes them out), and the resource ends with the tensor's last row, so that
+// chunk never reads past the allocation and rows past the end arrive as zeros.
+template <typename T, int D, int ROWS, int NT = 256>
+struct RaggedLoader {
+  static constexpr int NI = ROWS * D / 8 / NT;
+  static constexpr int RSTEP = NT / (D / 8);
+  static_assert(NI >= 1 && RSTEP % 16 == 0, "unsupported tile shape");
+  uint32_t lane_off;
+  int64_t row_bytes;
+
+  __device__ __forceinline__ void init(int64_t ld, int64_t d) {
+    const int tid = threadIdx.x;
+    const int row = tid / (D / 8);
+    const int c = (tid % (D / 8)) ^ tile_sw<D>(row);
+    lane_off = c * 8 < d ? static_cast<uint32_t>(row * ld * static_cast<int64_t>(sizeof(T)) + c * 16)
+                         : 0x80000000u;
+    row_bytes = d * static_cast<int64_t>(sizeof(T));
+  }
+
+  __device__ __forceinline__ void issue(T* tile, const T* gbase, int64_t ld, int64_t g0,
+                                        int64_t nrows, bool) const {
+    const int wave_chunk0 = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) & ~63);
+    int64_t left = (nrows - 1 - g0) * ld * static_cast<int64_t>(sizeof(T)) + row_bytes;
+    left = left < 0 ? 0 : left > 0x7fffffff ? 0x7fffffff : left;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(gbase + g0 * ld), 0, static_cast<int>(left), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t soff =
+          static_cast<uint32_t>(static_cast<int64_t>(i) * RSTEP * ld * static_cast<int64_t>(sizeof(T)));
+      dma_lds<16>(r, lane_off, soff, tile + (i * NT + wave_chunk0) * 8);
+    }
+  }
+};
+
+// Elements col .. col + 7 of a row of d (even; 4-byte aligned), zeros from d on.
+template <typename T>
+__device__ __forceinline__ typename Mfma<T>::vec8 load_cols8(const T* row, int col, int d) {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+  u32x4 w = {0, 0, 0, 0};
+  if (col + 8 <= d) {
+    w = *reinterpret_cast<const u32x4_a4*>(row + col);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (col + 2 * i < d) w[i] = *reinterpret_cast<const unsigned int*>(row + col + 2 * i);
+  }
+  return __builtin_bit_cast(typename Mfma<T>::vec8, w);
+}
+
+// Elements col .. col + 3 of a row of d (even; 4-byte aligned): those below d.
+template <typename T, typename T4>
+__device__ __forceinline__ void store_cols4(T* row, int col, int d, T4 v) {
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned int u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+  const u32x2 w = __builtin_bit_cast(u32x2, v);
+  if (col + 4 <= d)
+    *reinterpret_cast<u32x2_a4*>(row + col) = w;
+  else if (col < d)
+    *reinterpret_cast<unsigned int*>(row + col) = w[0];
+}
+
+// v = elements col .. col + 7 of an LDS tile's row: those from d (even) on
+// become zeros (the other operand is zero there too, but 0 x Inf would not be).
+template <typename T>
+__device__ __forceinline__ typename Mfma<T>::vec8 mask_cols(typename Mfma<T>::vec8 v, int col,
+                                                            int d) {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  u32x4 w = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] &= col + 2 * i < d ? ~0u : 0u;
+  return __builtin_bit_cast(typename Mfma<T>::vec8, w);
+}
+
+// Head dims of the ragged kernels: KR = ceil(d / 16) MFMA steps over a tile of
+// D = 64 or 128 columns.  Smaller ones and odd ones are refused.
+__host__ __device__ constexpr bool ragged_head_dim(int64_t d) {
+  return d % 2 == 0 && ((d > 32 && d < 64) || (d > 64 && d < 128));
+}
 
 // s_waitcnt vmcnt(N) (expcnt / lgkmcnt left unconstrained), gfx9 encoding.
 template <int N>

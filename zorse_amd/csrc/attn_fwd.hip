@@ -28,6 +28,16 @@
 // ragged end of the key range; tiles entirely masked for a wave are skipped,
 // tiles entirely visible skip the per-element mask.  Causal blocks are
 // launched heaviest-first.
+//
+// Head dims between 32 and 128 other than 64 (zk_attn_fwd_ragged): the same
+// kernels over the tile of the next larger dim, with the DMA's offsets, one
+// register mask and the stores stopping at the head's end, and only
+// ceil(d / 16) score steps and ceil(d / 32) output blocks computed.  Heads
+// start at any 4-byte address, so a 200-byte row of d = 100 spans up to three
+// 128-byte lines: forward / dQ / dK dV of 32 heads, 2048 causal tokens take
+// 67 / 86 / 124 us at d = 100, 54 / 73 / 96 at d = 84 and 39 / 57 / 79 at
+// d = 48, where zero-padded 128-wide heads take 62 / 81 / 115 (64-wide 38 /
+// 55 / 76) plus 226 us of copies and fills to make and undo them (d = 100).
 #include <type_traits>
 
 #include "attn_common.h"
@@ -54,13 +64,18 @@ __device__ __forceinline__ float fast_exp2(float x) {
 static constexpr float kRescaleThreshold = 8.0f;
 
 // kFull: Skv is a multiple of the key tile, so no tile runs past the end.
-template <typename T, int D, bool kFull>
+// KR: 0 for a head dim of D; else the head dim a.d is an even number in
+// (16 KR - 16, 16 KR], and the tile's columns from a.d on hold nothing: KR of
+// the D / 16 score steps and the 32-column blocks that cover a.d are computed.
+template <typename T, int D, bool kFull, int KR = 0>
 __global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
   typedef FwdCfg<T, D> C;
   typedef Mfma<T> M;
   typedef typename M::vec8 V8;
   constexpr int BM = C::BM, BN = C::BN, NT = C::NT;
+  constexpr int KS = KR ? KR : D / 16, NB = (KS + 1) / 2;
+  const int hd = KR ? static_cast<int>(a.d) : D;
   // each stage its own array: the compiler then sees that the next tile's
   // asynchronous loads do not alias this tile's reads (and adds no wait)
   __shared__ __attribute__((aligned(16))) T K0[BN * D], K1[BN * D], V0[BN * D], V1[BN * D];
@@ -82,10 +97,12 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
   const T* Vp = static_cast<const T*>(a.v) + b * a.v_sb + hk * a.v_sh;
 
   // Q^T operand: lane holds Q[my_q][16 ks + 8 g .. +7].
-  V8 qreg[D / 16];
+  V8 qreg[KS];
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    if (my_q < a.Sq)
+  for (int ks = 0; ks < KS; ++ks) {
+    if (my_q < a.Sq && KR)
+      qreg[ks] = load_cols8<T>(Qp + my_q * a.q_ss, 16 * ks + 8 * g, hd);
+    else if (my_q < a.Sq)
       qreg[ks] = *reinterpret_cast<const V8*>(Qp + my_q * a.q_ss + 16 * ks + 8 * g);
     else
       qreg[ks] = V8{};
@@ -98,9 +115,14 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
   const int64_t t_hi = kv_hi > kv_lo ? (kv_hi + BN - 1) / BN : t_lo;
 
   // K / V tiles double-buffered in LDS, loaded asynchronously one tile ahead
-  TileLoader<T, D, BN, NT> kload, vload;
-  kload.init(a.k_ss);
-  vload.init(a.v_ss);
+  std::conditional_t<KR != 0, RaggedLoader<T, D, BN, NT>, TileLoader<T, D, BN, NT>> kload, vload;
+  if constexpr (KR != 0) {
+    kload.init(a.k_ss, hd);
+    vload.init(a.v_ss, hd);
+  } else {
+    kload.init(a.k_ss);
+    vload.init(a.v_ss);
+  }
   auto issue = [&](int64_t k0, int st) {
     kload.issue(st ? K1 : K0, Kp, a.k_ss, k0, a.Skv, kFull);
     vload.issue(st ? V1 : V0, Vp, a.v_ss, k0, a.Skv, kFull);
@@ -113,9 +135,9 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
   const int rbase = 2 * tile_off<D>(l32, 8 * g);
   const int tbase = 2 * tile_off<D>(4 * g + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
 
-  f32x16 o[D / 32];
+  f32x16 o[NB];
 #pragma unroll
-  for (int nt = 0; nt < D / 32; ++nt) o[nt] = f32x16{};
+  for (int nt = 0; nt < NB; ++nt) o[nt] = f32x16{};
   float m_ref = -INFINITY, l_i = 0.f;
   const float c2 = a.scale_log2;
   // Visible keys of this lane's query form one range [vis_lo, vis_lo + vis_span]
@@ -173,9 +195,10 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
       for (int tt = 0; tt < BN / 32; ++tt) {
         s[tt] = f32x16{};
 #pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) {
-          const V8 kv = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(Kt) +
-                                                     (rb ^ (ks << 5)) + tt * 32 * D * 2);
+        for (int ks = 0; ks < KS; ++ks) {
+          V8 kv = *reinterpret_cast<const V8*>(reinterpret_cast<const char*>(Kt) +
+                                               (rb ^ (ks << 5)) + tt * 32 * D * 2);
+          if (KR && ks == KS - 1) kv = mask_cols<T>(kv, 16 * ks + 8 * g, hd);
           s[tt] = M::mma(kv, qreg[ks], s[tt]);
         }
       }
@@ -204,7 +227,7 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
         m_ref = m_new;
         l_i *= alpha;
 #pragma unroll
-        for (int nt = 0; nt < D / 32; ++nt) o[nt] *= alpha;
+        for (int nt = 0; nt < NB; ++nt) o[nt] *= alpha;
       }
       const float mc = m_ref == -INFINITY ? 0.f : m_ref * c2;
 
@@ -225,7 +248,7 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
 #pragma unroll
       for (int kk = 0; kk < BN / 16; ++kk) {
 #pragma unroll
-        for (int nt = 0; nt < D / 32; ++nt) {
+        for (int nt = 0; nt < NB; ++nt) {
           typedef short s16x4 __attribute__((ext_vector_type(4)));
           typedef short s16x8 __attribute__((ext_vector_type(8)));
           typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -257,13 +280,13 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
   // transposed store below write the same values (the compiler may round
   // o * inv in one step, e.g. v_fma_mix for fp16, or in two)
 #pragma unroll
-  for (int nt = 0; nt < D / 32; ++nt)
+  for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[nt][j] = to_f32(static_cast<T>(o[nt][j] * inv));
   if (my_q < a.Sq) {
     T* Op = static_cast<T*>(a.out) + b * a.o_sb + hq * a.o_sh + my_q * a.o_ss;
 #pragma unroll
-    for (int nt = 0; nt < D / 32; ++nt)
+    for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
       for (int a4 = 0; a4 < 4; ++a4) {
         const int d0 = 32 * nt + 8 * a4 + 4 * g;
@@ -271,7 +294,10 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
         T4 w;
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = static_cast<T>(o[nt][4 * a4 + e]);
-        *reinterpret_cast<T4*>(Op + d0) = w;
+        if constexpr (KR != 0)
+          store_cols4(Op, d0, hd, w);
+        else
+          *reinterpret_cast<T4*>(Op + d0) = w;
       }
     if (g == 0)
       a.lse_out[(b * a.Hq + hq) * a.Sq + my_q] =
@@ -283,9 +309,9 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
     // once every wave is past its last step)
     __syncthreads();
     const int64_t left = a.Sq - q0;
-    store_rows_transposed<T, D, BM, BN * D / BM>(
-        o, 1.f, K0, K1, V0, V1, static_cast<T*>(a.o_t) + hq * D * a.t_ld + b * a.Sq + q0, a.t_ld,
-        static_cast<int>(left < BM ? left : BM));
+    store_rows_transposed<T, D, BM, BN * D / BM, KR>(
+        o, 1.f, K0, K1, V0, V1, static_cast<T*>(a.o_t) + hq * hd * a.t_ld + b * a.Sq + q0, a.t_ld,
+        static_cast<int>(left < BM ? left : BM), hd);
   }
 }
 
@@ -295,7 +321,7 @@ using namespace zk;
 
 namespace zk {
 // Validates a descriptor; shared by forward and backward entry points.
-int check_attn_desc(const zk_attn_desc* d, const char* who, bool bwd) {
+int check_attn_desc(const zk_attn_desc* d, const char* who, bool bwd, bool ragged) {
   ZK_REQUIRE(d != nullptr, ZK_EINVAL, "%s: null descriptor", who);
   ZK_REQUIRE(d->dtype == ZK_BF16 || d->dtype == ZK_F16 || d->dtype == ZK_F32,
              ZK_EDTYPE, "%s: bad dtype %d", who, d->dtype);
@@ -313,27 +339,31 @@ int check_attn_desc(const zk_attn_desc* d, const char* who, bool bwd) {
                "%s: fp32 path supports head_dim <= 128 (got %lld)", who,
                (long long)d->d);
   } else {
-    ZK_REQUIRE(d->d == 64 || d->d == 128, ZK_EUNSUPPORTED,
+    ZK_REQUIRE(ragged || d->d == 64 || d->d == 128, ZK_EUNSUPPORTED,
                "%s: head_dim must be 64 or 128 (got %lld)", who, (long long)d->d);
-    // 16-byte vector access along d and along rows
+    ZK_REQUIRE(!ragged || ragged_head_dim(d->d), ZK_EUNSUPPORTED,
+               "%s: head_dim must be even, in 34 .. 62 or 66 .. 126 (got %lld)", who,
+               (long long)d->d);
+    // 16-byte (ragged: 4-byte) vector access along d and along rows
+    const int64_t vec = ragged ? 2 : 8;
     const int64_t strides[] = {d->q_sb, d->q_ss, d->q_sh, d->k_sb, d->k_ss,
                                d->k_sh, d->v_sb, d->v_ss, d->v_sh, d->o_sb,
                                d->o_ss, d->o_sh};
     for (int64_t s : strides)
-      ZK_REQUIRE(s % 8 == 0, ZK_EALIGN,
-                 "%s: strides must be multiples of 8 elements (got %lld)", who,
-                 (long long)s);
+      ZK_REQUIRE(s % vec == 0, ZK_EALIGN,
+                 "%s: strides must be multiples of %lld elements (got %lld)", who,
+                 (long long)vec, (long long)s);
     if (bwd) {
       const int64_t bs[] = {d->dq_sb, d->dq_ss, d->dq_sh, d->dk_sb, d->dk_ss,
                             d->dk_sh, d->dv_sb, d->dv_ss, d->dv_sh};
       for (int64_t s : bs)
-        ZK_REQUIRE(s % 8 == 0, ZK_EALIGN,
-                   "%s: grad strides must be multiples of 8 elements", who);
+        ZK_REQUIRE(s % vec == 0, ZK_EALIGN,
+                   "%s: grad strides must be multiples of %lld elements", who, (long long)vec);
     }
     // the tile loaders keep a 32-row span of one tensor in a 32-bit byte offset
     const int64_t rs[] = {d->q_ss, d->k_ss, d->v_ss, d->o_ss};
     for (int64_t s : rs)
-      ZK_REQUIRE(s >= 0 && s < (int64_t(1) << 26), ZK_EUNSUPPORTED,
+      ZK_REQUIRE(s >= 0 && s < (int64_t(1) << (ragged ? 23 : 26)), ZK_EUNSUPPORTED,
                  "%s: row stride %lld out of range", who, (long long)s);
   }
   ZK_REQUIRE(d->B * d->Hq * ((d->Sq + 127) / 128) < 0x7fffffffLL, ZK_EINVAL,
@@ -359,8 +389,8 @@ void fill_args(AttnArgs& a, const zk_attn_desc* d) {
 
 static int attn_fwd_impl(const char* who, const zk_attn_desc* desc, const void* q,
                          const void* k, const void* v, void* o, float* lse, void* o_t,
-                         int64_t ld_t, zk_stream_t stream) {
-  int rc = check_attn_desc(desc, who, false);
+                         int64_t ld_t, bool ragged, zk_stream_t stream) {
+  int rc = check_attn_desc(desc, who, false, ragged);
   if (rc != ZK_OK) return rc;
   if (o_t != nullptr) {
     ZK_REQUIRE(desc->dtype != ZK_F32, ZK_EUNSUPPORTED,
@@ -383,8 +413,35 @@ static int attn_fwd_impl(const char* who, const zk_attn_desc* desc, const void* 
     launch_attn_fwd_f32(a, s);
     return launch_status(who);
   }
-  ZK_REQUIRE(aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(o, 16),
-             ZK_EALIGN, "%s: q/k/v/o must be 16-byte aligned", who);
+  const int al = ragged ? 4 : 16;
+  ZK_REQUIRE(aligned(q, al) && aligned(k, al) && aligned(v, al) && aligned(o, al),
+             ZK_EALIGN, "%s: q/k/v/o must be %d-byte aligned", who, al);
+  if (ragged) {
+#define ZK_FWD_R(T, D, KR)                                                              \
+  do {                                                                                  \
+    constexpr int BM = FwdCfg<T, D>::BM, NT = FwdCfg<T, D>::NT;                         \
+    const int64_t n_qt = (desc->Sq + BM - 1) / BM;                                      \
+    const dim3 grid(static_cast<unsigned>(n_qt * desc->B * desc->Hq));                  \
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, KR>), grid, dim3(NT), 0, s, a, n_qt); \
+  } while (0)
+#define ZK_FWD_RT(T)                              \
+  switch ((desc->d + 15) / 16) {                  \
+    case 3: ZK_FWD_R(T, 64, 3); break;            \
+    case 4: ZK_FWD_R(T, 64, 4); break;            \
+    case 5: ZK_FWD_R(T, 128, 5); break;           \
+    case 6: ZK_FWD_R(T, 128, 6); break;           \
+    case 7: ZK_FWD_R(T, 128, 7); break;           \
+    default: ZK_FWD_R(T, 128, 8); break;          \
+  }
+    if (desc->dtype == ZK_BF16) {
+      ZK_FWD_RT(bf16)
+    } else {
+      ZK_FWD_RT(f16)
+    }
+#undef ZK_FWD_RT
+#undef ZK_FWD_R
+    return launch_status(who);
+  }
 #define ZK_FWD(T, D)                                                                    \
   do {                                                                                  \
     constexpr int BM = FwdCfg<T, D>::BM, NT = FwdCfg<T, D>::NT;                         \
@@ -406,12 +463,20 @@ static int attn_fwd_impl(const char* who, const zk_attn_desc* desc, const void* 
 
 extern "C" int zk_attn_fwd(const zk_attn_desc* desc, const void* q, const void* k, const void* v,
                            void* o, float* lse, zk_stream_t stream) {
-  return attn_fwd_impl("zk_attn_fwd", desc, q, k, v, o, lse, nullptr, 0, stream);
+  return attn_fwd_impl("zk_attn_fwd", desc, q, k, v, o, lse, nullptr, 0, false, stream);
+}
+
+extern "C" int zk_attn_fwd_ragged(const zk_attn_desc* desc, const void* q, const void* k,
+                                  const void* v, void* o, float* lse, zk_stream_t stream) {
+  const char* who = "zk_attn_fwd_ragged";
+  ZK_REQUIRE(desc == nullptr || desc->dtype != ZK_F32, ZK_EUNSUPPORTED,
+             "%s: 2-byte dtypes only", who);
+  return attn_fwd_impl(who, desc, q, k, v, o, lse, nullptr, 0, true, stream);
 }
 
 extern "C" int zk_attn_fwd_t(const zk_attn_desc* desc, const void* q, const void* k,
                              const void* v, void* o, float* lse, void* o_t, int64_t ld_t,
                              zk_stream_t stream) {
   ZK_REQUIRE(o_t != nullptr, ZK_EINVAL, "zk_attn_fwd_t: null transposed output");
-  return attn_fwd_impl("zk_attn_fwd_t", desc, q, k, v, o, lse, o_t, ld_t, stream);
+  return attn_fwd_impl("zk_attn_fwd_t", desc, q, k, v, o, lse, o_t, ld_t, false, stream);
 }

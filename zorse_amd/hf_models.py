@@ -28,8 +28,7 @@ Shapes, as the factories set them:
     mask HF's Mistral model builds) with models/mistral.py:16-26.
 llama_6.7b, 13b, 33b, 65b and the Mistral models have head dim 128, which the
 attention kernels take directly; llama_1b..5b have head dims 48, 68, 84, 98,
-110, for which the layer zero-pads q, k, v to 64 / 128 around the attention
-kernels (layer._attn_padded_dim).
+110, which run on the ragged attention kernels (kernels.attn_ragged_takes).
 """
 from __future__ import annotations
 

@@ -479,16 +479,31 @@ def _attn_desc(q, k, v, o, scale, causal, window, dq=None, dk=None, dv=None):
                          dtype_code(q.dtype))
 
 
+def attn_ragged_takes(*tensors: torch.Tensor) -> bool:
+    """Whether the ragged attention kernels take these [B, S, H, d] tensors as
+    they are: 2-byte types, even head dims of 34 .. 62 and 66 .. 126, rows that
+    start at 4-byte addresses less than 2^23 elements apart."""
+    for t in tensors:
+        d, (sb, ss, sh, unit) = t.shape[3], t.stride()
+        if t.dtype not in _LOWP or d % 2 or not (32 < d < 64 or 64 < d < 128) or unit != 1 \
+                or (sb | ss | sh) % 2 or not 0 <= ss < 1 << 23 or t.data_ptr() % 4:
+            return False
+    return True
+
+
 def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool = True,
              window: int = 0, scale: float | None = None, out: torch.Tensor | None = None,
-             out_t: torch.Tensor | None = None):
+             out_t: torch.Tensor | None = None, ragged: bool = False):
     """Flash attention forward on [B,S,H,d] views.  Returns (o, lse) with o
     [B,Sq,Hq,d] (contiguous unless ``out`` is given) and lse fp32 [B,Hq,Sq].
 
     ``out_t`` (2-byte types, Sq % 8 == 0): a [Hq d, >= B Sq] buffer with unit
     column stride that also receives O transposed (row head * d + i, column
     batch * Sq + position), from the kernel's epilogue -- the operand of the
-    o_proj weight gradient."""
+    o_proj weight gradient.
+
+    ``ragged`` (no ``out_t``): the kernels for 2-byte tensors whose head dim is
+    none of 64 and 128 (see attn_ragged_takes)."""
     dev = _require_gpu(q, k, v, out, out_t)
     B, Sq, Hq, d = q.shape
     if scale is None:
@@ -499,6 +514,12 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool 
         raise ValueError("out has the wrong shape")
     desc = _attn_desc(q, k, v, out, scale, causal, window)
     lse = torch.empty(B, Hq, Sq, device=dev, dtype=torch.float32)
+    if ragged:
+        if out_t is not None:
+            raise ValueError("the ragged kernels write no transposed output")
+        check(lib().zk_attn_fwd_ragged(desc, ptr(q), ptr(k), ptr(v), ptr(out), ptr(lse),
+                                       stream_handle(dev)), "zk_attn_fwd_ragged")
+        return out, lse
     if out_t is None:
         check(lib().zk_attn_fwd(desc, ptr(q), ptr(k), ptr(v), ptr(out), ptr(lse),
                                 stream_handle(dev)), "zk_attn_fwd")
@@ -514,7 +535,7 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool 
 
 def attn_bwd(q, k, v, o, do, lse, *, causal: bool = True, window: int = 0,
              scale: float | None = None, dq=None, dk=None, dv=None, rope=None,
-             transposed=None):
+             transposed=None, ragged: bool = False):
     """Flash attention backward.  Returns (dq, dk, dv); outputs may be given
     as (strided) views, e.g. slices of one fused [T, (Hq+2Hkv) d] buffer.
 
@@ -527,7 +548,9 @@ def attn_bwd(q, k, v, o, do, lse, *, causal: bool = True, window: int = 0,
     contiguous, one common row stride, a multiple of 8; 2-byte dtypes, S a
     multiple of 8) that also receive dq / dk / dv transposed -- the operand
     layout of the projections' weight-gradient GEMMs -- from the kernels'
-    epilogues."""
+    epilogues.
+
+    ``ragged`` (without ``rope`` and ``transposed``): as for attn_fwd."""
     dev = _require_gpu(q, k, v, o, do, lse, dq, dk, dv,
                        *(rope[:3] if rope is not None else ()),
                        *(transposed if transposed is not None else ()))
@@ -547,6 +570,13 @@ def attn_bwd(q, k, v, o, do, lse, *, causal: bool = True, window: int = 0,
     desc = _attn_desc(q, k, v, o, scale, causal, window, dq, dk, dv)
     nbytes = lib().zk_attn_bwd_workspace(desc)
     ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    if ragged:
+        if rope is not None or transposed is not None:
+            raise ValueError("the ragged kernels take neither rope nor transposed")
+        check(lib().zk_attn_bwd_ragged(desc, ptr(q), ptr(k), ptr(v), ptr(o), ptr(do), ptr(lse),
+                                       ptr(dq), ptr(dk), ptr(dv), ptr(ws), nbytes,
+                                       stream_handle(dev)), "zk_attn_bwd_ragged")
+        return dq, dk, dv
     if transposed is not None:
         ld_t = _check_transposed(transposed, q, k)
     if rope is None:

@@ -258,14 +258,17 @@ def _fused_gate_up_takes(n2, F):
             and h % 64 == 0 and T % 8 == 0 and F % 8 == 0)
 
 
-# Head dims the MFMA attention kernels do not take (they take 64 and 128; the
-# fp32 kernels any head dim up to 128): q, k, v are zero-padded to the next of
-# those, attention runs with the real head dim's scale -- the padded
+# Head dims other than 64 and 128 in 2-byte types (the fp32 kernels take any up
+# to 128): the ragged attention kernels read and write the heads as they lie in
+# the q|k|v buffer, and RoPE is a pass of its own (its pairs lie across the MFMA
+# layout's lanes) over q and k before, and over dq and dk after.  A 3B layer
+# (32 heads of 100, 2048 tokens, forward + backward): 1.9 ms, where zero-padded
+# copies of q, k, v, o and dO around the 128-wide kernels took 2.2 ms.
+#
+# What those do not take either (head dims up to 32): q, k, v are zero-padded to
+# 64 or 128, attention runs with the real head dim's scale -- the padded
 # coordinates add nothing to Q K^T, P V or any gradient -- and the results are
-# sliced back.  RoPE rotates the real coordinates in place before (forward),
-# and its transpose is applied to dq / dk after the backward.  The padding
-# copies are torch copies into zeroed buffers (head dims 48 - 110 of the
-# smaller llama_* HF-factory models only).
+# sliced back.  The padding copies are torch copies into zeroed buffers.
 def _attn_padded_dim(spec, dtype):
     d = spec.head_dim
     if dtype == torch.float32 or d in (64, 128):
@@ -336,6 +339,8 @@ def layer_forward(x: torch.Tensor, w: FlatViews, spec: LayerSpec, attn_cache=Non
         dp = _attn_padded_dim(spec, x.dtype)
         if dp is None:
             o, lse = K.attn_fwd(q, k, v, causal=spec.causal, window=spec.window)
+        elif K.attn_ragged_takes(q, k, v):
+            o, lse = K.attn_fwd(q, k, v, causal=spec.causal, window=spec.window, ragged=True)
         else:
             o, lse = K.attn_fwd(_pad_heads(q, dp), _pad_heads(k, dp), _pad_heads(v, dp),
                                 causal=spec.causal, window=spec.window,
@@ -422,6 +427,11 @@ def layer_backward(dout: torch.Tensor, saved, w: FlatViews, spec: LayerSpec,
                    rope=(cos, sin, positions, spec.interleaved_rope),
                    transposed=None if dqkvt is None else
                    (dqkvt[:kv0], dqkvt[kv0:kv1], dqkvt[kv1:]))
+    elif K.attn_ragged_takes(q, k, v, dq, dk, dv, o2.view(B, S, Hq, d), do2.view(B, S, Hq, d)):
+        K.attn_bwd(q, k, v, o2.view(B, S, Hq, d), do2.view(B, S, Hq, d), lse, causal=spec.causal,
+                   window=spec.window, dq=dq, dk=dk, dv=dv, ragged=True)
+        K.rope_(dq, dk, cos, sin, positions=positions, interleaved=spec.interleaved_rope,
+                inverse=True)
     else:
         grads = K.attn_bwd(*(_pad_heads(t, dp) for t in (q, k, v, o2.view(B, S, Hq, d),
                                                          do2.view(B, S, Hq, d))), lse,
