@@ -82,11 +82,12 @@ def test_gemm_misaligned_equals_aligned(dev):
 
 
 # B, S, K, Hq, Hkv, d: tiles 64 (heads of 64 in the epilogue, of 128 by the
-# pass), 64 x 128, 128 split, 128, masked 256
+# pass), 64 x 128, 128 split, 128, masked 256, 128 x 256
 @pytest.mark.parametrize("B,S,K,Hq,Hkv,d,inter", [
     (3, 11, 72, 4, 2, 64, False), (3, 11, 72, 2, 1, 128, True), (2, 37, 688, 64, 1, 128, False),
     (1, 197, 232, 62, 1, 128, True), (3, 619, 8, 63, 1, 128, False),
-    (1, 2184, 456, 27, 1, 128, False)])
+    (1, 2184, 456, 27, 1, 128, False), (4, 512, 512, 22, 1, 128, False),
+    (4, 512, 256, 40, 4, 64, True)])
 def test_gemm_rope_tiles(dev, B, S, K, Hq, Hkv, d, inter):
     """The RoPE epilogue of each tile writes what the product and the RoPE
     pass write, with positions that wrap inside a tile."""

@@ -59,13 +59,19 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
 //   4095 x 4096 x 32000 dX    731 / 1015 / 1323 / 2839 / -   (256)
 // The K-split tiles are for grids of at most one workgroup per CU, and not
 // built for weight gradients, whose reduction (the tokens) is the short side.
-static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_km) {
+// `half`: the 128 x 256 tile is a candidate too, again for at most one
+// workgroup per CU -- products on the grid (its masked form, measured, was 4 to
+// 8 % behind 128 x 128 up to K = 4096) without the SwiGLU epilogue, A along K:
+//   4096 x 2048 x 8192 NT      99.7, on 128 x 128 tiles 109
+//   2048 x 3072 x 16384 dX    177,   on 128 x 128 tiles 201
+static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_km, bool half) {
   struct Cost {
     gemm::Tile t;
     int per_cu;
     double launch, edge, step, part;
   };
   static constexpr Cost kAlongK[] = {{gemm::k256, 1, 0.5, 9.5, 1.29, 0.82},
+                                     {gemm::k128x256, 1, 0.5, 5.5, 0.745, 0.72},
                                      {gemm::k128, 2, 4.7, 0.8, 0.926, 0.73},
                                      {gemm::k128x2, 1, 0.0, 5.7, 0.59, 0.82},
                                      {gemm::k64, 2, 4.4, 0.0, 0.48, 0.60},
@@ -75,13 +81,15 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
                                      {gemm::k64, 2, 2.9, 1.9, 0.36, 0.59}};
   if (a_km && !b_km) return gemm::k128;  // no layer product: one tile is built
   const Cost* c = a_km ? kKMajor : kAlongK;
-  const int nc = a_km ? 3 : 5;
+  const int nc = a_km ? 3 : 6;
   const int64_t cus = device_cus(), steps = (K + gemm::BK - 1) / gemm::BK;
   gemm::Tile best = gemm::k256;
   double best_us = 0;
   for (int i = 0; i < nc; ++i) {
     const int64_t n = gemm::tile_count(c[i].t, M, N), cap = cus * c[i].per_cu;
-    if ((c[i].t == gemm::k128x2 || c[i].t == gemm::k64x128) && n > cus) continue;
+    const bool is_half = c[i].t == gemm::k128x256;
+    if ((is_half || c[i].t == gemm::k128x2 || c[i].t == gemm::k64x128) && n > cus) continue;
+    if (is_half && !half) continue;
     const int64_t full = n / cap, rem = n % cap;
     double part = 0;  // two per CU: a lone workgroup runs faster than a pair
     if (rem > 0)
@@ -121,27 +129,43 @@ extern "C" int zk_gemm_path(int64_t M, int64_t N, int64_t K, int64_t lda, int a_
 namespace {
 
 // A 2-byte product on tile t; on_grid: tiled_takes.
-template <typename T, int EPI>
-void launch_256(bool on_grid, const gemm::GemmArgs& ga, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(gemm::tile_count(gemm::k256, ga.M, ga.N)));
-  if (on_grid)
-    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, EPI, false, false>), grid, dim3(256), 0, s, ga);
+template <typename T, int EPI, int MB>
+void launch_tiled(bool on_grid, const gemm::GemmArgs& ga, hipStream_t s) {
+  const gemm::Tile t = MB == 8 ? gemm::k256 : gemm::k128x256;
+  const dim3 grid(static_cast<unsigned>(gemm::tile_count(t, ga.M, ga.N)));
+  if (on_grid || MB == 4)
+    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, EPI, false, false, false, MB>), grid, dim3(256),
+                       0, s, ga);
   else
-    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, EPI, false, false, true>), grid, dim3(256), 0, s,
-                       ga);
+    hipLaunchKernelGGL((gemm::gemm_tiled_kernel<T, EPI, false, false, true, 8>), grid, dim3(256),
+                       0, s, ga);
 }
 
 template <int EPI>
 void launch_mfma(bool bf, gemm::Tile t, bool on_grid, int a_km, int b_km, const gemm::GemmArgs& ga,
                  hipStream_t s) {
-  if (t != gemm::k256)
+  const bool half = t == gemm::k128x256;
+  if (t != gemm::k256 && !half) {
     gemm::launch_ring(bf, EPI, a_km, b_km, t, ga, s);
-  else if (a_km || b_km)
-    gemm::launch_tiled_kmajor(bf, a_km, b_km, !on_grid, ga, s);
-  else if (bf)
-    launch_256<bf16, EPI>(on_grid, ga, s);
+    return;
+  }
+  if (a_km || b_km) {
+    gemm::launch_tiled_kmajor(bf, a_km, b_km, !on_grid, half, ga, s);
+    return;
+  }
+  if constexpr (EPI != 1) {
+    if (half) {
+      if (bf)
+        launch_tiled<bf16, EPI, 4>(on_grid, ga, s);
+      else
+        launch_tiled<f16, EPI, 4>(on_grid, ga, s);
+      return;
+    }
+  }
+  if (bf)
+    launch_tiled<bf16, EPI, 8>(on_grid, ga, s);
   else
-    launch_256<f16, EPI>(on_grid, ga, s);
+    launch_tiled<f16, EPI, 8>(on_grid, ga, s);
 }
 
 template <typename T>
@@ -208,7 +232,7 @@ extern "C" int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, 
   if (mfma && dtype == ZK_F32)
     gemm::launch_ring_f32(a_km, b_km, ga, s);
   else if (mfma)
-    launch_mfma<0>(dtype == ZK_BF16, a_km && !b_km && on_grid ? gemm::k256 : pick_tile(M, N, K, a_km, b_km),
+    launch_mfma<0>(dtype == ZK_BF16, a_km && !b_km && on_grid ? gemm::k256 : pick_tile(M, N, K, a_km, b_km, on_grid),
                    on_grid, a_km, b_km, ga, s);
   else if (dtype == ZK_BF16)
     launch_general<bf16>(a_km, b_km, ga, s);
@@ -261,10 +285,10 @@ extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t l
              aligned(b, 16) && aligned(c, 16) && (head_dim == 64 || head_dim == 128) &&
              aligned(cos, 16) && aligned(sin, 16) && S < (int64_t(1) << 30) &&
              n_pos < (int64_t(1) << 24);
-  const gemm::Tile tile = epi ? pick_tile(M, N, K, false, false) : gemm::k256;
+  const gemm::Tile tile = epi ? pick_tile(M, N, K, false, false, on_grid) : gemm::k256;
   // the 256-wide tile rotates whole 128-column blocks of sequences of at least
   // 128 tokens; a 64-wide one holds heads of 64 only
-  if (tile == gemm::k256) epi = epi && rot_cols % 128 == 0 && S >= 128;
+  if (tile == gemm::k256 || tile == gemm::k128x256) epi = epi && rot_cols % 128 == 0 && S >= 128;
   if (tile == gemm::k64) epi = epi && head_dim == 64;
   if (!epi) {
     const int rc = zk_gemm(a, lda, 0, b, ldb, 0, c, ldc, nullptr, 0, M, N, K, dtype, stream);
@@ -354,7 +378,7 @@ extern "C" int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
   ga.N = 2 * F;
   ga.K = K;
   const bool on_grid = tiled_takes(M, 2 * F, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype);
-  launch_mfma<1>(dtype == ZK_BF16, pick_tile(M, 2 * F, K, false, false), on_grid, 0, 0, ga,
+  launch_mfma<1>(dtype == ZK_BF16, pick_tile(M, 2 * F, K, false, false, false), on_grid, 0, 0, ga,
                  as_stream(stream));
   return launch_status("zk_gemm_swiglu");
 }

@@ -292,9 +292,9 @@ __device__ __forceinline__ float silu_fast(float g) {
 
 // AKM / BKM: operand A / B is K-major (see the top of the file).  EPI 1
 // takes NT operands only.
-// Operand-read order of a set (see mm_ld): A0, B0 .. B7, A1 .. A7, with A
-// pieces numbered 0 .. 7 and B pieces 8 .. 15.
-__device__ constexpr int kReadOrder[16] = {0, 8, 9, 10, 11, 12, 13, 14, 15, 1, 2, 3, 4, 5, 6, 7};
+// Operand-read order of a set (see mm_ld): A0, B0 .. B7, A1 .. A(MB-1), with
+// A pieces numbered 0 .. MB-1 and B pieces MB .. MB+7.
+constexpr int read_order(int MB, int i) { return i == 0 ? 0 : i <= 8 ? MB + i - 1 : i - 8; }
 
 // RAG: M, N, K off the grid (M and N multiples of 8 where an operand is
 // contiguous along them, K of 8 for an NT operand).  The buffer resources end
@@ -302,11 +302,16 @@ __device__ constexpr int kReadOrder[16] = {0, 8, 9, 10, 11, 12, 13, 14, 15, 1, 2
 // columns of an NT tile past K are sent out of range lane by lane, K is
 // padded to an even number of steps (at least four) that way, and stores are
 // masked per 8-column chunk.  The SwiGLU epilogue takes silu in the IEEE form.
-template <typename T, int EPI, bool AKM, bool BKM, bool RAG = false>
+// MB: 16-row MFMA blocks per wave along M -- 8 (the 256 x 256 tile) or 4 (a
+// 128 x 256 tile, on the grid, not for the SwiGLU epilogue or A K-major: a
+// product with half a round of 256 x 256 tiles gets twice the workgroups with
+// half the work each, and a third more MFMA work per byte loaded than in 128 x
+// 128 tiles).
+template <typename T, int EPI, bool AKM, bool BKM, bool RAG = false, int MB = 8>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_tiled_kernel(GemmArgs args) {
   static_assert(EPI == 0 || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
-  constexpr int MB = 8;         // 16-row MFMA blocks per wave along M
+  static_assert(MB == 8 || (MB == 4 && EPI != 1 && !AKM && !RAG), "128-row tiles");
   constexpr int TBM = 32 * MB;  // tile rows
   constexpr int WR = 16 * MB;   // rows per wave
   const T* __restrict__ A = static_cast<const T*>(args.a);
@@ -447,14 +452,16 @@ void gemm_tiled_kernel(GemmArgs args) {
                            static_cast<uint32_t>(16 * p * ldb * static_cast<int64_t>(sizeof(T))), p);
     }
   };
-  // The 64 MFMAs of set q in rows of eight.  After row c: A piece c (LK 1: of
-  // step k into ring stage lst) or B piece c (LK 2: into B stage lst), and,
-  // when RD, two operand pieces of substep s0 of stages (ra, rb) into set q0,
-  // in the order the next set's MFMAs use them: its first row needs A piece 0
-  // and all eight B pieces, row c A piece c, so the reads go A0, B0 .. B7, A1
-  // .. A7 (B7 is in flight from row 4, three rows before it is needed; read
-  // last, it stalled the next set's first MFMA for the LDS latency at every
-  // substep).  The fences keep this order.
+  // The 8 MB MFMAs of set q in rows of eight.  After row c: A piece c (LK 1:
+  // of step k into ring stage lst) or 8 / MB B pieces (LK 2: into B stage
+  // lst), and, when RD, (MB + 8) / MB operand pieces of substep s0 of stages
+  // (ra, rb) into set q0, in the order the next set's MFMAs use them: its
+  // first row needs A piece 0 and all eight B pieces, row c A piece c, so the
+  // reads go A0, B0 .. B7, A1 .. A(MB-1) (for MB = 8, B7 is in flight from row
+  // 4, three rows before it is needed; read last, it stalled the next set's
+  // first MFMA for the LDS latency at every substep).  The fences keep this
+  // order.
+  constexpr int RPR = (MB + 8) / MB, BPR = 8 / MB;
   auto mm_ld = [&](int q, int lk, int lst, int64_t k, bool rd, int ra, int rb, int s0,
                    int q0) __attribute__((always_inline)) {
 #pragma unroll
@@ -462,11 +469,14 @@ void gemm_tiled_kernel(GemmArgs args) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[c][j] = Mm::mma16(xa[q][c], xb[q][j], acc[c][j]);
       if (rd) {
-        rd_piece(ra, rb, s0, q0, kReadOrder[2 * c]);
-        rd_piece(ra, rb, s0, q0, kReadOrder[2 * c + 1]);
+#pragma unroll
+        for (int u = 0; u < RPR; ++u) rd_piece(ra, rb, s0, q0, read_order(MB, RPR * c + u));
       }
       if (lk == 1) loadA(lst, k, c);
-      if (lk == 2) loadB(lst, k, c);
+      if (lk == 2) {
+#pragma unroll
+        for (int u = 0; u < BPR; ++u) loadB(lst, k, BPR * c + u);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -548,8 +558,14 @@ void gemm_tiled_kernel(GemmArgs args) {
   int el = lane;
   asm volatile("" : "+v"(el));  // keep the epilogue's index math after the loop
   // each wave's 16 x 132-float staging area (and for EPI 1 the z tile after
-  // it) in a 32 KB A stage each (Bs0 for wave 3)
-  float* ws = reinterpret_cast<float*>(wave < 3 ? &As[wave * (TBM * BK)] : Bs0);
+  // it) in a 32 KB A stage each (Bs0 for wave 3); for 128-row tiles two in the
+  // 48 KB A ring, Bs0 and Bs1
+  float* ws;
+  if constexpr (MB == 8)
+    ws = reinterpret_cast<float*>(wave < 3 ? &As[wave * (TBM * BK)] : Bs0);
+  else
+    ws = wave < 2 ? reinterpret_cast<float*>(As) + wave * (16 * 132)
+                  : reinterpret_cast<float*>(wave == 2 ? Bs0 : Bs1);
   const int e16 = el & 15, eq = el >> 4;
   typedef T T8 __attribute__((ext_vector_type(8)));
   // EPI 2: the wave's 128 columns hold whole heads (head dim 2 rhalf = 64 or
@@ -854,17 +870,19 @@ __global__ __launch_bounds__(256) void gemm_gen_kernel(GemmArgs args) {
 }
 
 // The tiled kernel with A and / or B K-major (gemm_kmajor.hip), bf16 or fp16;
-// ragged: off the grid (RAG), not for A K-major with B along K.
-void launch_tiled_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, bool ragged, const GemmArgs& ga,
-                         hipStream_t s);
+// ragged: off the grid (RAG), not for A K-major with B along K; half: the 128 x
+// 256 tile, on the grid with B K-major alone.
+void launch_tiled_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, bool ragged, bool half,
+                         const GemmArgs& ga, hipStream_t s);
 
-// Tiles of the 2-byte MFMA kernels: the 256 x 256 pipeline above, and the
+// Tiles of the 2-byte MFMA kernels: the 256 x 256 pipeline above, its 128 x 256
+// form (k128x256: on the grid, A along K, plain and RoPE epilogues), and the
 // small-tile kernel of gemm_ring.h with 4 waves (k128: 128 x 128, k64: 64 x
 // 64, two workgroups per CU) or 8 waves split over K (k128x2: 128 x 128,
 // k64x128: 64 x 128, one workgroup per CU).
-enum Tile { k256, k128, k128x2, k64, k64x128 };
+enum Tile { k256, k128x256, k128, k128x2, k64, k64x128 };
 inline int tile_rows(Tile t) { return t == k256 ? 256 : t == k64 || t == k64x128 ? 64 : 128; }
-inline int tile_cols(Tile t) { return t == k256 ? 256 : t == k64 ? 64 : 128; }
+inline int tile_cols(Tile t) { return t == k256 || t == k128x256 ? 256 : t == k64 ? 64 : 128; }
 inline int64_t tile_count(Tile t, int64_t M, int64_t N) {
   return ((M + tile_rows(t) - 1) / tile_rows(t)) * ((N + tile_cols(t) - 1) / tile_cols(t));
 }

@@ -9,8 +9,12 @@ namespace gemm {
 
 namespace {
 template <typename T>
-void launch_t(bool akm, bool bkm, bool ragged, const GemmArgs& ga, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(((ga.M + BM - 1) / BM) * ((ga.N + BN - 1) / BN)));
+void launch_t(bool akm, bool bkm, bool ragged, bool half, const GemmArgs& ga, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(tile_count(half ? k128x256 : k256, ga.M, ga.N)));
+  if (half) {
+    hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, false, true, false, 4>), grid, dim3(256), 0, s, ga);
+    return;
+  }
 #define ZK_TILED(A, B, R) \
   hipLaunchKernelGGL((gemm_tiled_kernel<T, 0, A, B, R>), grid, dim3(256), 0, s, ga)
   if (akm && bkm) {
@@ -24,12 +28,12 @@ void launch_t(bool akm, bool bkm, bool ragged, const GemmArgs& ga, hipStream_t s
 }
 }  // namespace
 
-void launch_tiled_kmajor(bool bf16_, bool a_kmajor, bool b_kmajor, bool ragged, const GemmArgs& ga,
-                         hipStream_t s) {
+void launch_tiled_kmajor(bool bf16_, bool a_kmajor, bool b_kmajor, bool ragged, bool half,
+                         const GemmArgs& ga, hipStream_t s) {
   if (bf16_)
-    launch_t<bf16>(a_kmajor, b_kmajor, ragged, ga, s);
+    launch_t<bf16>(a_kmajor, b_kmajor, ragged, half, ga, s);
   else
-    launch_t<f16>(a_kmajor, b_kmajor, ragged, ga, s);
+    launch_t<f16>(a_kmajor, b_kmajor, ragged, half, ga, s);
 }
 
 }  // namespace gemm
