@@ -177,6 +177,17 @@ int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb
             int b_kmajor, void* c, int64_t ldc, const void* r, int64_t ldr, int64_t M,
             int64_t N, int64_t K, int dtype, zk_stream_t stream);
 
+/* zk_gemm with a workspace: a product whose tiles would leave most CUs idle
+ * over a long reduction splits it over workgroups, partial sums in fp32 in the
+ * workspace (16-byte aligned), and adds them in a second launch.  The bytes
+ * it wants (0: none); with less it runs as zk_gemm does.  ldr < 0: no R. */
+int64_t zk_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor,
+                          int64_t ldb, int b_kmajor, int64_t ldc, int64_t ldr, int dtype);
+int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
+               int b_kmajor, void* c, int64_t ldc, const void* r, int64_t ldr,
+               int64_t M, int64_t N, int64_t K, int dtype, void* workspace,
+               int64_t workspace_bytes, zk_stream_t stream);
+
 /* Whether a launch with 16-byte aligned pointers lies on the grid of the
  * 256 x 256 MFMA pipeline (host-only, no GPU call): ZK_GEMM_TILED -- 2-byte type, M and N multiples
  * of 256, K a multiple of 128 and at least 256, leading dimensions multiples

@@ -64,7 +64,8 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
 // 8 % behind 128 x 128 up to K = 4096) without the SwiGLU epilogue, A along K:
 //   4096 x 2048 x 8192 NT      99.7, on 128 x 128 tiles 109
 //   2048 x 3072 x 16384 dX    177,   on 128 x 128 tiles 201
-static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_km, bool half) {
+static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_km, bool half,
+                            double* cost = nullptr) {
   struct Cost {
     gemm::Tile t;
     int per_cu;
@@ -103,6 +104,52 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     if (i == 0 || us < best_us) {
       best = c[i].t;
       best_us = us;
+    }
+  }
+  if (cost != nullptr) *cost = best_us;
+  return best;
+}
+
+// Splitting the reduction over workgroups (gemm_split.hip): `parts` ranges of
+// split_k on tiles of at most one workgroup per CU, when the estimate of the
+// rule above for tiles and parts, plus the sum over the parts (5 us with its
+// launch, and 8 bytes an output and part at 3.5 TB/s), is 11 us below that of
+// the best single pass: a layer whose products are that short is bound by the
+// host, whom the workspace and the second launch cost 7 us (a forward of the
+// 2048-wide layer at 128 tokens: 112 us, 121 with its down product split, 22
+// against 15 us).  A along K, 2-byte types.  Measured, us, single pass / split:
+//     64 x 4096 x 11008 NT     47 /  24     64 x 2688 x 21504 dX    93 /  28
+//    256 x 4096 x 22016 dX    122 /  67    512 x 5120 x 13824 NT   130 /  77
+//   1024 x 2688 x 21504 dX    168 / 111   2046 x 1536 x 49152 dX   424 / 245
+struct Split {
+  gemm::Tile tile;
+  int parts;  // 0: not split
+  int64_t split_k;
+};
+static Split pick_split(int64_t M, int64_t N, int64_t K, bool on_grid) {
+  struct Cost {
+    gemm::Tile t;
+    double launch, edge, step;
+  };
+  static constexpr Cost kCost[] = {{gemm::k256, 0.5, 9.5, 1.29},
+                                   {gemm::k128x2, 0.0, 5.7, 0.59},
+                                   {gemm::k64x128, 0.0, 5.1, 0.45}};
+  Split best{gemm::k256, 0, 0};
+  const int64_t cus = device_cus(), steps = (K + gemm::BK - 1) / gemm::BK;
+  if (K < 1024 || M * N > (int64_t(1) << 24)) return best;
+  double best_us = 0;
+  pick_tile(M, N, K, false, false, on_grid, &best_us);
+  best_us -= 11;
+  for (const Cost& c : kCost) {
+    const int64_t n = gemm::tile_count(c.t, M, N);
+    for (int64_t p = 2; p <= 16 && n * p <= cus && steps / p >= 4; ++p) {
+      const int64_t st = (steps + p - 1) / p;
+      if ((steps + st - 1) / st != p) continue;  // the last range would be empty
+      const double us = c.launch + c.edge + st * c.step + 5.0 + 8e-6 / 3.5 * p * M * N;
+      if (us < best_us) {
+        best_us = us;
+        best = Split{c.t, static_cast<int>(p), st * gemm::BK};
+      }
     }
   }
   return best;
@@ -187,9 +234,28 @@ void launch_general(int a_km, int b_km, const gemm::GemmArgs& ga, hipStream_t s)
 
 }  // namespace
 
+extern "C" int64_t zk_gemm_workspace(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor,
+                                     int64_t ldb, int b_kmajor, int64_t ldc, int64_t ldr,
+                                     int dtype) {
+  if (a_kmajor || (dtype != ZK_BF16 && dtype != ZK_F16) ||
+      !masked_takes(M, N, K, lda, 0, ldb, b_kmajor != 0, ldc, ldr < 0 ? 8 : ldr, dtype))
+    return 0;
+  const Split sp = pick_split(
+      M, N, K, tiled_takes(M, N, K, lda, 0, ldb, b_kmajor != 0, ldc, ldr < 0 ? 8 : ldr, dtype));
+  return sp.parts * M * N * 4;
+}
+
 extern "C" int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
                        int b_kmajor, void* c, int64_t ldc, const void* r, int64_t ldr, int64_t M,
                        int64_t N, int64_t K, int dtype, zk_stream_t stream) {
+  return zk_gemm_ws(a, lda, a_kmajor, b, ldb, b_kmajor, c, ldc, r, ldr, M, N, K, dtype, nullptr, 0,
+                    stream);
+}
+
+extern "C" int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
+                          int b_kmajor, void* c, int64_t ldc, const void* r, int64_t ldr,
+                          int64_t M, int64_t N, int64_t K, int dtype, void* workspace,
+                          int64_t workspace_bytes, zk_stream_t stream) {
   ZK_REQUIRE(valid_dtype(dtype), ZK_EDTYPE, "zk_gemm: bad dtype %d", dtype);
   ZK_REQUIRE(M >= 0 && N >= 0 && K >= 0, ZK_EINVAL, "zk_gemm: bad shape");
   const int a_km = a_kmajor != 0, b_km = b_kmajor != 0;
@@ -229,6 +295,18 @@ extern "C" int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, 
   ga.N = N;
   ga.K = K;
   hipStream_t s = as_stream(stream);
+  if (mfma && !a_km && dtype != ZK_F32 && workspace != nullptr && aligned(workspace, 16)) {
+    const Split sp = pick_split(M, N, K, on_grid);
+    if (sp.parts > 0 && workspace_bytes >= sp.parts * M * N * 4) {
+      gemm::GemmArgs part = ga;
+      part.c = workspace;
+      part.split_k = sp.split_k;
+      gemm::launch_split(dtype == ZK_BF16, b_km, sp.tile, sp.parts, part, s);
+      gemm::launch_split_sum(dtype == ZK_BF16, static_cast<const float*>(workspace), sp.parts, ga,
+                             s);
+      return launch_status("zk_gemm");
+    }
+  }
   if (mfma && dtype == ZK_F32)
     gemm::launch_ring_f32(a_km, b_km, ga, s);
   else if (mfma)

@@ -145,6 +145,7 @@ struct GemmArgs {
   const int64_t* rpos;
   int64_t rnpos, rS, rcols;
   int rhalf, rpair;
+  int64_t split_k;  // EPI 3: the reduction range of one workgroup
 };
 
 // NT tile swizzle: the 16-byte chunk c of row r sits at chunk position
@@ -291,7 +292,8 @@ __device__ __forceinline__ float silu_fast(float g) {
 }
 
 // AKM / BKM: operand A / B is K-major (see the top of the file).  EPI 1
-// takes NT operands only.
+// takes NT operands only.  EPI 3: workgroup (x, y) of the grid sums the y-th
+// split_k of the reduction and stores it in fp32 to C + y M N, rows of N.
 // Operand-read order of a set (see mm_ld): A0, B0 .. B7, A1 .. A(MB-1), with
 // A pieces numbered 0 .. MB-1 and B pieces MB .. MB+7.
 constexpr int read_order(int MB, int i) { return i == 0 ? 0 : i <= 8 ? MB + i - 1 : i - 8; }
@@ -310,14 +312,21 @@ constexpr int read_order(int MB, int i) { return i == 0 ? 0 : i <= 8 ? MB + i - 
 template <typename T, int EPI, bool AKM, bool BKM, bool RAG = false, int MB = 8>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_tiled_kernel(GemmArgs args) {
-  static_assert(EPI == 0 || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
+  static_assert(EPI == 0 || (!AKM && !BKM) || (EPI == 3 && !AKM && RAG),
+                "the SwiGLU and RoPE epilogues take NT operands, partial sums A along K");
   static_assert(MB == 8 || (MB == 4 && EPI != 1 && !AKM && !RAG), "128-row tiles");
   constexpr int TBM = 32 * MB;  // tile rows
   constexpr int WR = 16 * MB;   // rows per wave
   const T* __restrict__ A = static_cast<const T*>(args.a);
   const T* __restrict__ B = static_cast<const T*>(args.b);
   const int64_t lda = args.lda, ldb = args.ldb;
-  const int64_t M = args.M, N = args.N, K = args.K;
+  const int64_t k_first = EPI == 3 ? blockIdx.y * args.split_k : 0;
+  const int64_t k_left = args.K - k_first;
+  const int64_t M = args.M, N = args.N, K = EPI == 3 && args.split_k < k_left ? args.split_k : k_left;
+  if constexpr (EPI == 3) {
+    A += k_first;
+    B += BKM ? k_first * args.ldb : k_first;
+  }
   typedef Mfma<T> Mm;
   typedef typename Mm::vec8 V8;
   __shared__ __attribute__((aligned(16))) T As[3 * TBM * BK];  // ring of three
@@ -679,6 +688,12 @@ void gemm_tiled_kernel(GemmArgs args) {
         const int64_t grow = row0 + rr;
         const int64_t gcol = n0 + wn * 128 + 8 * ch;
         if (RAG && (grow >= M || gcol >= N)) continue;
+        if constexpr (EPI == 3) {
+          float* const W = reinterpret_cast<float*>(C) + (blockIdx.y * M + grow) * N + gcol;
+          *reinterpret_cast<float4*>(W) = lo;
+          *reinterpret_cast<float4*>(W + 4) = hi;
+          continue;
+        }
         if (R != nullptr) {
           const T8 rv = *reinterpret_cast<const T8*>(R + grow * args.ldr + gcol);
 #pragma unroll
@@ -893,6 +908,11 @@ void launch_ring(bool bf16, int epi, bool a_kmajor, bool b_kmajor, Tile t, const
                  hipStream_t s);
 void launch_ring_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, Tile t, const GemmArgs& ga,
                         hipStream_t s);
+// The partial sums of a reduction split into `parts` ranges of ga.split_k (EPI
+// 3 of either kernel, into the workspace ga.c), and their sum: A along K, tiles
+// k256, k128x2 and k64x128 (gemm_split.hip).
+void launch_split(bool bf16, bool b_kmajor, Tile t, int parts, const GemmArgs& ga, hipStream_t s);
+void launch_split_sum(bool bf16, const float* ws, int parts, const GemmArgs& out, hipStream_t s);
 // fp32 (gemm_f32.hip)
 void launch_ring_f32(bool a_kmajor, bool b_kmajor, const GemmArgs& ga, hipStream_t s);
 

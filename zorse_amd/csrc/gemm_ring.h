@@ -157,7 +157,7 @@ __device__ __forceinline__ typename RingOp<T>::vec kmaj_operand_n(const T* tile,
 template <typename T, int EPI, bool AKM, bool BKM, int MB, int NB, int RB, int WPE, int KS>
 __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void gemm_ring_kernel(GemmArgs args) {
-  static_assert(EPI == 0 || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
+  static_assert(EPI == 0 || (EPI == 3 && !AKM) || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
   constexpr int TBM = 32 * MB, TBN = 32 * NB, WR = 16 * MB, WC = 16 * NB;
   typedef RingOp<T> Mm;
   typedef typename Mm::vec V8;
@@ -174,7 +174,10 @@ void gemm_ring_kernel(GemmArgs args) {
   T* const Bs = lds + RA * TA::EL;
 
   const int64_t lda = args.lda, ldb = args.ldb;
-  const int64_t M = args.M, N = args.N, K = args.K;
+  // EPI 3: the blockIdx.y-th split_k of the reduction, into C + blockIdx.y M N
+  const int64_t k_first = EPI == 3 ? blockIdx.y * args.split_k : 0;
+  const int64_t k_left = args.K - k_first;
+  const int64_t M = args.M, N = args.N, K = EPI == 3 && args.split_k < k_left ? args.split_k : k_left;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, q4 = lane >> 4;
   const int wm = (wave >> 1) & 1, wn = wave & 1;
@@ -191,11 +194,13 @@ void gemm_ring_kernel(GemmArgs args) {
 
   // first element of each operand's tile, bytes left from there to the
   // operand's end, and the bytes of one K step
-  const char* Ab = static_cast<const char*>(args.a) + ES * (AKM ? m0 : m0 * lda);
+  const char* Ab = static_cast<const char*>(args.a) +
+                   ES * (AKM ? m0 + k_first * lda : m0 * lda + k_first);
   const int64_t a_left = ES * (AKM ? (K - 1) * lda + M - m0 : (M - 1 - m0) * lda + K);
   const int64_t a_step = AKM ? ES * BK * lda : ES * BK;
   const int64_t b_rows = EPI == 1 ? N / 2 : N, b_r0 = EPI == 1 ? f0 : n0;
-  const char* Bb = static_cast<const char*>(args.b) + ES * (BKM ? b_r0 : b_r0 * ldb);
+  const char* Bb = static_cast<const char*>(args.b) +
+                   ES * (BKM ? b_r0 + k_first * ldb : b_r0 * ldb + k_first);
   const char* B2b = EPI == 1 ? static_cast<const char*>(args.b2) + ES * b_r0 * ldb : nullptr;
   const int64_t b_left = ES * (BKM ? (K - 1) * ldb + b_rows - b_r0 : (b_rows - 1 - b_r0) * ldb + K);
   const int64_t b_step = BKM ? ES * BK * ldb : ES * BK;
@@ -489,6 +494,10 @@ void gemm_ring_kernel(GemmArgs args) {
       if (gr >= M || gc >= N) continue;
       float v[8];
       chunk(row, 8 * ch, v);
+      if constexpr (EPI == 3) {
+        Vec8<float>::store(static_cast<float*>(args.c) + (blockIdx.y * M + gr) * N + gc, v);
+        continue;
+      }
       if constexpr (EPI == 2) if (gc < args.rcols) {
         // this chunk rotated: its pair is the chunk rhalf columns away in the
         // same head (half-split) or inside the chunk (interleaved); the

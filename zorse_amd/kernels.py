@@ -9,6 +9,7 @@ GPU tensor these functions raise.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -217,6 +218,13 @@ def _gemm_operand(name: str, t: torch.Tensor):
     return rows, cols, max(ld, 1)
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace(dev, M, N, K, lda, ldb, b_kmajor, ldc, ldr, code) -> int:
+    """Bytes zk_gemm_ws wants for a product with A along the reduction -- a
+    function of the sizes alone, looked up in 0.3 us where the call takes 2."""
+    return lib().zk_gemm_workspace(M, N, K, lda, 0, ldb, b_kmajor, ldc, ldr, code)
+
+
 def gemm(a: torch.Tensor, b: torch.Tensor, *, a_kmajor: bool = False, b_kmajor: bool = False,
          residual: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """C = op(a) op(b)^T (+ residual) from the hand-written GEMMs (zk_gemm):
@@ -224,7 +232,9 @@ def gemm(a: torch.Tensor, b: torch.Tensor, *, a_kmajor: bool = False, b_kmajor: 
     [K, N]), each with unit column stride -- so x W^T is gemm(x, W), dY W is
     gemm(dY, W, b_kmajor=True) and dY^T X is gemm(dY, X, a_kmajor=True,
     b_kmajor=True), all on the tensors as stored.  bf16 / fp16 (fp32
-    accumulation, one rounding) or fp32; every tensor shares the dtype.
+    accumulation, one rounding) or fp32; every tensor shares the dtype.  Long
+    reductions onto few tiles are split over workgroups (zk_gemm_ws, its
+    workspace allocated here on the current stream).
     ``out`` / ``residual``: [M, N] with unit column stride."""
     dev = _require_gpu(a, b, residual, out)
     if a.dtype != b.dtype or a.dtype not in (torch.float32, *_LOWP):
@@ -246,9 +256,19 @@ def gemm(a: torch.Tensor, b: torch.Tensor, *, a_kmajor: bool = False, b_kmajor: 
         if residual.shape != (M, N) or residual.dtype != a.dtype:
             raise ValueError(f"gemm: residual must be [{M}, {N}] of the operands' dtype")
         _, _, ldr = _gemm_operand("residual", residual)
+    code = dtype_code(a.dtype)
+    if K >= 1024 and not a_kmajor and M * N <= 1 << 24:  # may split its reduction
+        nbytes = _gemm_workspace(dev, M, N, K, lda, ldb, int(b_kmajor), ldc,
+                                 ldr if residual is not None else -1, code)
+        if nbytes:
+            ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+            check(lib().zk_gemm_ws(ptr(a), lda, 0, ptr(b), ldb, int(b_kmajor), ptr(out), ldc,
+                                   ptr(residual) if residual is not None else None, ldr, M, N, K,
+                                   code, ptr(ws), nbytes, stream_handle(dev)), "zk_gemm_ws")
+            return out
     check(lib().zk_gemm(ptr(a), lda, int(a_kmajor), ptr(b), ldb, int(b_kmajor), ptr(out), ldc,
                         ptr(residual) if residual is not None else None, ldr, M, N, K,
-                        dtype_code(a.dtype), stream_handle(dev)), "zk_gemm")
+                        code, stream_handle(dev)), "zk_gemm")
     return out
 
 
@@ -258,7 +278,7 @@ def gemm_rope(x: torch.Tensor, w: torch.Tensor, *, seq_len: int, rot_cols: int, 
     """x W^T with the rotary embedding applied to its first ``rot_cols``
     columns (whole heads of ``head_dim``), rows being tokens b * seq_len + s
     (zk_gemm_rope): the q|k|v projection and the RoPE pass in one call, equal
-    to gemm(x, w) followed by rope_ on the q and k heads.  cos / sin /
+    to gemm(x, w) in one pass followed by rope_ on the q and k heads.  cos / sin /
     positions as for rope_."""
     dev = _require_gpu(x, w, cos, sin, positions, out)
     if x.dtype != w.dtype or x.dtype not in (torch.float32, *_LOWP):
