@@ -400,6 +400,23 @@ int zk_ce_fwd_chunk(const void* logits, int64_t rows, int64_t cols, int64_t ld,
 int zk_ce_bwd_chunk(void* logits, int64_t rows, int64_t cols, int64_t ld,
                     const int64_t* labels, int64_t col0, const float* lse,
                     float scale, int dtype, zk_stream_t stream);
+/* The same with scale = *grad / max(*n_valid, 1) read on the device. */
+int zk_ce_bwd_chunk_mean(void* logits, int64_t rows, int64_t cols, int64_t ld,
+                         const int64_t* labels, int64_t col0, const float* lse,
+                         const float* grad, const int64_t* n_valid, int dtype,
+                         zk_stream_t stream);
+/* Before the first chunk: row_label = label, or -1 where it is ignore_index;
+ * run_max = -inf, run_sum = target_logit = 0; stats = {rows with a label,
+ * rows whose label is outside [0, vocab)}, written to device memory and to
+ * host memory the device can write (valid once the stream has passed). */
+int zk_ce_labels(const int64_t* labels, int64_t rows, int64_t vocab, int64_t ignore_index,
+                 int64_t* row_label, float* run_max, float* run_sum, float* target_logit,
+                 int64_t* stats, int64_t* host_stats, zk_stream_t stream);
+/* After the last: lse per row and loss = sum of (lse - target_logit) over the
+ * labelled rows / max(stats[0], 1). */
+int zk_ce_finish(const int64_t* row_label, int64_t rows, const float* run_max,
+                 const float* run_sum, const float* target_logit, const int64_t* stats,
+                 float* lse, float* loss, zk_stream_t stream);
 
 /* ------------------------------------------------------------- Utilities --
  * Dtype conversion of a contiguous buffer (the autocast weight cast and the

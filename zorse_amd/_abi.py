@@ -124,6 +124,10 @@ SIGNATURES = {
     "zk_cast": (_int, [_ptr, _int, _ptr, _int, _i64, _int, _ptr]),
     "zk_ce_fwd_chunk": (_int, [_ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _int,
                                _ptr]),
+    "zk_ce_bwd_chunk_mean": (_int, [_ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _int,
+                                    _ptr]),
+    "zk_ce_labels": (_int, [_ptr, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "zk_ce_finish": (_int, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "zk_ce_bwd_chunk": (_int, [_ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _f32, _int, _ptr]),
     "zk_transpose": (_int, [_ptr, _i64, _ptr, _i64, _i64, _i64, _int, _ptr]),
     "zk_copy_to_host": (_int, [_ptr, _ptr, _i64, _int, _ptr]),

@@ -35,11 +35,11 @@ def _fwd_chunk(logits, labels, col0, run_max, run_sum, target):
           "zk_ce_fwd_chunk")
 
 
-def _bwd_chunk(logits, labels, col0, lse, scale):
-    check(lib().zk_ce_bwd_chunk(ptr(logits), logits.shape[0], logits.shape[1], logits.stride(0),
-                                ptr(labels), col0, ptr(lse), float(scale),
-                                dtype_code(logits.dtype), stream_handle(logits.device)),
-          "zk_ce_bwd_chunk")
+def _bwd_chunk(logits, labels, col0, lse, grad, stats):
+    check(lib().zk_ce_bwd_chunk_mean(ptr(logits), logits.shape[0], logits.shape[1],
+                                     logits.stride(0), ptr(labels), col0, ptr(lse), ptr(grad),
+                                     ptr(stats), dtype_code(logits.dtype),
+                                     stream_handle(logits.device)), "zk_ce_bwd_chunk_mean")
 
 
 class LMHeadCrossEntropyFunction(torch.autograd.Function):
@@ -58,23 +58,33 @@ class LMHeadCrossEntropyFunction(torch.autograd.Function):
         x = x.contiguous()
         w = weight if weight.dtype == x.dtype else weight.to(x.dtype)
         T, V = x.shape[0], w.shape[0]
-        ignored = labels == ignore_index
-        if bool((~ignored & ((labels < 0) | (labels >= V))).any()):
+        dev, given = x.device, labels.contiguous()
+        # row labels (-1: ignored, skipped by the kernels), running max, sum and
+        # label logit; stats = (labelled rows, labels out of range), which the
+        # host reads after the chunks are enqueued, without waiting for them
+        labels = torch.empty_like(given)
+        run_max, run_sum, target, lse = torch.empty(4, T, device=dev, dtype=torch.float32)
+        stats = torch.empty(2, device=dev, dtype=torch.int64)
+        host = torch.empty(2, dtype=torch.int64, pin_memory=True)
+        loss = torch.empty((), device=dev, dtype=torch.float32)
+        check(lib().zk_ce_labels(ptr(given), T, V, ignore_index, ptr(labels), ptr(run_max),
+                                 ptr(run_sum), ptr(target), ptr(stats), ptr(host),
+                                 stream_handle(dev)), "zk_ce_labels")
+        checked = torch.cuda.Event()
+        checked.record(torch.cuda.current_stream(dev))
+        try:
+            for c0 in range(0, V, chunk):
+                logits = K.gemm(x, w[c0:c0 + chunk])
+                _fwd_chunk(logits, labels, c0, run_max, run_sum, target)
+            check(lib().zk_ce_finish(ptr(labels), T, ptr(run_max), ptr(run_sum), ptr(target),
+                                     ptr(stats), ptr(lse), ptr(loss), stream_handle(dev)),
+                  "zk_ce_finish")
+        finally:  # the kernel writes host memory: it outlives that
+            checked.synchronize()
+        if int(host[1]):
             raise ValueError(f"labels must lie in [0, {V}) or equal ignore_index "
                              f"({ignore_index})")
-        # the kernels skip rows whose label is negative
-        labels = torch.where(ignored, torch.full_like(labels, -1), labels).contiguous()
-        run_max = torch.full((T,), float("-inf"), device=x.device, dtype=torch.float32)
-        run_sum = torch.zeros(T, device=x.device, dtype=torch.float32)
-        target = torch.zeros(T, device=x.device, dtype=torch.float32)
-        for c0 in range(0, V, chunk):
-            logits = K.gemm(x, w[c0:c0 + chunk])
-            _fwd_chunk(logits, labels, c0, run_max, run_sum, target)
-        lse = run_max + torch.log(run_sum)
-        valid = labels >= 0
-        n_valid = valid.sum()
-        loss = torch.where(valid, lse - target, torch.zeros_like(lse)).sum() / n_valid.clamp(min=1)
-        ctx.save_for_backward(x, w, labels, lse, n_valid)
+        ctx.save_for_backward(x, w, labels, lse, stats)
         ctx.chunk = chunk
         ctx.weight_dtype = weight.dtype
         # one chunk covered the vocabulary: keep its logits for the backward
@@ -83,15 +93,16 @@ class LMHeadCrossEntropyFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        x, w, labels, lse, n_valid = ctx.saved_tensors
+        x, w, labels, lse, stats = ctx.saved_tensors
         chunk = ctx.chunk
-        T, V = x.shape[0], w.shape[0]
-        scale = (g / n_valid.clamp(min=1)).item()
+        V = w.shape[0]
+        g = g.to(device=x.device, dtype=torch.float32)
+        lse, labels, stats = lse.contiguous(), labels.contiguous(), stats.contiguous()
         if ctx.logits is not None:
             # the forward's logits, overwritten in place by their gradient (a
             # second backward through a retained graph recomputes them)
             dlog, ctx.logits = ctx.logits, None
-            _bwd_chunk(dlog, labels, 0, lse, scale)
+            _bwd_chunk(dlog, labels, 0, lse, g, stats)
             dx = K.gemm(dlog, w, b_kmajor=True)
             dw = K.gemm(dlog, x, a_kmajor=True, b_kmajor=True)
             if dw.dtype != ctx.weight_dtype:
@@ -102,7 +113,7 @@ class LMHeadCrossEntropyFunction(torch.autograd.Function):
         for c0 in range(0, V, chunk):
             wc = w[c0:c0 + chunk]
             dlog = K.gemm(x, wc)
-            _bwd_chunk(dlog, labels, c0, lse, scale)
+            _bwd_chunk(dlog, labels, c0, lse, g, stats)
             dx.add_(K.gemm(dlog, wc, b_kmajor=True))
             K.gemm(dlog, x, a_kmajor=True, b_kmajor=True, out=dw[c0:c0 + chunk])
         if dw.dtype != ctx.weight_dtype:
