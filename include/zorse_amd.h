@@ -225,6 +225,14 @@ int zk_rope(void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh, void* k,
             int64_t Hq, int64_t Hkv, int64_t d, const float* cos,
             const float* sin, int64_t n_pos, const int64_t* positions,
             int pairing, int inverse, int dtype, zk_stream_t stream);
+/* The rotated copies q_out / k_out (contiguous [B, S, H, d]) of q and k, for
+ * positions 0 .. S-1: 2-byte types, d 64 or 128, strides multiples of 8
+ * elements, pointers 16-byte aligned. */
+int zk_rope_copy(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh, void* q_out,
+                 const void* k, int64_t k_sb, int64_t k_ss, int64_t k_sh, void* k_out,
+                 int64_t B, int64_t S, int64_t Hq, int64_t Hkv, int64_t d,
+                 const float* cos, const float* sin, int64_t n_pos, int pairing,
+                 int dtype, zk_stream_t stream);
 
 /* The q|k|v projection with the rotary embedding fused: c = a b^T (the
  * zk_gemm_nt product: a [M, K], b [N, K], c [M, N] with row strides lda /

@@ -98,6 +98,8 @@ SIGNATURES = {
                                 _i64, _i64, _i64, _int, _ptr]),
     "zk_gemm_rope": (_int, [_ptr, _i64, _ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i64,
                             _i64, _i64, _ptr, _ptr, _i64, _ptr, _int, _int, _ptr]),
+    "zk_rope_copy": (_int, [_ptr, _i64, _i64, _i64, _ptr, _ptr, _i64, _i64, _i64, _ptr, _i64,
+                            _i64, _i64, _i64, _i64, _ptr, _ptr, _i64, _int, _int, _ptr]),
     "zk_rope": (_int, [_ptr, _i64, _i64, _i64, _ptr, _i64, _i64, _i64, _i64,
                        _i64, _i64, _i64, _i64, _ptr, _ptr, _i64, _ptr, _int,
                        _int, _int, _ptr]),

@@ -113,9 +113,7 @@ class FlashAttentionFunction(torch.autograd.Function):
         B, S, Hq, d = q.shape
         if rope_theta is not None:
             cos, sin = rope_tables(S, d, rope_theta, q.dtype, q.device, interleaved)
-            q = q.contiguous().clone()
-            k = k.contiguous().clone()
-            K.rope_(q, k, cos, sin, interleaved=interleaved)
+            q, k = K.rope_copy(q, k, cos, sin, interleaved=interleaved)
         o, lse = K.attn_fwd(q, k, v, causal=causal, window=window, scale=scale)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.cfg = (causal, window, scale, rope_theta, interleaved)

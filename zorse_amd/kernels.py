@@ -472,6 +472,35 @@ def rope_(q: torch.Tensor, k: torch.Tensor | None, cos: torch.Tensor, sin: torch
                         int(inverse), dtype_code(q.dtype), stream_handle(dev)), "zk_rope")
 
 
+def rope_copy(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+              interleaved: bool = False):
+    """Rotated contiguous copies of q [B,S,Hq,d] and k [B,S,Hkv,d], positions
+    0 .. S-1: in one pass (zk_rope_copy) for head dims 64 and 128 of 2-byte
+    types with 16-byte aligned rows, else copies rotated in place."""
+    dev = _require_gpu(q, k, cos, sin)
+    if q.dim() == 4 and k.dim() == 4 and q.dtype in _LOWP and k.dtype == q.dtype:
+        B, S, Hq, d = q.shape
+        (qb, qs, qh, qu), (kb, ks, kh, ku) = q.stride(), k.stride()
+        if k.shape[:2] == (B, S) and k.shape[3] == d and d in (64, 128) and qu == ku == 1 \
+                and (qb | qs | qh | kb | ks | kh) % 8 == 0 \
+                and (q.data_ptr() | k.data_ptr() | cos.data_ptr() | sin.data_ptr()) % 16 == 0 \
+                and 0 < Hq and 0 < k.shape[2] and Hq + k.shape[2] < 65536 and B < 65536 \
+                and cos.shape == sin.shape == (cos.shape[0], d // 2) and cos.shape[0] >= S \
+                and cos.dtype == sin.dtype == torch.float32 \
+                and cos.is_contiguous() and sin.is_contiguous():
+            q_out = torch.empty(q.shape, device=dev, dtype=q.dtype)
+            k_out = torch.empty(k.shape, device=dev, dtype=q.dtype)
+            check(lib().zk_rope_copy(
+                ptr(q), qb, qs, qh, ptr(q_out), ptr(k), kb, ks, kh, ptr(k_out), B, S, Hq,
+                k.shape[2], d, ptr(cos), ptr(sin), cos.shape[0],
+                _abi.ZK_ROPE_INTERLEAVED if interleaved else _abi.ZK_ROPE_HALF,
+                dtype_code(q.dtype), stream_handle(dev)), "zk_rope_copy")
+            return q_out, k_out
+    q, k = q.contiguous().clone(), k.contiguous().clone()
+    rope_(q, k, cos, sin, interleaved=interleaved)
+    return q, k
+
+
 # -------------------------------------------------------------- Attention --
 
 def _attn_desc(q, k, v, o, scale, causal, window, dq=None, dk=None, dv=None):
