@@ -84,6 +84,7 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
   const Cost* c = a_km ? kKMajor : kAlongK;
   const int nc = a_km ? 3 : 6;
   const int64_t cus = device_cus(), steps = (K + gemm::BK - 1) / gemm::BK;
+  const int64_t tiles256 = gemm::tile_count(gemm::k256, M, N);
   gemm::Tile best = gemm::k256;
   double best_us = 0;
   for (int i = 0; i < nc; ++i) {
@@ -101,6 +102,16 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     // chain: the share of the chip it holds counts more than its own time
     // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone)
     if (a_km && n < cus) us *= 0.15 + 0.85 * static_cast<double>(n) / cus;
+    // and one of two rounds of 256 x 256 or more stays on those unless a smaller
+    // tile is clearly ahead: twice the operand reads and a stream of short
+    // workgroups slow the chain beside it.  5120 x 13824 x 2048: 495 us on 128 x
+    // 128 tiles and 501 on 256 x 256, but the input gradient beside it takes 429
+    // against 290; forward + backward of the 13B layer, 2048 tokens, 3745 / 3680
+    // us, of the 14336-wide grouped-query layer, 1527 tokens, 2382 / 2350.  Below
+    // two rounds the smaller tile's own time decides (1B grouped-query layer, 1024
+    // tokens, 680 against 705 us), as it does more than 8 % ahead (7B, 512 tokens,
+    // 908 against 925).
+    if (a_km && i > 0 && tiles256 >= 2 * cus) us *= 1.08;
     if (i == 0 || us < best_us) {
       best = c[i].t;
       best_us = us;
