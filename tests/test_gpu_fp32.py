@@ -95,3 +95,49 @@ def test_attention_fp32_masked_values_do_not_leak(dev):
     dq, _, _ = K.attn_bwd(q, k, v, o, do, lse, causal=True)
     sdq, _, _ = K.attn_bwd(*short[:3], so, short[3], slse, causal=True)
     assert_close(dq[:, :keep], sdq.double(), torch.float32, "dq")
+
+
+def _rows_reference(q, k, v, do, window):
+    """Causal attention and its gradients in float64 over the keys each query
+    sees, a row at a time, so that a hidden infinity or NaN never meets a zero
+    weight.  [S, d] each."""
+    S, scale = q.shape[0], q.shape[1] ** -0.5
+    o, (dq, dk, dv) = torch.zeros_like(q), (torch.zeros_like(t) for t in (q, k, v))
+    for i in range(S):
+        js = slice(max(0, i - window + 1) if window else 0, i + 1)
+        p = torch.softmax((k[js] @ q[i]) * scale, 0)
+        o[i] = p @ v[js]
+        ds = p * (v[js] @ do[i] - o[i] @ do[i]) * scale
+        dq[i] = ds @ k[js]
+        dk[js] += torch.outer(ds, q[i])
+        dv[js] += torch.outer(p, do[i])
+    return o, dq, dk, dv
+
+
+@pytest.mark.parametrize("window", [0, 9])
+@pytest.mark.parametrize("d", [64, 18])
+@pytest.mark.parametrize("kind", ["minus_inf_scores", "nan_key", "nan_query"])
+def test_attention_fp32_nonfinite_rows_stay_nonfinite(dev, kind, d, window):
+    """A query whose visible scores are all -inf, or one of them NaN, has no
+    softmax: its output is NaN, and so are the gradients that its weights reach
+    -- not zeros, which would hide it from the loss.  The NaNs are where the
+    float64 rows have them and the finite values are theirs."""
+    from zorse_amd import kernels as K
+    S = 40
+    q, k, v, do = (_randn((S, d), 30 + i, "cpu") for i in range(4))
+    if kind == "minus_inf_scores":
+        q, k[:6] = q.abs(), float("-inf")
+    elif kind == "nan_key":
+        k[7, 3] = float("nan")
+    else:
+        q[5, 2] = float("nan")
+    dev4 = [t.to(dev)[None, :, None] for t in (q, k, v, do)]
+    o, lse = K.attn_fwd(*dev4[:3], causal=True, window=window)
+    got = (o, *K.attn_bwd(*dev4[:3], o, dev4[3], lse, causal=True, window=window))
+    ref = _rows_reference(*(t.double() for t in (q, k, v, do)), window)
+    for name, g, r in zip(("o", "dq", "dk", "dv"), got, ref):
+        g = g[0, :, 0].double().cpu()
+        # an infinite weight times a gradient may be infinite or NaN
+        assert torch.equal(g.isfinite(), r.isfinite()), name
+        ok = r.isfinite()
+        assert_close(torch.where(ok, g, 0), torch.where(ok, r, 0), torch.float32, name)

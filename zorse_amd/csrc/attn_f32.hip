@@ -280,8 +280,9 @@ __global__ __launch_bounds__(256) void attn_fwd_f32(AttnArgs a, int64_t n_qt) {
   }
   l = group_sum(l);
   if (my_q >= a.Sq) return;
+  // no weight although keys are visible: every score is -inf or NaN, and so is O
   store_row<D, kVec>(static_cast<float*>(a.out) + b * a.o_sb + hq * a.o_sh + my_q * a.o_ss, o,
-                     l > 0.f ? 1.0f / l : 0.f, d);
+                     l > 0.f ? 1.0f / l : t0 < t1 ? NAN : 0.f, d);
   if (q4 == 0) a.lse_out[(b * a.Hq + hq) * a.Sq + my_q] = l > 0.f ? m + logf(l) : -INFINITY;
 }
 
@@ -316,8 +317,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_f32(AttnArgs a, int64_t n_qt)
     del = group_sum(del);
     if (in) {
       const int64_t i = (b * a.Hq + hq) * a.Sq + my_q;
-      lse = a.lse[i];
-      if (lse == -INFINITY) lse = INFINITY;  // an empty row: probabilities 0
+      lse = a.lse[i];  // -inf where O is NaN: the row's gradients are not finite either
       if (q4 == 0) {
         a.delta[i] = del;
         a.lse2[i] = lse;
