@@ -141,3 +141,65 @@ def test_attention_fp32_nonfinite_rows_stay_nonfinite(dev, kind, d, window):
         assert torch.equal(g.isfinite(), r.isfinite()), name
         ok = r.isfinite()
         assert_close(torch.where(ok, g, 0), torch.where(ok, r, 0), torch.float32, name)
+
+
+# S, d, aligned: one token, both sides of the row kernels' limits (S d of 128 at
+# 1024 heads, 512 at 4096 up to four tokens, two thirds of that unaligned), and
+# the padded element counts of each instance
+@pytest.mark.parametrize("S,d,heads,causal,window,rope", [
+    (1, 64, 1024, True, 0, False), (4, 32, 1024, True, 0, True), (5, 32, 1024, True, 0, False),
+    (8, 16, 1024, False, 0, False), (4, 128, 4096, True, 2, True), (3, 6, 1026, True, 0, True),
+    (2, 70, 4098, True, 0, True), (1, 126, 1024, True, 0, False), (7, 13, 1026, False, 0, False)])
+def test_attention_fp32_short_sequences(dev, S, d, heads, causal, window, rope):
+    """Many sequences of a few tokens: the row kernels, GQA of two heads each,
+    in the dimensions where a pass of one kind meets one of the other (the keys'
+    heads are half the queries')."""
+    from zorse_amd import kernels as K
+    from zorse_amd.functional import rope_tables
+    B, Hq, Hkv = heads // 2, 4, 2  # the keys' heads: `heads`; the queries': twice as many
+    print(f"short sequences S={S} d={d} heads={heads}", flush=True)
+    q, do = _randn((B, S, Hq, d), 40, "cpu"), _randn((B, S, Hq, d), 41, "cpu")
+    k, v = _randn((B, S, Hkv, d), 42, "cpu"), _randn((B, S, Hkv, d), 43, "cpu")
+    g = [t.to(dev) for t in (q, k, v)]
+    o, lse = K.attn_fwd(*g, causal=causal, window=window)
+    ro, rlse = O.attention(q.double(), k.double(), v.double(), causal, window)
+    assert_close(o, ro, torch.float32, "o")
+    assert_close(lse, rlse, torch.float32, "lse")
+    got = K.attn_bwd(*g, o, do.to(dev), lse, causal=causal, window=window)
+    ref = O.attention_bwd(q.double(), k.double(), v.double(), do.double(), causal, window)
+    big = [t.abs().max().item() for t in (do, v, q, k)]
+    floor = (d + 2) * 2.0 ** -24 * d * big[0] * big[1] * max(big[2:]) / d ** 0.5
+    for name, x, r in zip(("dq", "dk", "dv"), got, ref):
+        diff = (x.double().cpu() - r).abs().max().item()
+        assert diff <= 1e-4 * r.abs().max().item() + (floor if name != "dv" else 0), (name, diff)
+    if rope:  # the fused rotation is the rotation pass over the plain gradients
+        for inter in (False, True):
+            cos, sin = rope_tables(S, d, 1e4, torch.float32, dev, inter)
+            rot = K.attn_bwd(*g, o, do.to(dev), lse, causal=causal, window=window,
+                             rope=(cos, sin, None, inter))
+            want = [t.clone() for t in got]
+            K.rope_(want[0], want[1], cos, sin, interleaved=inter, inverse=True)
+            for x, r in zip(rot, want):
+                assert_close(x, r.double(), torch.float32, "rope")
+
+
+def test_attention_fp32_short_sequences_cost_their_rows(dev):
+    """Attention over 65536 sequences of one token takes less than 8 times as
+    long as over 4096 (12 us, the floor of a launch; 0.5 ms when every sequence
+    takes a workgroup of 64 rows)."""
+    from zorse_amd import kernels as K
+
+    def best(B):
+        x = _randn((B, 1, 1, 16), 50, dev)
+        K.attn_fwd(x, x, x)
+        times = []
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            for _ in range(10):
+                K.attn_fwd(x, x, x)
+            t1.record()
+            t1.synchronize()
+            times.append(t0.elapsed_time(t1))
+        return min(times)
+    assert best(65536) < 8 * best(4096)

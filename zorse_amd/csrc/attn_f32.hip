@@ -176,16 +176,17 @@ __device__ __forceinline__ void store_row(float* dst, const f32x4 (&x)[D / 16], 
 
 // The transpose of the RoPE rotation on one row of a tensor just stored
 // (gradients of queries / keys the forward rotated), by the 16-lane column's
-// four lanes after a barrier: pairs (i, i + d / 2) or (2 i, 2 i + 1), the
-// formula of rope_inverse_regs.
-__device__ __forceinline__ void rope_inverse_row(float* x, const AttnArgs& a, int64_t row, int q4) {
+// four lanes after a barrier (lanes first, first + step, ..): pairs
+// (i, i + d / 2) or (2 i, 2 i + 1), the formula of rope_inverse_regs.
+__device__ __forceinline__ void rope_inverse_row(float* x, const AttnArgs& a, int64_t row,
+                                                 int first, int step) {
   int64_t pos = a.rope_pos != nullptr ? a.rope_pos[row] : row;
   if (pos < 0) pos = 0;
   if (pos > a.rope_npos - 1) pos = a.rope_npos - 1;
   const int half = static_cast<int>(a.d / 2);
   const float* ct = a.rope_cos + pos * half;
   const float* st = a.rope_sin + pos * half;
-  for (int i = q4; i < half; i += 4) {
+  for (int i = first; i < half; i += step) {
     const int ia = a.rope_interleaved ? 2 * i : i;
     const int ib = a.rope_interleaved ? 2 * i + 1 : i + half;
     const float u = x[ia], w = x[ib];
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_f32(AttnArgs a, int64_t n_qt)
   if (in) store_row<D, kVec>(out, dq, a.scale, d);
   if (a.rope_cos != nullptr) {
     __syncthreads();  // the row's four lanes have stored it
-    if (in) rope_inverse_row(out, a, my_q, q4);
+    if (in) rope_inverse_row(out, a, my_q, q4, 4);
   }
 }
 
@@ -448,8 +449,176 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_f32(AttnArgs a) {
   }
   if (a.rope_cos != nullptr) {
     __syncthreads();
-    if (in) rope_inverse_row(dkp, a, my_k, q4);
+    if (in) rope_inverse_row(dkp, a, my_k, q4, 4);
   }
+}
+
+// ---- many sequences of a few tokens: one thread per row --------------------
+// The kernels above give each (batch, head) a workgroup of 64 rows, and with it
+// a workgroup's latency however few its rows are; here a thread walks its row's
+// keys (or its key's queries) by itself (by_rows below says when).
+
+// Elements 4 c .. 4 c + 3 of a row of d, zeros from d on.
+template <bool kVec>
+__device__ __forceinline__ float4 row4(const float* row, int c, int d) {
+  const float* p = row + 4 * c;
+  if (kVec) return *reinterpret_cast<const float4*>(p);
+  const int n = d - 4 * c;
+  return make_float4(p[0], n > 1 ? p[1] : 0.f, n > 2 ? p[2] : 0.f, n > 3 ? p[3] : 0.f);
+}
+template <int D, bool kVec>
+__device__ __forceinline__ float row_dot(const float* x, const float* y, int d) {
+  float s = 0.f;
+#pragma unroll
+  for (int c = 0; c < D / 4; ++c)
+    if (4 * c < d) {
+      const float4 u = row4<kVec>(x, c, d), w = row4<kVec>(y, c, d);
+      s = fmaf(u.x, w.x, s);
+      s = fmaf(u.y, w.y, s);
+      s = fmaf(u.z, w.z, s);
+      s = fmaf(u.w, w.w, s);
+    }
+  return s;
+}
+// acc = f acc + w x
+template <int D, bool kVec>
+__device__ __forceinline__ void row_add(float4 (&acc)[D / 4], float f, float w, const float* x,
+                                        int d) {
+#pragma unroll
+  for (int c = 0; c < D / 4; ++c)
+    if (4 * c < d) {
+      const float4 u = row4<kVec>(x, c, d);
+      acc[c] = make_float4(fmaf(acc[c].x, f, w * u.x), fmaf(acc[c].y, f, w * u.y),
+                           fmaf(acc[c].z, f, w * u.z), fmaf(acc[c].w, f, w * u.w));
+    }
+}
+template <int D, bool kVec>
+__device__ __forceinline__ void row_put(float* dst, const float4 (&x)[D / 4], float scale, int d) {
+#pragma unroll
+  for (int c = 0; c < D / 4; ++c)
+    if (4 * c < d) {
+      const float v[4] = {x[c].x * scale, x[c].y * scale, x[c].z * scale, x[c].w * scale};
+      float* p = dst + 4 * c;
+      if (kVec) {
+        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (4 * c + e < d) p[e] = v[e];
+      }
+    }
+}
+template <int D>
+__device__ __forceinline__ void row_zero(float4 (&x)[D / 4]) {
+#pragma unroll
+  for (int c = 0; c < D / 4; ++c) x[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+template <int D, bool kVec>
+__global__ __launch_bounds__(64) void attn_fwd_rows_f32(AttnArgs a) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  if (row >= a.B * a.Hq * a.Sq) return;
+  const int64_t qi = row % a.Sq, bh = row / a.Sq;
+  const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
+  const int d = static_cast<int>(a.d);
+  const float* Q = static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh + qi * a.q_ss;
+  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
+  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
+  float4 o[D / 4];
+  row_zero<D>(o);
+  float m = -INFINITY, l = 0.f;
+  for (int64_t j = 0; j < a.Skv; ++j) {
+    if (!attn_visible(qi, j, a.Skv, a.causal, a.window)) continue;
+    const float s = row_dot<D, kVec>(Q, K + j * a.k_ss, d) * a.scale;
+    const float m_new = fmaxf(m, s);
+    const float ref = m_new == -INFINITY ? 0.f : m_new;  // no weight yet
+    const float alpha = expf(m - ref), p = expf(s - ref);
+    l = l * alpha + p;
+    row_add<D, kVec>(o, alpha, p, V + j * a.v_ss, d);
+    m = m_new;
+  }
+  row_put<D, kVec>(static_cast<float*>(a.out) + b * a.o_sb + hq * a.o_sh + qi * a.o_ss, o,
+                   l > 0.f ? 1.0f / l : a.Skv > 0 ? NAN : 0.f, d);
+  a.lse_out[row] = l > 0.f ? m + logf(l) : -INFINITY;
+}
+
+template <int D, bool kVec>
+__global__ __launch_bounds__(64) void attn_bwd_dq_rows_f32(AttnArgs a) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  if (row >= a.B * a.Hq * a.Sq) return;
+  const int64_t qi = row % a.Sq, bh = row / a.Sq;
+  const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
+  const int d = static_cast<int>(a.d);
+  const int64_t orow = b * a.o_sb + hq * a.o_sh + qi * a.o_ss;
+  const float* Q = static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh + qi * a.q_ss;
+  const float* G = static_cast<const float*>(a.dout) + orow;
+  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh;
+  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh;
+  const float lse = a.lse[row], del = row_dot<D, kVec>(static_cast<const float*>(a.o) + orow, G, d);
+  a.lse2[row] = lse;
+  a.delta[row] = del;
+  float4 dq[D / 4];
+  row_zero<D>(dq);
+  for (int64_t j = 0; j < a.Skv; ++j) {
+    if (!attn_visible(qi, j, a.Skv, a.causal, a.window)) continue;
+    const float* k = K + j * a.k_ss;
+    const float p = expf(row_dot<D, kVec>(Q, k, d) * a.scale - lse);
+    row_add<D, kVec>(dq, 1.f, p * (row_dot<D, kVec>(G, V + j * a.v_ss, d) - del), k, d);
+  }
+  float* out = static_cast<float*>(a.dq) + b * a.dq_sb + hq * a.dq_sh + qi * a.dq_ss;
+  row_put<D, kVec>(out, dq, a.scale, d);
+  if (a.rope_cos != nullptr) rope_inverse_row(out, a, qi, 0, 1);
+}
+
+template <int D, bool kVec>
+__global__ __launch_bounds__(64) void attn_bwd_dkdv_rows_f32(AttnArgs a) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  if (row >= a.B * a.Hkv * a.Skv) return;
+  const int64_t kj = row % a.Skv, bh = row / a.Skv;
+  const int64_t b = bh / a.Hkv, hk = bh % a.Hkv, n_rep = a.Hq / a.Hkv;
+  const int d = static_cast<int>(a.d);
+  const float* K = static_cast<const float*>(a.k) + b * a.k_sb + hk * a.k_sh + kj * a.k_ss;
+  const float* V = static_cast<const float*>(a.v) + b * a.v_sb + hk * a.v_sh + kj * a.v_ss;
+  float4 dk[D / 4], dv[D / 4];
+  row_zero<D>(dk);
+  row_zero<D>(dv);
+  for (int64_t hq = hk * n_rep; hq < (hk + 1) * n_rep; ++hq) {
+    const float* Q = static_cast<const float*>(a.q) + b * a.q_sb + hq * a.q_sh;
+    const float* G = static_cast<const float*>(a.dout) + b * a.o_sb + hq * a.o_sh;
+    for (int64_t qi = 0; qi < a.Sq; ++qi) {
+      if (!attn_visible(qi, kj, a.Skv, a.causal, a.window)) continue;
+      const int64_t i = (b * a.Hq + hq) * a.Sq + qi;
+      const float* q = Q + qi * a.q_ss;
+      const float* g = G + qi * a.o_ss;
+      const float p = expf(row_dot<D, kVec>(q, K, d) * a.scale - a.lse2[i]);
+      row_add<D, kVec>(dv, 1.f, p, g, d);
+      row_add<D, kVec>(dk, 1.f, p * (row_dot<D, kVec>(g, V, d) - a.delta[i]), q, d);
+    }
+  }
+  float* dkp = static_cast<float*>(a.dk) + b * a.dk_sb + hk * a.dk_sh + kj * a.dk_ss;
+  row_put<D, kVec>(dkp, dk, a.scale, d);
+  row_put<D, kVec>(static_cast<float*>(a.dv) + b * a.dv_sb + hk * a.dv_sh + kj * a.dv_ss, dv, 1.f, d);
+  if (a.rope_cos != nullptr) rope_inverse_row(dkp, a, kj, 0, 1);
+}
+
+// Which kernels a pass takes, `heads` the (batch, head) pairs of its rows: a
+// workgroup costs its latency over the chip (8 ns forward and 24 backward once
+// there are 2048, 15 and 55 for head dims above 64), a row the walk over S keys of
+// d elements, never less than 12 us forward and 20 backward in all.  Measured, us
+// forward + backward, tiles / rows, at 1024, 2048 and 16384 heads:
+//   S 1, d 64     47 / 37     79 / 36     527 / 40
+//   S 8, d 16     46 / 39     78 / 40     544 / 73
+//   S 4, d 32     51 / 45     79 / 44     545 / 71
+//   S 4, d 64     47 / 67     81 / 68     549 / 135
+//   S 16, d 16    46 / 65     80 / 67     541 / 215
+//   S 4, d 128    84 / 126   156 / 128   1160 / 268
+//   S 32, d 16    50 / 122    84 / 130    575 / 744
+//   S 2, d 50     53 / 70     91 / 70     625 / 129   (not 16-byte aligned)
+// and 512 heads are even up to S d = 64, slower from there.
+bool by_rows(const AttnArgs& a, int64_t heads, bool vec) {
+  const int64_t S = a.Sq > a.Skv ? a.Sq : a.Skv;
+  const int64_t cost = vec ? S * a.d : S * a.d * 3 / 2;
+  return heads >= 1024 && cost <= heads / 8 && cost <= (S <= 4 ? 512 : 256);
 }
 
 // float4 accesses: head dim and strides multiples of 4, pointers of 16 bytes
@@ -477,9 +646,28 @@ bool vec4_ok(int64_t d, std::initializer_list<int64_t> strides,
       hipLaunchKernelGGL((KERNEL<128, false>), GRID, dim3(256), 0, s, __VA_ARGS__);          \
   } while (0)
 
+#define ZK_F32_ROWS(KERNEL, ROWS)                                                              \
+  do {                                                                                         \
+    const dim3 grid(static_cast<unsigned>(((ROWS) + 63) / 64));                                \
+    if (a.d <= 16) {                                                                           \
+      if (vec) hipLaunchKernelGGL((KERNEL<16, true>), grid, dim3(64), 0, s, a);                \
+      else hipLaunchKernelGGL((KERNEL<16, false>), grid, dim3(64), 0, s, a);                   \
+    } else if (a.d <= 64) {                                                                    \
+      if (vec) hipLaunchKernelGGL((KERNEL<64, true>), grid, dim3(64), 0, s, a);                \
+      else hipLaunchKernelGGL((KERNEL<64, false>), grid, dim3(64), 0, s, a);                   \
+    } else {                                                                                   \
+      if (vec) hipLaunchKernelGGL((KERNEL<128, true>), grid, dim3(64), 0, s, a);               \
+      else hipLaunchKernelGGL((KERNEL<128, false>), grid, dim3(64), 0, s, a);                  \
+    }                                                                                          \
+  } while (0)
+
 void launch_attn_fwd_f32(const AttnArgs& a, hipStream_t s) {
   const bool vec = vec4_ok(a.d, {a.q_sb, a.q_ss, a.q_sh, a.k_sb, a.k_ss, a.k_sh, a.v_sb, a.v_ss,
                                  a.v_sh, a.o_sb, a.o_ss, a.o_sh}, {a.q, a.k, a.v, a.out});
+  if (by_rows(a, a.B * a.Hq, vec)) {
+    ZK_F32_ROWS(attn_fwd_rows_f32, a.B * a.Hq * a.Sq);
+    return;
+  }
   const int64_t n_qt = (a.Sq + 63) / 64;
   const dim3 grid(static_cast<unsigned>(n_qt * a.B * a.Hq));
   ZK_F32_DISPATCH(attn_fwd_f32, grid, a, n_qt);
@@ -491,11 +679,15 @@ void launch_attn_bwd_f32(const AttnArgs& a, hipStream_t s) {
                                  a.dk_ss, a.dk_sh, a.dv_sb, a.dv_ss, a.dv_sh},
                            {a.q, a.k, a.v, a.o, a.dout, a.dq, a.dk, a.dv});
   const int64_t n_qt = (a.Sq + 63) / 64, n_kt = (a.Skv + 63) / 64;
-  if (n_qt > 0) {
+  if (n_qt > 0 && by_rows(a, a.B * a.Hq, vec)) {
+    ZK_F32_ROWS(attn_bwd_dq_rows_f32, a.B * a.Hq * a.Sq);
+  } else if (n_qt > 0) {
     const dim3 grid(static_cast<unsigned>(n_qt * a.B * a.Hq));
     ZK_F32_DISPATCH(attn_bwd_dq_f32, grid, a, n_qt);
   }
-  if (n_kt > 0) {
+  if (n_kt > 0 && by_rows(a, a.B * a.Hkv, vec)) {
+    ZK_F32_ROWS(attn_bwd_dkdv_rows_f32, a.B * a.Hkv * a.Skv);
+  } else if (n_kt > 0) {
     const dim3 grid(static_cast<unsigned>(n_kt * a.B * a.Hkv));
     ZK_F32_DISPATCH(attn_bwd_dkdv_f32, grid, a);
   }
