@@ -203,3 +203,30 @@ def test_attention_fp32_short_sequences_cost_their_rows(dev):
             times.append(t0.elapsed_time(t1))
         return min(times)
     assert best(65536) < 8 * best(4096)
+
+
+@pytest.mark.parametrize("S,d", [(1, 4), (5, 35)])
+def test_attention_fp32_more_workgroups_than_one_grid_dimension(dev, S, d):
+    """2^24 + 64 heads: 2^32 threads and more, past what one grid dimension of a
+    launch holds, for the row kernels and for the tiles.  Every head holds the
+    same values (expanded views) and gives the same bits."""
+    from zorse_amd import kernels as K
+    B, H = (1 << 18) + 1, 64
+    print(f"{B * H} heads of {S} x {d}", flush=True)
+    one = [_randn((1, S, 1, d), 60 + i, dev) for i in range(4)]
+    q, k, v, do = (t.expand(B, S, H, d) for t in one)
+    want, wlse = K.attn_fwd(*one[:3])
+    o, lse = K.attn_fwd(q, k, v)
+    assert torch.equal(o[:1, :, :1], o[-1:, :, -1:])
+    assert_close(o[:1, :, :1], want.double(), torch.float32, "o")
+    for t in o.split(1 << 14):
+        assert bool((t == o[:1, :, :1]).all())
+    del o
+    assert_close(lse[:1, :1], wlse.double(), torch.float32, "lse")
+    assert bool((lse == lse[:1, :1]).all())
+    grads = K.attn_bwd(q, k, v, want.expand(B, S, H, d), do, lse)
+    ref = K.attn_bwd(*one[:3], want, one[3], wlse)
+    for g, r in zip(grads, ref):
+        assert_close(g[:1, :, :1], r.double(), torch.float32, "gradient")
+        for t in g.split(1 << 14):
+            assert bool((t == g[:1, :, :1]).all())

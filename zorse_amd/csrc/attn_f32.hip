@@ -213,11 +213,24 @@ __device__ __forceinline__ void tile_range(const AttnArgs& a, int64_t r0, int64_
   hi = hi > lo * kTile ? (hi + kTile - 1) / kTile : lo;
 }
 
+// A launch holds fewer than 2^32 threads along x: workgroup n of any number is
+// (n % kGridX, n / kGridX), those past the last one leave at once.
+constexpr int64_t kGridX = int64_t(1) << 20;
+__device__ __forceinline__ int64_t group_id() {
+  return static_cast<int64_t>(blockIdx.y) * kGridX + blockIdx.x;
+}
+dim3 group_grid(int64_t n) {
+  return n <= kGridX ? dim3(static_cast<unsigned>(n))
+                     : dim3(static_cast<unsigned>(kGridX), static_cast<unsigned>((n + kGridX - 1) / kGridX));
+}
+
 template <int D, bool kVec>
 __global__ __launch_bounds__(256) void attn_fwd_f32(AttnArgs a, int64_t n_qt) {
   __shared__ __attribute__((aligned(16))) float Ks[kTile * (D + 4)], Vs[kTile * (D + 4)];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
-  const int64_t nbh = a.B * a.Hq, qt = n_qt - 1 - blockIdx.x / nbh, bh = blockIdx.x % nbh;
+  const int64_t bid = group_id(), nbh = a.B * a.Hq;
+  if (bid >= n_qt * nbh) return;
+  const int64_t qt = n_qt - 1 - bid / nbh, bh = bid % nbh;
   const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
   const int64_t q0 = qt * 64, my_q = q0 + 16 * wave + l16;
   const int d = static_cast<int>(a.d);
@@ -292,7 +305,9 @@ template <int D, bool kVec>
 __global__ __launch_bounds__(256) void attn_bwd_dq_f32(AttnArgs a, int64_t n_qt) {
   __shared__ __attribute__((aligned(16))) float Ks[kTile * (D + 4)], Vs[kTile * (D + 4)];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
-  const int64_t nbh = a.B * a.Hq, qt = n_qt - 1 - blockIdx.x / nbh, bh = blockIdx.x % nbh;
+  const int64_t bid = group_id(), nbh = a.B * a.Hq;
+  if (bid >= n_qt * nbh) return;
+  const int64_t qt = n_qt - 1 - bid / nbh, bh = bid % nbh;
   const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
   const int64_t q0 = qt * 64, my_q = q0 + 16 * wave + l16;
   const int d = static_cast<int>(a.d);
@@ -371,11 +386,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_f32(AttnArgs a, int64_t n_qt)
 // dK and dV of 64 keys per workgroup, summed over the query heads of the
 // group; after attn_bwd_dq_f32 (delta, lse2).
 template <int D, bool kVec>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_f32(AttnArgs a) {
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_f32(AttnArgs a, int64_t n_kt) {
   __shared__ __attribute__((aligned(16))) float Qs[kTile * (D + 4)], Gs[kTile * (D + 4)];
   __shared__ __attribute__((aligned(16))) float ls[kTile], ds[kTile];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
-  const int64_t nbh = a.B * a.Hkv, kt = blockIdx.x / nbh, bh = blockIdx.x % nbh;
+  const int64_t bid = group_id(), nbh = a.B * a.Hkv;
+  if (bid >= n_kt * nbh) return;
+  const int64_t kt = bid / nbh, bh = bid % nbh;
   const int64_t b = bh / a.Hkv, hk = bh % a.Hkv, n_rep = a.Hq / a.Hkv;
   const int64_t k0 = kt * 64, my_k = k0 + 16 * wave + l16;
   const int d = static_cast<int>(a.d);
@@ -516,7 +533,7 @@ __device__ __forceinline__ void row_zero(float4 (&x)[D / 4]) {
 
 template <int D, bool kVec>
 __global__ __launch_bounds__(64) void attn_fwd_rows_f32(AttnArgs a) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  const int64_t row = group_id() * 64 + threadIdx.x;
   if (row >= a.B * a.Hq * a.Sq) return;
   const int64_t qi = row % a.Sq, bh = row / a.Sq;
   const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
@@ -544,7 +561,7 @@ __global__ __launch_bounds__(64) void attn_fwd_rows_f32(AttnArgs a) {
 
 template <int D, bool kVec>
 __global__ __launch_bounds__(64) void attn_bwd_dq_rows_f32(AttnArgs a) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  const int64_t row = group_id() * 64 + threadIdx.x;
   if (row >= a.B * a.Hq * a.Sq) return;
   const int64_t qi = row % a.Sq, bh = row / a.Sq;
   const int64_t b = bh / a.Hq, hq = bh % a.Hq, hk = hq / (a.Hq / a.Hkv);
@@ -572,7 +589,7 @@ __global__ __launch_bounds__(64) void attn_bwd_dq_rows_f32(AttnArgs a) {
 
 template <int D, bool kVec>
 __global__ __launch_bounds__(64) void attn_bwd_dkdv_rows_f32(AttnArgs a) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  const int64_t row = group_id() * 64 + threadIdx.x;
   if (row >= a.B * a.Hkv * a.Skv) return;
   const int64_t kj = row % a.Skv, bh = row / a.Skv;
   const int64_t b = bh / a.Hkv, hk = bh % a.Hkv, n_rep = a.Hq / a.Hkv;
@@ -648,7 +665,7 @@ bool vec4_ok(int64_t d, std::initializer_list<int64_t> strides,
 
 #define ZK_F32_ROWS(KERNEL, ROWS)                                                              \
   do {                                                                                         \
-    const dim3 grid(static_cast<unsigned>(((ROWS) + 63) / 64));                                \
+    const dim3 grid = group_grid(((ROWS) + 63) / 64);                                          \
     if (a.d <= 16) {                                                                           \
       if (vec) hipLaunchKernelGGL((KERNEL<16, true>), grid, dim3(64), 0, s, a);                \
       else hipLaunchKernelGGL((KERNEL<16, false>), grid, dim3(64), 0, s, a);                   \
@@ -669,7 +686,7 @@ void launch_attn_fwd_f32(const AttnArgs& a, hipStream_t s) {
     return;
   }
   const int64_t n_qt = (a.Sq + 63) / 64;
-  const dim3 grid(static_cast<unsigned>(n_qt * a.B * a.Hq));
+  const dim3 grid = group_grid(n_qt * a.B * a.Hq);
   ZK_F32_DISPATCH(attn_fwd_f32, grid, a, n_qt);
 }
 
@@ -682,14 +699,14 @@ void launch_attn_bwd_f32(const AttnArgs& a, hipStream_t s) {
   if (n_qt > 0 && by_rows(a, a.B * a.Hq, vec)) {
     ZK_F32_ROWS(attn_bwd_dq_rows_f32, a.B * a.Hq * a.Sq);
   } else if (n_qt > 0) {
-    const dim3 grid(static_cast<unsigned>(n_qt * a.B * a.Hq));
+    const dim3 grid = group_grid(n_qt * a.B * a.Hq);
     ZK_F32_DISPATCH(attn_bwd_dq_f32, grid, a, n_qt);
   }
   if (n_kt > 0 && by_rows(a, a.B * a.Hkv, vec)) {
     ZK_F32_ROWS(attn_bwd_dkdv_rows_f32, a.B * a.Hkv * a.Skv);
   } else if (n_kt > 0) {
-    const dim3 grid(static_cast<unsigned>(n_kt * a.B * a.Hkv));
-    ZK_F32_DISPATCH(attn_bwd_dkdv_f32, grid, a);
+    const dim3 grid = group_grid(n_kt * a.B * a.Hkv);
+    ZK_F32_DISPATCH(attn_bwd_dkdv_f32, grid, a, n_kt);
   }
 }
 
