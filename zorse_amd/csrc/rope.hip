@@ -327,6 +327,12 @@ extern "C" int zk_rope(void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   bool pos2 = dtype != ZK_F32 && d % 4 == 0 && d <= 1024 && aligned(q, 4) &&
               (k == nullptr || aligned(k, 4)) && aligned(cos, 8) && aligned(sin, 8) &&
               S < 0x7fffffff && B < 65536;
+  // A workgroup a position costs 0.5 ns, whatever its heads give it to do: with
+  // less than a wavefront's work, H d / 4 < 64, the general pass is ahead.  us
+  // general / position-major, at 65536 positions: 1 head of 16 7 / 35, 4 of 48
+  // 25 / 35, 2 of 100 32 / 36, 16 of 16 37 / 35, 4 of 100 60 / 42; up to 8192
+  // positions either takes a launch's 7 us.
+  pos2 = pos2 && H * (d / 4) >= 64;
   pos2 = pos2 && q_sb % 2 == 0 && q_ss % 2 == 0 && q_sh % 2 == 0;
   if (k != nullptr) pos2 = pos2 && k_sb % 2 == 0 && k_ss % 2 == 0 && k_sh % 2 == 0;
   if (pos2) {
