@@ -49,3 +49,19 @@ def test_one_head_costs_less_than_sixteen(dev):
             times.append(t0.elapsed_time(t1))
         return min(times)
     assert best(1) < 0.7 * best(16)
+
+
+def test_more_positions_than_one_grid_dimension(dev):
+    """2^24 positions (2^32 threads of the position-major pass, past what a launch
+    holds) of 64 heads of 4: the general pass, every position's rotation."""
+    from zorse_amd import kernels as K
+    S, H, d = 1 << 24, 64, 4
+    print(f"rope {S} positions of {H} x {d}", flush=True)
+    base = torch.randn(1, 8, H, d, generator=torch.Generator().manual_seed(2)).bfloat16().to(dev)
+    cos, sin = _tables(8, d // 2, dev)
+    want = base.clone()
+    K.rope_(want, None, cos, sin)
+    q = base.expand(S // 8, 8, H, d).reshape(1, S, H, d)
+    K.rope_(q, None, cos, sin, positions=torch.arange(S, device=dev) % 8)
+    for part in q.view(S // 8, 8, H, d).split(1 << 17):
+        assert bool((part == want).all())

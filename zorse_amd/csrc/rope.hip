@@ -326,7 +326,7 @@ extern "C" int zk_rope(void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   // rows of d / 2 floats, an even number)
   bool pos2 = dtype != ZK_F32 && d % 4 == 0 && d <= 1024 && aligned(q, 4) &&
               (k == nullptr || aligned(k, 4)) && aligned(cos, 8) && aligned(sin, 8) &&
-              S < 0x7fffffff && B < 65536;
+              S < (int64_t(1) << 24) && B < 65536;  // 256 threads a position, below 2^32
   // A workgroup a position costs 0.5 ns, whatever its heads give it to do: with
   // less than a wavefront's work, H d / 4 < 64, the general pass is ahead.  us
   // general / position-major, at 65536 positions: 1 head of 16 7 / 35, 4 of 48
