@@ -197,6 +197,27 @@ int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t 
 enum zk_gemm_kernel { ZK_GEMM_GENERAL = 0, ZK_GEMM_TILED = 1 };
 int zk_gemm_path(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor, int64_t ldb,
                  int b_kmajor, int64_t ldc, int64_t ldr, int dtype);
+/* The kernel of a launch with 16-byte aligned pointers and no workspace
+ * (host-only; the device's CU count, 256 without a device): zk_gemm,
+ * zk_gemm_swiglu (ZK_TILE_GENERAL: the two products and the activation pass)
+ * and zk_gemm_rope (ZK_TILE_GENERAL: zk_gemm and the RoPE pass).  The _K2
+ * tiles have eight waves, four on each half of a K step. */
+enum zk_gemm_tile_id {
+  ZK_TILE_GENERAL = 0,
+  ZK_TILE_256 = 1,
+  ZK_TILE_256_MASKED = 2,
+  ZK_TILE_128X256 = 3,
+  ZK_TILE_128 = 4,
+  ZK_TILE_128_K2 = 5,
+  ZK_TILE_64 = 6,
+  ZK_TILE_64X128_K2 = 7
+};
+int zk_gemm_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor, int64_t ldb,
+                 int b_kmajor, int64_t ldc, int64_t ldr, int dtype);
+int zk_gemm_swiglu_tile(int64_t M, int64_t F, int64_t K, int64_t ld_x, int64_t ld_w,
+                        int64_t ld_gu, int dtype);
+int zk_gemm_rope_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                      int64_t S, int64_t rot_cols, int64_t head_dim, int64_t n_pos, int dtype);
 
 /* zk_gemm with both operands contiguous along the reduction (a [M, K],
  * b [N, K]): the nn.Linear forward x W^T of the projections above

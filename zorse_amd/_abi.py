@@ -88,6 +88,10 @@ SIGNATURES = {
     "zk_gemm_ws": (_int, [_ptr, _i64, _int, _ptr, _i64, _int, _ptr, _i64, _ptr, _i64, _i64, _i64,
                           _i64, _int, _ptr, _i64, _ptr]),
     "zk_gemm_path": (_int, [_i64, _i64, _i64, _i64, _int, _i64, _int, _i64, _i64, _int]),
+    "zk_gemm_tile": (_int, [_i64, _i64, _i64, _i64, _int, _i64, _int, _i64, _i64, _int]),
+    "zk_gemm_swiglu_tile": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
+    "zk_gemm_rope_tile": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                                 _int]),
     "zk_gemm_nt": (_int, [_ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _i64, _i64, _i64,
                           _int, _ptr]),
     "zk_gemm_swiglu": (_int, [_ptr, _i64, _ptr, _ptr, _i64, _ptr, _ptr, _i64, _ptr, _i64, _ptr,

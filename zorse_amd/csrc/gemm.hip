@@ -39,14 +39,14 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
   const int wide = dtype == ZK_F32 ? 1 : 0;
   const int64_t lim_a = int64_t(1) << ((a_km ? 24 : 22) - wide),
                 lim_b = int64_t(1) << ((b_km ? 24 : 22) - wide);
-  return lda < lim_a && ldb < lim_b &&
-         gemm::tile_count(gemm::k64, M, N) < 0x7fffffffLL;
+  return lda < lim_a && ldb < lim_b && gemm::tile_count(gemm::k64, M, N) < 0x7fffffffLL;
 }
 
 // The tile a 2-byte product runs on: the one with the least estimated time
-//   launch + (full rounds + part) (edge + steps * step),
+//   launch + (full rounds + part) max(edge + steps * step, least),
 // rounds of the tiles the CUs hold at once (cap workgroups each), `part` the
-// share of a round's time that a partly filled last round takes.  Constants
+// share of a round's time that a partly filled last round takes, `least` what
+// storing a round's tiles takes.  Constants
 // in us, fitted to 372 products timed on an MI355X in every tile (32 to 4095
 // tokens by the widths of the layers and heads from 1536 to 49152, forward,
 // input- and weight-gradient layouts, weights not in any cache): over those
@@ -69,13 +69,16 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
   struct Cost {
     gemm::Tile t;
     int per_cu;
-    double launch, edge, step, part;
+    double launch, edge, step, part, least = 0;
   };
-  static constexpr Cost kAlongK[] = {{gemm::k256, 1, 0.5, 9.5, 1.29, 0.82},
+  // least (and the four steps a masked 256 x 256 tile always runs): 3848 x 2744
+  // x 24 takes 14 us on 256 x 256 tiles, 9.6 on 128 x 128 and 17 on 64 x 64, where
+  // the steps alone make 11, 8 and 7; gate|up of 2048 x 13952 x 64 40 / 26 / 43
+  static constexpr Cost kAlongK[] = {{gemm::k256, 1, 0.5, 9.5, 1.29, 0.82, 14.5},
                                      {gemm::k128x256, 1, 0.5, 5.5, 0.745, 0.72},
-                                     {gemm::k128, 2, 4.7, 0.8, 0.926, 0.73},
+                                     {gemm::k128, 2, 4.7, 0.8, 0.926, 0.73, 3.6},
                                      {gemm::k128x2, 1, 0.0, 5.7, 0.59, 0.82},
-                                     {gemm::k64, 2, 4.4, 0.0, 0.48, 0.60},
+                                     {gemm::k64, 2, 4.4, 0.0, 0.48, 0.60, 2.3},
                                      {gemm::k64x128, 1, 0.0, 5.1, 0.45, 0.92}};
   static constexpr Cost kKMajor[] = {{gemm::k256, 1, 4.0, 10.4, 1.31, 0.73},
                                      {gemm::k128, 2, 4.0, 3.0, 0.79, 0.59},
@@ -97,7 +100,8 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     if (rem > 0)
       part = c[i].per_cu == 2 ? (rem <= cus ? c[i].part : 1.0)
                               : c[i].part + (1 - c[i].part) * static_cast<double>(rem) / cap;
-    double us = c[i].launch + (c[i].edge + steps * c[i].step) * (full + part);
+    const double round = c[i].edge + steps * c[i].step;
+    double us = c[i].launch + (round > c[i].least ? round : c[i].least) * (full + part);
     // a K-major A is a weight gradient, which runs beside the input-gradient
     // chain: the share of the chip it holds counts more than its own time
     // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone)
@@ -166,6 +170,60 @@ static Split pick_split(int64_t M, int64_t N, int64_t K, bool on_grid) {
   return best;
 }
 
+// Which kernel a launch with 16-byte aligned pointers and no workspace takes.
+struct Plan {
+  bool on_grid, mfma;  // mfma false: the general kernel
+  gemm::Tile tile;
+};
+static Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km, int64_t ldb, int b_km,
+                      int64_t ldc, int64_t ldr, int dtype) {
+  Plan p{tiled_takes(M, N, K, lda, a_km, ldb, b_km, ldc, ldr, dtype), false, gemm::k256};
+  p.mfma = p.on_grid || masked_takes(M, N, K, lda, a_km, ldb, b_km, ldc, ldr, dtype);
+  if (!p.mfma) return p;
+  if (dtype == ZK_F32)
+    p.tile = gemm::f32_tile(M, N);
+  else if (!(a_km && !b_km && p.on_grid))
+    p.tile = pick_tile(M, N, K, a_km, b_km, p.on_grid);
+  return p;
+}
+// gate|up with the SwiGLU epilogue: N = 2 F.
+static Plan plan_swiglu(int64_t M, int64_t N, int64_t K, int64_t ld_x, int64_t ld_w, int64_t ld_gu,
+                        int dtype) {
+  Plan p{tiled_takes(M, N, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype),
+         masked_takes(M, N, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype), gemm::k256};
+  if (p.mfma) p.tile = pick_tile(M, N, K, false, false, false);
+  return p;
+}
+// mfma: the product rotates in the epilogue.
+static Plan plan_rope(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                      int64_t S, int64_t rot_cols, int64_t head_dim, int64_t n_pos, int dtype) {
+  Plan p{tiled_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype), false, gemm::k256};
+  if (dtype == ZK_F32 || !masked_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype) ||
+      (head_dim != 64 && head_dim != 128) || S >= (int64_t(1) << 30) ||
+      n_pos >= (int64_t(1) << 24))
+    return p;
+  p.tile = pick_tile(M, N, K, false, false, p.on_grid);
+  // the 256-wide tile rotates whole 128-column blocks of sequences of at least
+  // 128 tokens; a 64-wide one holds heads of 64 only
+  if (p.tile == gemm::k256 || p.tile == gemm::k128x256)
+    p.mfma = rot_cols % 128 == 0 && S >= 128;
+  else
+    p.mfma = p.tile != gemm::k64 || head_dim == 64;
+  return p;
+}
+static int tile_id(const Plan& p) {
+  if (!p.mfma) return ZK_TILE_GENERAL;
+  switch (p.tile) {
+    case gemm::k256: return p.on_grid ? ZK_TILE_256 : ZK_TILE_256_MASKED;
+    case gemm::k128x256: return ZK_TILE_128X256;
+    case gemm::k128: return ZK_TILE_128;
+    case gemm::k128x2: return ZK_TILE_128_K2;
+    case gemm::k64: return ZK_TILE_64;
+    case gemm::k64x128: return ZK_TILE_64X128_K2;
+  }
+  return ZK_TILE_GENERAL;
+}
+
 }  // namespace zk
 
 using namespace zk;
@@ -182,6 +240,27 @@ extern "C" int zk_gemm_path(int64_t M, int64_t N, int64_t K, int64_t lda, int a_
                      dtype)
              ? ZK_GEMM_TILED
              : ZK_GEMM_GENERAL;
+}
+
+extern "C" int zk_gemm_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor, int64_t ldb,
+                            int b_kmajor, int64_t ldc, int64_t ldr, int dtype) {
+  ZK_REQUIRE(valid_dtype(dtype), ZK_EDTYPE, "zk_gemm_tile: bad dtype %d", dtype);
+  return tile_id(plan_gemm(M, N, K, lda, a_kmajor != 0, ldb, b_kmajor != 0, ldc, ldr < 0 ? 8 : ldr,
+                           dtype));
+}
+
+extern "C" int zk_gemm_swiglu_tile(int64_t M, int64_t F, int64_t K, int64_t ld_x, int64_t ld_w,
+                                   int64_t ld_gu, int dtype) {
+  ZK_REQUIRE(dtype == ZK_BF16 || dtype == ZK_F16, ZK_EDTYPE,
+             "zk_gemm_swiglu_tile: 2-byte dtypes only (got %d)", dtype);
+  return tile_id(plan_swiglu(M, 2 * F, K, ld_x, ld_w, ld_gu, dtype));
+}
+
+extern "C" int zk_gemm_rope_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                 int64_t ldc, int64_t S, int64_t rot_cols, int64_t head_dim,
+                                 int64_t n_pos, int dtype) {
+  ZK_REQUIRE(valid_dtype(dtype), ZK_EDTYPE, "zk_gemm_rope_tile: bad dtype %d", dtype);
+  return tile_id(plan_rope(M, N, K, lda, ldb, ldc, S, rot_cols, head_dim, n_pos, dtype));
 }
 
 namespace {
@@ -288,8 +367,8 @@ extern "C" int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* 
                  (r == nullptr || ldr < (int64_t(1) << 40)) && rows_a < (int64_t(1) << 40) &&
                  rows_b < (int64_t(1) << 40) && M < (int64_t(1) << 40),
              ZK_EINVAL, "zk_gemm: sizes out of range");
-  const bool on_grid = tiled_takes(M, N, K, lda, a_km, ldb, b_km, ldc, r ? ldr : 8, dtype);
-  bool mfma = on_grid || masked_takes(M, N, K, lda, a_km, ldb, b_km, ldc, r ? ldr : 8, dtype);
+  const Plan pl = plan_gemm(M, N, K, lda, a_km, ldb, b_km, ldc, r ? ldr : 8, dtype);
+  bool mfma = pl.mfma;
   for (const void* p : ptrs) mfma = mfma && (p == nullptr || aligned(p, 16));
   const int64_t nwg = ((M + gemm::GBM - 1) / gemm::GBM) * ((N + gemm::GBM - 1) / gemm::GBM);
   ZK_REQUIRE(nwg < 0x7fffffffLL, ZK_EINVAL, "zk_gemm: grid too large");
@@ -307,7 +386,7 @@ extern "C" int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* 
   ga.K = K;
   hipStream_t s = as_stream(stream);
   if (mfma && !a_km && dtype != ZK_F32 && workspace != nullptr && aligned(workspace, 16)) {
-    const Split sp = pick_split(M, N, K, on_grid);
+    const Split sp = pick_split(M, N, K, pl.on_grid);
     if (sp.parts > 0 && workspace_bytes >= sp.parts * M * N * 4) {
       gemm::GemmArgs part = ga;
       part.c = workspace;
@@ -321,8 +400,7 @@ extern "C" int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* 
   if (mfma && dtype == ZK_F32)
     gemm::launch_ring_f32(a_km, b_km, ga, s);
   else if (mfma)
-    launch_mfma<0>(dtype == ZK_BF16, a_km && !b_km && on_grid ? gemm::k256 : pick_tile(M, N, K, a_km, b_km, on_grid),
-                   on_grid, a_km, b_km, ga, s);
+    launch_mfma<0>(dtype == ZK_BF16, pl.tile, pl.on_grid, a_km, b_km, ga, s);
   else if (dtype == ZK_BF16)
     launch_general<bf16>(a_km, b_km, ga, s);
   else if (dtype == ZK_F16)
@@ -369,16 +447,9 @@ extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t l
   if (M == 0 || N == 0) return ZK_OK;
   ZK_REQUIRE(c != nullptr && (K == 0 || (a != nullptr && b != nullptr)), ZK_EINVAL,
              "zk_gemm_rope: null pointer");
-  const bool on_grid = tiled_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype);
-  bool epi = dtype != ZK_F32 && masked_takes(M, N, K, lda, 0, ldb, 0, ldc, 8, dtype) && aligned(a, 16) &&
-             aligned(b, 16) && aligned(c, 16) && (head_dim == 64 || head_dim == 128) &&
-             aligned(cos, 16) && aligned(sin, 16) && S < (int64_t(1) << 30) &&
-             n_pos < (int64_t(1) << 24);
-  const gemm::Tile tile = epi ? pick_tile(M, N, K, false, false, on_grid) : gemm::k256;
-  // the 256-wide tile rotates whole 128-column blocks of sequences of at least
-  // 128 tokens; a 64-wide one holds heads of 64 only
-  if (tile == gemm::k256 || tile == gemm::k128x256) epi = epi && rot_cols % 128 == 0 && S >= 128;
-  if (tile == gemm::k64) epi = epi && head_dim == 64;
+  const Plan pl = plan_rope(M, N, K, lda, ldb, ldc, S, rot_cols, head_dim, n_pos, dtype);
+  const bool epi = pl.mfma && aligned(a, 16) && aligned(b, 16) && aligned(c, 16) &&
+                   aligned(cos, 16) && aligned(sin, 16);
   if (!epi) {
     const int rc = zk_gemm(a, lda, 0, b, ldb, 0, c, ldc, nullptr, 0, M, N, K, dtype, stream);
     if (rc != ZK_OK || rot_cols == 0) return rc;
@@ -404,7 +475,7 @@ extern "C" int zk_gemm_rope(const void* a, int64_t lda, const void* b, int64_t l
   ga.rcols = rot_cols;
   ga.rhalf = static_cast<int>(head_dim / 2);
   ga.rpair = pairing;
-  launch_mfma<2>(dtype == ZK_BF16, tile, on_grid, 0, 0, ga, as_stream(stream));
+  launch_mfma<2>(dtype == ZK_BF16, pl.tile, pl.on_grid, 0, 0, ga, as_stream(stream));
   return launch_status("zk_gemm_rope");
 }
 
@@ -440,7 +511,8 @@ extern "C" int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
              "zk_gemm_swiglu: leading dimension out of range");
   ZK_REQUIRE(((M + 127) / 128) * ((F + 63) / 64) < 0x7fffffffLL, ZK_EINVAL,
              "zk_gemm_swiglu: grid too large");
-  if (!masked_takes(M, 2 * F, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype)) {
+  const Plan pl = plan_swiglu(M, 2 * F, K, ld_x, ld_w, ld_gu, dtype);
+  if (!pl.mfma) {
     // rows too far apart for a tile's buffer resource: the two products and the
     // activation as separate launches
     int rc = zk_gemm(x, ld_x, 0, w_gate, ld_w, 0, g_out, ld_gu, nullptr, 0, M, F, K, dtype, stream);
@@ -466,8 +538,6 @@ extern "C" int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
   ga.M = M;
   ga.N = 2 * F;
   ga.K = K;
-  const bool on_grid = tiled_takes(M, 2 * F, K, ld_x, 0, ld_w, 0, ld_gu, 8, dtype);
-  launch_mfma<1>(dtype == ZK_BF16, pick_tile(M, 2 * F, K, false, false, false), on_grid, 0, 0, ga,
-                 as_stream(stream));
+  launch_mfma<1>(dtype == ZK_BF16, pl.tile, pl.on_grid, 0, 0, ga, as_stream(stream));
   return launch_status("zk_gemm_swiglu");
 }

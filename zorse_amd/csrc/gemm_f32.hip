@@ -17,9 +17,8 @@ void launch_t(bool small, const GemmArgs& ga, hipStream_t s) {
 }
 }  // namespace
 
-// 128 x 128 tiles where they fill the CUs, else 64 x 64.
 void launch_ring_f32(bool a_kmajor, bool b_kmajor, const GemmArgs& ga, hipStream_t s) {
-  const bool small = tile_count(k128, ga.M, ga.N) < device_cus();
+  const bool small = f32_tile(ga.M, ga.N) == k64;
   if (!a_kmajor && !b_kmajor)
     launch_t<false, false>(small, ga, s);
   else if (!a_kmajor)

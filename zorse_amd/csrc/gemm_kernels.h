@@ -913,7 +913,10 @@ void launch_ring_kmajor(bool bf16, bool a_kmajor, bool b_kmajor, Tile t, const G
 // k256, k128x2 and k64x128 (gemm_split.hip).
 void launch_split(bool bf16, bool b_kmajor, Tile t, int parts, const GemmArgs& ga, hipStream_t s);
 void launch_split_sum(bool bf16, const float* ws, int parts, const GemmArgs& out, hipStream_t s);
-// fp32 (gemm_f32.hip)
+// fp32 (gemm_f32.hip): 128 x 128 tiles where they fill the CUs, else 64 x 64
+inline Tile f32_tile(int64_t M, int64_t N) {
+  return tile_count(k128, M, N) < device_cus() ? k64 : k128;
+}
 void launch_ring_f32(bool a_kmajor, bool b_kmajor, const GemmArgs& ga, hipStream_t s);
 
 }  // namespace gemm
