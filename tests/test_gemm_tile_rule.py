@@ -35,3 +35,11 @@ def test_few_k_steps_count_their_stores(lib, M, N, K, b_km):
 def test_few_k_steps_gate_up(lib, M, F, K):
     """The same of gate|up, three outputs: 64 x 64 tiles 1.2 to 1.6 times the time."""
     assert lib.zk_gemm_swiglu_tile(M, F, K, K, K, 2 * F, BF16) == T128
+
+
+@pytest.mark.parametrize("M,N,K,tile", [((1 << 30) - 64, 8, 8, T128), (1 << 30, 8, 8, GENERAL),
+                                        (8, (1 << 30) + 8, 16, GENERAL), (1 << 29, 72, 8, GENERAL)])
+def test_masked_tiles_fit_one_grid_dimension(lib, M, N, K, tile):
+    """A launch holds fewer than 2^32 threads along its grid, 2^24 tiles of 256:
+    products of as many 64 x 64 tiles keep to the general kernel's larger ones."""
+    assert _tile(lib, M, N, K) == tile

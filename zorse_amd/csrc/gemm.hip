@@ -9,6 +9,11 @@
 
 namespace zk {
 
+// A launch's grid dimension holds fewer than 2^32 threads, a tile has 256 (the
+// 512-thread ones run at most one per CU): products of more 64 x 64 tiles stay
+// on the general kernel's 128 x 128.
+static constexpr int64_t kMaxTiles = int64_t(1) << 24;
+
 // Whether the 256 x 256 pipeline takes a launch: 2-byte type, M and N
 // multiples of 256, K a multiple of 128 and at least 256, leading dimensions
 // multiples of 8 (16-byte tile rows and stores), and every tile of an operand
@@ -39,7 +44,7 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
   const int wide = dtype == ZK_F32 ? 1 : 0;
   const int64_t lim_a = int64_t(1) << ((a_km ? 24 : 22) - wide),
                 lim_b = int64_t(1) << ((b_km ? 24 : 22) - wide);
-  return lda < lim_a && ldb < lim_b && gemm::tile_count(gemm::k64, M, N) < 0x7fffffffLL;
+  return lda < lim_a && ldb < lim_b && gemm::tile_count(gemm::k64, M, N) < kMaxTiles;
 }
 
 // The tile a 2-byte product runs on: the one with the least estimated time
