@@ -13,9 +13,10 @@
 // One workgroup per row; each thread covers 8 consecutive columns per access
 // (16-byte accesses for 2-byte types; the forward has four in flight and takes
 // one rescale for the 32 values) and the row reductions use wave shuffles plus
-// one LDS exchange.  Both passes are bound by HBM: 2046 rows of 49152 bf16
-// columns (201 MB) take 42 us forward, 58 with one access in flight and the
-// IEEE exp, and 66 us backward (402 MB).
+// one LDS exchange.  Both passes are bound by HBM: 4096 rows of 49152 bf16
+// columns (403 MB) take 81 us forward with exp_neg, 103 with expf and 107 with
+// one access in flight besides, 76 with exp_neg's first line alone; 2046 rows
+// 66 us backward (402 MB).
 //
 // zk_ce_labels and zk_ce_finish are what precedes and follows the chunks, one
 // workgroup each: checked row labels, the number of valid rows and the initial
@@ -25,6 +26,21 @@
 #include "vec.h"
 
 namespace zk {
+
+// e^x for x <= 0 (0 for -inf, NaN for NaN): 2^p, p = x log2(e) rounded, times
+// 1 + r for what the rounding left out, r = x - p ln(2).  Without r it is off by
+// |p| 2^-25, several ulps at x = -10.  expf, which reduces p to its fraction and
+// scales back, takes twice the instructions.  Largest and rms error of a sum
+// dominated by e^-5.6 to e^-8: 9.3e-8 and 3.1e-8, with expf 8.8e-8 and 3.0e-8,
+// without r 3.1e-7 and 1.0e-7 (of one sign on average).  r is kept in [-1, 1] so
+// that 0 times it stays 0 where p is -inf.
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.693147180559945309f;
+  constexpr float kLn2Lo = static_cast<float>(0.693147180559945309 - kLn2);
+  const float p = x * kLog2e, w = __builtin_amdgcn_exp2f(p);
+  const float r = fmaf(-p, kLn2Lo, fmaf(-p, kLn2, x));
+  return fmaf(w, __builtin_amdgcn_fmed3f(r, -1.0f, 1.0f), w);
+}
 
 template <int NT>
 __device__ __forceinline__ void block_max_sum(float& m, float& s, float* red) {
@@ -67,7 +83,6 @@ __global__ __launch_bounds__(NT) void ce_fwd_chunk(const T* __restrict__ logits,
   float m = -INFINITY, s = 0.f;
   if (vec) {
     constexpr int U = 4;
-    constexpr float kLog2e = 1.4426950408889634f;
     for (int64_t c = threadIdx.x * 8; c < cols; c += U * NT * 8) {
       float v[U][8];
 #pragma unroll
@@ -85,11 +100,11 @@ __global__ __launch_bounds__(NT) void ce_fwd_chunk(const T* __restrict__ logits,
 #pragma unroll
         for (int i = 0; i < 8; ++i) nm = fmaxf(nm, v[u][i]);
       if (nm == -INFINITY) continue;  // nothing but -inf so far
-      float acc = m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - nm) * kLog2e);
+      float acc = m == -INFINITY ? 0.f : s * exp_neg(m - nm);
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc += __builtin_amdgcn_exp2f((v[u][i] - nm) * kLog2e);
+        for (int i = 0; i < 8; ++i) acc += exp_neg(v[u][i] - nm);
       s = acc;
       m = nm;
     }
