@@ -52,3 +52,19 @@ def test_minus_infinity_logits(dev):
     LH._fwd_chunk(logits, torch.tensor([8201, -1], device=dev), 0, m, s, t)
     assert torch.equal(m, torch.ones_like(m)) and torch.allclose(s, torch.full_like(s, 8.0))
     assert t.tolist() == [1.0, 0.0]
+
+
+@pytest.mark.parametrize("bad", [4096, -1])
+def test_bad_labels_are_refused_before_any_product(dev, bad):
+    """A label out of range raises with no logits (67 MB here) allocated."""
+    from zorse_amd.lm_head import lm_head_cross_entropy
+    T, V = 4096, 4096
+    x, w = torch.randn(T, 64, device=dev), torch.randn(V, 64, device=dev)
+    labels = torch.zeros(T, dtype=torch.int64, device=dev)
+    labels[T - 1] = bad
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    with pytest.raises(ValueError, match="labels must lie in"):
+        lm_head_cross_entropy(x, w, labels)
+    assert torch.cuda.max_memory_allocated() - before < 1 << 20

@@ -21,8 +21,10 @@
 // zk_ce_labels and zk_ce_finish are what precedes and follows the chunks, one
 // workgroup each: checked row labels, the number of valid rows and the initial
 // accumulators; the rows' log-sum-exp and the mean loss.  As tensor operations
-// they were 30 launches of 2 to 5 us and two waits of the host for the device
-// (a head of 2046 tokens, 1536 wide, 49152 columns: 1098 us, 952 so).
+// they were 30 launches of 2 to 5 us and two waits of the host for the device (a
+// head of 2046 tokens, 1536 wide, 49152 columns: 1098 us against 931).  One wait
+// is left, for the label check before any logits are allocated; with the check
+// read after the products the same head took 910.
 #include "vec.h"
 
 namespace zk {

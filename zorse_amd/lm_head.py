@@ -61,7 +61,7 @@ class LMHeadCrossEntropyFunction(torch.autograd.Function):
         dev, given = x.device, labels.contiguous()
         # row labels (-1: ignored, skipped by the kernels), running max, sum and
         # label logit; stats = (labelled rows, labels out of range), which the
-        # host reads after the chunks are enqueued, without waiting for them
+        # host reads before any logits are allocated
         labels = torch.empty_like(given)
         run_max, run_sum, target, lse = torch.empty(4, T, device=dev, dtype=torch.float32)
         stats = torch.empty(2, device=dev, dtype=torch.int64)
@@ -72,18 +72,16 @@ class LMHeadCrossEntropyFunction(torch.autograd.Function):
                                  stream_handle(dev)), "zk_ce_labels")
         checked = torch.cuda.Event()
         checked.record(torch.cuda.current_stream(dev))
-        try:
-            for c0 in range(0, V, chunk):
-                logits = K.gemm(x, w[c0:c0 + chunk])
-                _fwd_chunk(logits, labels, c0, run_max, run_sum, target)
-            check(lib().zk_ce_finish(ptr(labels), T, ptr(run_max), ptr(run_sum), ptr(target),
-                                     ptr(stats), ptr(lse), ptr(loss), stream_handle(dev)),
-                  "zk_ce_finish")
-        finally:  # the kernel writes host memory: it outlives that
-            checked.synchronize()
+        checked.synchronize()
         if int(host[1]):
             raise ValueError(f"labels must lie in [0, {V}) or equal ignore_index "
                              f"({ignore_index})")
+        for c0 in range(0, V, chunk):
+            logits = K.gemm(x, w[c0:c0 + chunk])
+            _fwd_chunk(logits, labels, c0, run_max, run_sum, target)
+        check(lib().zk_ce_finish(ptr(labels), T, ptr(run_max), ptr(run_sum), ptr(target),
+                                 ptr(stats), ptr(lse), ptr(loss), stream_handle(dev)),
+              "zk_ce_finish")
         ctx.save_for_backward(x, w, labels, lse, stats)
         ctx.chunk = chunk
         ctx.weight_dtype = weight.dtype
