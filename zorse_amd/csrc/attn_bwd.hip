@@ -344,18 +344,20 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv(AttnArgs a) {
         }
       }
   }
-  if (a.dk_t != nullptr) {
-    // dK^T / dV^T rows hk D .. +D-1, token columns b Skv + k0 ..; the V rows'
-    // LDS (128 x D elements) holds the tile once every wave is past its last step
-    __syncthreads();
-    const int64_t left = a.Skv - k0;
-    const int nc = static_cast<int>(left < BK ? left : BK);
-    const int64_t off = hk * hd * a.t_ld + b * a.Skv + k0;
-    T* tile = &Vw[0][0];  // all D rows in one array (the other pointers are unused)
-    store_rows_transposed<T, D, BK, D, KR>(dk, a.scale, tile, tile, tile, tile,
-                                       static_cast<T*>(a.dk_t) + off, a.t_ld, nc, hd);
-    store_rows_transposed<T, D, BK, D, KR>(dv, 1.f, tile, tile, tile, tile,
-                                       static_cast<T*>(a.dv_t) + off, a.t_ld, nc, hd);
+  if constexpr (KR == 0) {
+    if (a.dk_t != nullptr) {
+      // dK^T / dV^T rows hk D .. +D-1, token columns b Skv + k0 ..; the V rows'
+      // LDS (128 x D elements) holds the tile once every wave is past its last step
+      __syncthreads();
+      const int64_t left = a.Skv - k0;
+      const int nc = static_cast<int>(left < BK ? left : BK);
+      const int64_t off = hk * D * a.t_ld + b * a.Skv + k0;
+      T* tile = &Vw[0][0];  // all D rows in one array (the other pointers are unused)
+      store_rows_transposed<T, D, BK, D>(dk, a.scale, tile, tile, tile, tile,
+                                         static_cast<T*>(a.dk_t) + off, a.t_ld, nc);
+      store_rows_transposed<T, D, BK, D>(dv, 1.f, tile, tile, tile, tile,
+                                         static_cast<T*>(a.dv_t) + off, a.t_ld, nc);
+    }
   }
 }
 
@@ -616,14 +618,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq(AttnArgs a, int64_t n_qt) 
           *reinterpret_cast<T4*>(dqp + d0) = w;
       }
   }
-  if (a.dq_t != nullptr) {
-    // dQ^T rows hq D .. +D-1, token columns b Sq + q0 ..; the K / V stages
-    // hold the tile once every wave is past its last step
-    __syncthreads();
-    const int64_t left = a.Sq - q0;
-    store_rows_transposed<T, D, BM, BN * D / BM, KR>(
-        dq, a.scale, K0, K1, V0, V1, static_cast<T*>(a.dq_t) + hq * hd * a.t_ld + b * a.Sq + q0,
-        a.t_ld, static_cast<int>(left < BM ? left : BM), hd);
+  if constexpr (KR == 0) {
+    if (a.dq_t != nullptr) {
+      // dQ^T rows hq D .. +D-1, token columns b Sq + q0 ..; the K / V stages
+      // hold the tile once every wave is past its last step
+      __syncthreads();
+      const int64_t left = a.Sq - q0;
+      store_rows_transposed<T, D, BM, BN * D / BM>(
+          dq, a.scale, K0, K1, V0, V1, static_cast<T*>(a.dq_t) + hq * D * a.t_ld + b * a.Sq + q0,
+          a.t_ld, static_cast<int>(left < BM ? left : BM));
+    }
   }
 }
 

@@ -65,13 +65,11 @@ void launch_attn_bwd_f32(const AttnArgs& a, hipStream_t s);
 // values pass through an LDS tile [D][NCOL] held by up to four arrays the
 // caller no longer needs, RP feature rows each (p0 first); every wave must be
 // done with them on entry.  16-byte stores, NCOL / 8 lanes per feature row.
-// Ends with a barrier, so the arrays may be reused at once.  NB: the 32-row
-// blocks x holds; KR > 0 (a ragged head dim): only the first `d` feature rows
-// are stored.
-template <typename T, int D, int NCOL, int RP, int KR, int NB>
-__device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[NB], float scale,
+// Ends with a barrier, so the arrays may be reused at once.
+template <typename T, int D, int NCOL, int RP>
+__device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[D / 32], float scale,
                                                       T* p0, T* p1, T* p2, T* p3, T* dst,
-                                                      int64_t ld, int ncols, int d) {
+                                                      int64_t ld, int ncols) {
   static_assert(RP % 32 == 0 && D <= 4 * RP, "feature rows per array");
   constexpr int NT = 2 * NCOL;  // threads: 64 per 32 columns
   const int tid = threadIdx.x, l32 = tid & 31, g = (tid >> 5) & 1, wave = tid >> 6;
@@ -81,7 +79,7 @@ __device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[NB], flo
     return p + (r % RP) * NCOL;
   };
 #pragma unroll
-  for (int nt = 0; nt < NB; ++nt)
+  for (int nt = 0; nt < D / 32; ++nt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const int r = 32 * nt + 8 * (j >> 2) + 4 * g + (j & 3);
@@ -91,10 +89,10 @@ __device__ __forceinline__ void store_rows_transposed(const f32x16 (&x)[NB], flo
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   constexpr int CPR = NCOL / 8;  // 16-byte chunks per feature row
 #pragma unroll
-  for (int i = 0; i < 32 * NB * CPR / NT; ++i) {
+  for (int i = 0; i < D * CPR / NT; ++i) {
     const int id = NT * i + tid;
     const int r = id / CPR, col = 8 * (id % CPR);
-    if (col < ncols && (KR == 0 || r < d))
+    if (col < ncols)
       *reinterpret_cast<u32x4*>(dst + r * ld + col) = *reinterpret_cast<const u32x4*>(row_ptr(r) + col);
   }
   __syncthreads();

@@ -63,6 +63,18 @@ __device__ __forceinline__ float fast_exp2(float x) {
 // log2-domain growth of the running maximum tolerated before rescaling
 static constexpr float kRescaleThreshold = 8.0f;
 
+// x s rounded to T.  For fp16 the compiler makes one rounding of a product and
+// its conversion (v_fma_mix) where the result has two uses, as in the kernels
+// that also store transposed, and two roundings where pairs of results are only
+// packed (v_cvt_pk_f16_f32); a result of its own (KR != 0) keeps the first form,
+// so that a ragged head has a padded one's bits.
+template <typename T, int KR>
+__device__ __forceinline__ T scaled(float x, float s) {
+  T t = static_cast<T>(x * s);
+  if constexpr (KR != 0 && std::is_same_v<T, f16>) asm("" : "+v"(t));
+  return t;
+}
+
 // kFull: Skv is a multiple of the key tile, so no tile runs past the end.
 // KR: 0 for a head dim of D; else the head dim a.d is an even number in
 // (16 KR - 16, 16 KR], and the tile's columns from a.d on hold nothing: KR of
@@ -282,7 +294,7 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
 #pragma unroll
   for (int nt = 0; nt < NB; ++nt)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) o[nt][j] = to_f32(static_cast<T>(o[nt][j] * inv));
+    for (int j = 0; j < 16; ++j) o[nt][j] = to_f32(scaled<T, KR>(o[nt][j], inv));
   if (my_q < a.Sq) {
     T* Op = static_cast<T*>(a.out) + b * a.o_sb + hq * a.o_sh + my_q * a.o_ss;
 #pragma unroll
@@ -303,15 +315,17 @@ void attn_fwd_kernel(AttnArgs a, int64_t n_qt) {
       a.lse_out[(b * a.Hq + hq) * a.Sq + my_q] =
           l_tot > 0.f ? m_ref * a.scale + logf(l_tot) : -INFINITY;
   }
-  if (a.o_t != nullptr) {
-    // O^T rows hq D .. +D-1, token columns b Sq + q0 ..: the same rounded
-    // values as the row store, through an LDS tile in the K / V stages (free
-    // once every wave is past its last step)
-    __syncthreads();
-    const int64_t left = a.Sq - q0;
-    store_rows_transposed<T, D, BM, BN * D / BM, KR>(
-        o, 1.f, K0, K1, V0, V1, static_cast<T*>(a.o_t) + hq * hd * a.t_ld + b * a.Sq + q0, a.t_ld,
-        static_cast<int>(left < BM ? left : BM), hd);
+  if constexpr (KR == 0) {
+    if (a.o_t != nullptr) {
+      // O^T rows hq D .. +D-1, token columns b Sq + q0 ..: the same rounded
+      // values as the row store, through an LDS tile in the K / V stages (free
+      // once every wave is past its last step)
+      __syncthreads();
+      const int64_t left = a.Sq - q0;
+      store_rows_transposed<T, D, BM, BN * D / BM>(
+          o, 1.f, K0, K1, V0, V1, static_cast<T*>(a.o_t) + hq * D * a.t_ld + b * a.Sq + q0,
+          a.t_ld, static_cast<int>(left < BM ? left : BM));
+    }
   }
 }
 
