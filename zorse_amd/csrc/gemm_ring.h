@@ -65,9 +65,6 @@ struct RingTile {
   uint32_t lane_off;  // bytes from the tile's first element
   int kcol;           // NT: this lane's first k of the tile
   int wave_by;        // LDS bytes before this wave's first instruction
-  // FOLD: an NT tile whose one instruction loads rows 0 .. 31 of two sources
-  // (waves 0 - 3 and 4 - 7)
-  template <bool FOLD = false>
   __device__ __forceinline__ void init(int64_t ld) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -83,7 +80,7 @@ struct RingTile {
     } else {
       const int row = tid >> 3;
       const int c = (tid & 7) ^ nt_sw(row);
-      lane_off = static_cast<uint32_t>((FOLD ? row & 31 : row) * ld * ES + c * 16);
+      lane_off = static_cast<uint32_t>(row * ld * ES + c * 16);
       kcol = c * (16 / ES);
       wave_by = w * 1024;
     }
@@ -208,9 +205,8 @@ void gemm_ring_kernel(GemmArgs args) {
   TA ta;
   TB tb;
   ta.init(lda);
-  constexpr bool kFold = EPI == 1 && TB::NI == 1;  // one instruction: gate and up rows
-  tb.template init<kFold>(ldb);
-  const bool up_wave = __builtin_amdgcn_readfirstlane(wave) >= 4;
+  static_assert(EPI != 1 || TB::NI % 2 == 0, "gate and up rows are loaded by instructions of their own");
+  tb.init(ldb);
   const uint32_t lds_a = lds_addr(As), lds_b = lds_addr(Bs);
   f32x4 acc[MB][NB];
 #pragma unroll
@@ -275,7 +271,6 @@ void gemm_ring_kernel(GemmArgs args) {
     Src s;
     s.r = rsrc_left(Bb + k * b_step, b_left - k * b_step);
     if constexpr (EPI == 1) s.r2 = rsrc_left(B2b + k * b_step, b_left - k * b_step);
-    if constexpr (kFold) s.r = up_wave ? s.r2 : s.r;
     s.voff = BKM || k * BK + tb.kcol < K ? tb.lane_off : 0x80000000u;
     return s;
   };
@@ -283,7 +278,7 @@ void gemm_ring_kernel(GemmArgs args) {
     ta.issue(lds_a + st * (ES * TA::EL), s.r, s.voff, lda, i);
   };
   auto load_b = [&](const Src& s, int st, int i) __attribute__((always_inline)) {
-    if constexpr (EPI == 1 && !kFold) {
+    if constexpr (EPI == 1) {
       // pieces of the first half: gate rows 32 i .., of the second: up rows
       if (i < TB::NI / 2)
         tb.issue(lds_b + st * (ES * TB::EL), s.r, s.voff, ldb, i);
