@@ -48,9 +48,9 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
 }
 
 // The tile a 2-byte product runs on: the one with the least estimated time
-//   launch + (full rounds + part) max(edge + steps * step, least),
+//   launch + max((full rounds + part) (edge + steps * step), rounds * store),
 // rounds of the tiles the CUs hold at once (cap workgroups each), `part` the
-// share of a round's time that a partly filled last round takes, `least` what
+// share of a round's time that a partly filled last round takes, `store` what
 // storing a round's tiles takes.  Constants
 // in us, fitted to 372 products timed on an MI355X in every tile (32 to 4095
 // tokens by the widths of the layers and heads from 1536 to 49152, forward,
@@ -74,12 +74,12 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
   struct Cost {
     gemm::Tile t;
     int per_cu;
-    double launch, edge, step, part, least = 0;
+    double launch, edge, step, part, store = 0;
   };
-  // least (and the four steps a masked 256 x 256 tile always runs): 3848 x 2744
-  // x 24 takes 14 us on 256 x 256 tiles, 9.6 on 128 x 128 and 17 on 64 x 64, where
-  // the steps alone make 11, 8 and 7; gate|up of 2048 x 13952 x 64 40 / 26 / 43
-  static constexpr Cost kAlongK[] = {{gemm::k256, 1, 0.5, 9.5, 1.29, 0.82, 14.5},
+  // store, and the four steps a 256 x 256 tile always runs: 3848 x 2744 x 24 takes
+  // 14 us on 256 x 256 tiles, 9.6 on 128 x 128 and 17 on 64 x 64, where the steps
+  // alone make 11, 8 and 7; gate|up of 2048 x 13952 x 64 40 / 26 / 43
+  static constexpr Cost kAlongK[] = {{gemm::k256, 1, 0.5, 9.5, 1.29, 0.82},
                                      {gemm::k128x256, 1, 0.5, 5.5, 0.745, 0.72},
                                      {gemm::k128, 2, 4.7, 0.8, 0.926, 0.73, 3.6},
                                      {gemm::k128x2, 1, 0.0, 5.7, 0.59, 0.82},
@@ -105,8 +105,10 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     if (rem > 0)
       part = c[i].per_cu == 2 ? (rem <= cus ? c[i].part : 1.0)
                               : c[i].part + (1 - c[i].part) * static_cast<double>(rem) / cap;
-    const double round = c[i].edge + steps * c[i].step;
-    double us = c[i].launch + (round > c[i].least ? round : c[i].least) * (full + part);
+    const int64_t run = i == 0 && !a_km && steps < 4 ? 4 : steps;
+    double us = (c[i].edge + run * c[i].step) * (full + part);
+    const double stores = c[i].store * static_cast<double>(n) / cap;
+    us = c[i].launch + (us > stores ? us : stores);
     // a K-major A is a weight gradient, which runs beside the input-gradient
     // chain: the share of the chip it holds counts more than its own time
     // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone)
