@@ -54,8 +54,8 @@ def test_gemm_kernel_choice(lib):
     weight-gradient products -- and leading dimensions whose tiles stay within
     one buffer resource (2 GiB): 256 rows of a [rows, K] operand (ld < 2^22
     elements) or 64 rows of a K-major one (ld < 2^24).  Everything else --
-    ragged shapes, fp32, leading dimensions off 8 or past the bound -- runs
-    the masked kernel."""
+    ragged shapes, fp32, leading dimensions off 8 or past the bound -- is off
+    that grid."""
     TILED, GEN = 1, 0
     bf16, f32 = 2, 0
     path = lib.zk_gemm_path
@@ -521,7 +521,7 @@ def test_hf_factory_routes_structure():
     s = H.get_layers(mm)[0].spec
     assert (s.kv_heads, s.window, s.ffn, s.rope_theta) == (8, 4096, 14336, 1e4)
     assert H.get_layers(mm)[0].flat_param.numel() == 218_112_000
-    # the smaller llama_* models' head dims (padded around the attention kernels)
+    # the smaller llama_* models' head dims (on the ragged attention kernels)
     for name, d in (("llama_1b", 48), ("llama_2b", 68), ("llama_3b", 84), ("llama_4b", 98),
                     ("llama_5b", 110)):
         with torch.device("meta"):

@@ -217,10 +217,10 @@ def test_layer_every_product_hand_written(dev, name, transposed, monkeypatch):
     weight gradients dY^T X (o and down on the token-major dY, X as stored;
     gate|up and q|k|v on the dY^T the SwiGLU / attention backward kernels
     write from their epilogues, or with set_transposed_wgrad(False) on dY as
-    stored too) -- each on the
-    MFMA pipeline (zk_gemm_path "tiled"); no torch GEMM, no transpose pass
-    and no separate RoPE pass is called.  Parity against the fp64 oracle as
-    every layer test."""
+    stored too) -- each on the grid of the
+    MFMA pipeline (zk_gemm_path "tiled"), aligned operands that one of its tiles
+    takes; the layer calls no torch GEMM, no transpose pass and no RoPE pass of
+    its own.  Parity against the fp64 oracle as every layer test."""
     from zorse_amd import kernels as K
     from zorse_amd import layer as LY
     kw, window, dtype, (B, S) = HIP_GEMM[name]
@@ -892,8 +892,8 @@ def test_hf_mistral_route_layer_and_profiler_protocol(dev):
                                      (110, torch.bfloat16)])
 def test_layer_padded_head_dims(dev, d, dtype):
     """Head dims of the smaller llama_* HF-factory models (llama_1b: 48,
-    llama_2b: 68, llama_5b: 110), which the attention kernels take zero-padded
-    to 64 / 128: a 4-head layer (hidden 4 d, FFN 16 d, 2 x 96 tokens, GQA 4:2
+    llama_2b: 68, llama_5b: 110), which the ragged attention kernels take as
+    they lie: a 4-head layer (hidden 4 d, FFN 16 d, 2 x 96 tokens, GQA 4:2
     for d = 68) against the fp64 oracle with the precision-matched bar."""
     from zorse_amd import layer as LY
     kv = 2 if d == 68 else 4
@@ -905,3 +905,23 @@ def test_layer_padded_head_dims(dev, d, dtype):
     x = torch.randn(2, 96, 4 * d, generator=g).to(dtype)
     dout = torch.randn(2, 96, 4 * d, generator=g).to(dtype)
     _check_layer(layer, x, dout, dtype, f"padded head dim {d}")
+
+
+@pytest.mark.parametrize("d,dtype", [(16, torch.bfloat16), (32, torch.float16), (6, torch.bfloat16)])
+def test_layer_zero_padded_head_dims(dev, d, dtype, monkeypatch):
+    """Head dims up to 32 of 2-byte types, whose q, k, v, o and dO go through the
+    attention kernels zero-padded to 64: a 4-head layer (hidden 64, FFN 256, 2 x
+    96 tokens, GQA 4:2 for d = 32) against the fp64 oracle as above, with the
+    eight padded copies of a forward and a backward counted."""
+    from zorse_amd import layer as LY
+    kw = dict(hidden_size=64, num_attention_heads=4, num_key_value_heads=2 if d == 32 else 4,
+              head_dim=d, intermediate_size=256, rope_theta=1e4)
+    layer = _layer(kw, dev, param_dtype=dtype, seed=501 + d)
+    assert layer.spec.head_dim == d and LY._attn_padded_dim(layer.spec, dtype) == 64
+    padded, real = [], LY._pad_heads
+    monkeypatch.setattr(LY, "_pad_heads", lambda t, dp: padded.append(dp) or real(t, dp))
+    g = torch.Generator().manual_seed(502 + d)
+    x = torch.randn(2, 96, 64, generator=g).to(dtype)
+    dout = torch.randn(2, 96, 64, generator=g).to(dtype)
+    _check_layer(layer, x, dout, dtype, f"zero-padded head dim {d}")
+    assert padded and set(padded) == {64} and len(padded) % 8 == 0
