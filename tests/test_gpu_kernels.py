@@ -186,8 +186,9 @@ def _layout_operands(M, N, Kd, dtype, a_km, b_km, seed, dev, pad=0):
     return ad, bd, am, bm
 
 
-# (M, N, K): on the 256 x 256 grid (the tiled MFMA pipeline, one to 48 tiles,
-# 2 to 64 K steps) and off it (the masked kernel: ragged M, N and K)
+# (M, N, K): on the 256 x 256 grid (in whichever tile the rule picks; At_B, with
+# one form, always in the pipeline) and off it: ragged M, N and K, the last with
+# rows that are not 16-byte aligned (the general kernel)
 GEMM_SHAPES = [(256, 256, 256), (512, 768, 384), (768, 512, 1280), (1024, 2048, 4096),
                (300, 200, 72), (136, 520, 1000), (1, 7, 5)]
 
@@ -308,18 +309,17 @@ def _assert_z_of_gu(z, gu, F, dtype):
     assert (diff != 0).sum().item() <= max(1, z.numel() // 1000), "too many z elements differ"
 
 
-# B, S, K, Hq, Hkv, d, interleaved, explicit positions, dtype: the first two
-# and the 200-token ones take the GEMM's RoPE epilogue, the others the product
-# and the pass (off the 256 grid, rotated columns not whole 128-column blocks,
-# fp32, sequences under 128 tokens)
+# B, S, K, Hq, Hkv, d, interleaved, explicit positions, dtype: heads of 64 take
+# the RoPE epilogue (of the 64 x 64 tile; of the 128 x 256 one with 32 x 200
+# tokens, as the head of 128 there), the other heads of 128 and fp32 the product
+# and the pass; tests/test_gpu_gemm_tiles.py names every tile
 GEMM_ROPE_CASES = [
     (2, 256, 512, 4, 2, 128, False, False, torch.bfloat16),
     (1, 512, 256, 8, 4, 64, True, True, torch.float16),
     (2, 100, 192, 4, 2, 128, False, True, torch.bfloat16),
     (2, 128, 256, 2, 1, 64, False, False, torch.bfloat16),
     (1, 64, 128, 2, 2, 64, True, False, torch.float32),
-    # 64-token sequences: on the GEMM's grid, but below the epilogue's 128
-    # (the product and the pass)
+    # 64-token sequences: below the 128 that the 256-wide tiles' epilogue needs
     (4, 64, 256, 4, 2, 64, False, True, torch.bfloat16),
     # 200-token sequences: a wave's 128 rows cross a sequence boundary
     (32, 200, 256, 4, 2, 64, False, True, torch.bfloat16),
@@ -355,18 +355,18 @@ def test_gemm_rope_equals_gemm_then_rope(dev, case):
 
 @pytest.mark.parametrize("M,F,K,dtype", [(200, 72, 128, torch.bfloat16), (136, 200, 192, torch.float16),
                                           (8, 8, 64, torch.bfloat16), (1024, 704, 512, torch.bfloat16),
-                                          # the 256 x 256 pipeline (M % 256, F % 128, K % 128)
+                                          # on the 256 x 256 grid (M % 256, F % 128, K % 128)
                                           (256, 128, 256, torch.bfloat16),
                                           (512, 384, 512, torch.float16),
                                           (1024, 640, 1280, torch.bfloat16)])
 def test_gemm_swiglu(dev, M, F, K, dtype):
     """zk_gemm_swiglu (gate|up GEMM + SwiGLU epilogue) vs the fp64 oracle on
     the same rounded inputs: g, u within the bf16/fp16 bar; z bit-equal to the
-    SwiGLU kernel applied to the returned g, u on the 128 x 64 kernel (ragged
-    shapes), and within two ulps in at most 1 element in 10^3 on the 256 x 256
-    pipeline, whose epilogue takes silu from the hardware exp2 / reciprocal;
-    z^T an exact transpose; both dtypes."""
+    SwiGLU kernel applied to the returned g, u on every tile but the 256 x 256
+    pipeline on its grid, whose epilogue takes silu from the hardware exp2 /
+    reciprocal (the 7B shape below); z^T an exact transpose; both dtypes."""
     from zorse_amd import kernels as K_
+    from zorse_amd._abi import dtype_code, lib
     print(f"gemm_swiglu M={M} F={F} K={K} {dtype}", flush=True)
     x = _rand((M, K), dtype, 71)
     w = _rand((2 * F, K), dtype, 72, 0.05)
@@ -376,20 +376,21 @@ def test_gemm_swiglu(dev, M, F, K, dtype):
     assert_close(gu[:, :F], ref[:, :F], dtype, "g")
     assert_close(gu[:, F:], ref[:, F:], dtype, "u")
     assert_close(z, O.swiglu(ref[:, :F].to(dtype).double(), ref[:, F:].to(dtype).double()), dtype, "z")
-    if K_.gemm_nt_supported(M, 2 * F, K):
-        # the 256 x 256 pipeline's epilogue: hardware exp2 / reciprocal
-        _assert_z_of_gu(z, gu, F, dtype)
-    else:
-        # the 128 x 64 kernel: the SwiGLU kernel's IEEE form, bit for bit
-        assert torch.equal(z, K_.swiglu_fwd(gu[:, :F], gu[:, F:]))
+    assert K_.GEMM_TILES[lib().zk_gemm_swiglu_tile(M, F, K, K, K, 2 * F, dtype_code(dtype))] != "256"
+    # the SwiGLU kernel's IEEE form, bit for bit
+    assert torch.equal(z, K_.swiglu_fwd(gu[:, :F], gu[:, F:]))
     assert torch.equal(zt, z.t())
 
 
 def test_gemm_swiglu_llama7b_shape(dev):
     """The 7B layer shape (4096 tokens, F = 11008, K = 4096) against a plain
-    PyTorch fp32 GEMM of the same rounded inputs; the epilogue as above."""
+    PyTorch fp32 GEMM of the same rounded inputs; on the 256 x 256 pipeline, z
+    within two ulps in at most 1 element in 10^3."""
     from zorse_amd import kernels as K_
+    from zorse_amd._abi import dtype_code, lib
     M, F, K = 4096, 11008, 4096
+    assert K_.GEMM_TILES[lib().zk_gemm_swiglu_tile(M, F, K, K, K, 2 * F,
+                                                   dtype_code(torch.bfloat16))] == "256"
     g = torch.Generator(device="cpu").manual_seed(73)
     x = torch.randn(M, K, generator=g).to(dev, torch.bfloat16)
     w = (0.02 * torch.randn(2 * F, K, generator=g)).to(dev, torch.bfloat16)

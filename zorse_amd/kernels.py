@@ -320,12 +320,28 @@ def gemm_rope(x: torch.Tensor, w: torch.Tensor, *, seq_len: int, rot_cols: int, 
 
 def gemm_path(M: int, N: int, K: int, lda: int, ldb: int, ldc: int, dtype: torch.dtype,
               a_kmajor: bool = False, b_kmajor: bool = False, ldr: int = -1) -> str:
-    """Which kernel zk_gemm runs for a launch with 16-byte aligned pointers:
-    "tiled" (the 256 x 256 MFMA pipeline) or "general" (host-only query)."""
+    """Whether a launch with 16-byte aligned pointers lies on the grid of the
+    256 x 256 MFMA pipeline: "tiled" or "general" (host-only query; gemm_tile
+    names the kernel it runs)."""
     code = lib().zk_gemm_path(M, N, K, lda, int(a_kmajor), ldb, int(b_kmajor), ldc, ldr,
                               dtype_code(dtype))
     check(code if code < 0 else 0, "zk_gemm_path")
     return "tiled" if code == 1 else "general"
+
+
+# The kernels of a 2-byte or fp32 product, in the order of enum zk_gemm_tile_id:
+# "k2" tiles have eight waves, four on each half of a K step.
+GEMM_TILES = ("general", "256", "256 masked", "128x256", "128", "128 k2", "64", "64x128 k2")
+
+
+def gemm_tile(M: int, N: int, K: int, lda: int, ldb: int, ldc: int, dtype: torch.dtype,
+              a_kmajor: bool = False, b_kmajor: bool = False, ldr: int = -1) -> str:
+    """The kernel (of GEMM_TILES) zk_gemm runs for a launch with 16-byte aligned
+    pointers and no workspace (host-only query)."""
+    code = lib().zk_gemm_tile(M, N, K, lda, int(a_kmajor), ldb, int(b_kmajor), ldc, ldr,
+                              dtype_code(dtype))
+    check(code if code < 0 else 0, "zk_gemm_tile")
+    return GEMM_TILES[code]
 
 
 def gemm_nt(a: torch.Tensor, b: torch.Tensor, residual: torch.Tensor | None = None,
