@@ -171,8 +171,9 @@ int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
  * fused add: one fp32 rounding of the accumulated product plus r.  Any
  * shape; bf16 / fp16 (fp32 accumulation) or fp32; every tensor shares
  * `dtype`; pointers aligned to the element size.  2-byte products run the
- * MFMA tile (256 x 256 down to 64 x 64) with the least estimated time; fp32
- * and operands that are not 16-byte aligned run a masked 128 x 128 kernel. */
+ * MFMA tile (256 x 256 down to 64 x 64) with the least estimated time, fp32
+ * ones 128 x 128 or 64 x 64 tiles; operands whose rows are not 16-byte aligned
+ * (or sizes along them not multiples of 8) run a masked 128 x 128 kernel. */
 int zk_gemm(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
             int b_kmajor, void* c, int64_t ldc, const void* r, int64_t ldr, int64_t M,
             int64_t N, int64_t K, int dtype, zk_stream_t stream);
@@ -193,7 +194,8 @@ int zk_gemm_ws(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t 
  * of 256, K a multiple of 128 and at least 256, leading dimensions multiples
  * of 8, and each operand's tile within one buffer resource (lda / ldb below
  * 2^22 elements for a [rows, K] operand, 2^24 for a K-major one); otherwise
- * ZK_GEMM_GENERAL, a kernel with masked edges.  ldr < 0: no residual. */
+ * ZK_GEMM_GENERAL, off that grid: a masked or small tile, or the general
+ * kernel.  zk_gemm_tile names the kernel itself.  ldr < 0: no residual. */
 enum zk_gemm_kernel { ZK_GEMM_GENERAL = 0, ZK_GEMM_TILED = 1 };
 int zk_gemm_path(int64_t M, int64_t N, int64_t K, int64_t lda, int a_kmajor, int64_t ldb,
                  int b_kmajor, int64_t ldc, int64_t ldr, int dtype);

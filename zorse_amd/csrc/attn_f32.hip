@@ -21,7 +21,8 @@
 // Bound by latency at the sizes fp32 layers have (the parity layer's shape, 2
 // sequences x 4 heads x 128 x 64, is 16 workgroups).  There a thread per row
 // took 1770 us forward, 1955 us for dQ and 1976 us for dK / dV; these kernels
-// take 16, 26 and 31 us.
+// take 16, 26 and 31 us.  Many sequences of a few tokens are a thread per row's
+// still (by_rows).
 #include "attn_common.h"
 #include "vec.h"
 

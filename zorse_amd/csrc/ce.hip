@@ -15,8 +15,9 @@
 // one rescale for the 32 values) and the row reductions use wave shuffles plus
 // one LDS exchange.  Both passes are bound by HBM: 4096 rows of 49152 bf16
 // columns (403 MB) take 81 us forward with exp_neg, 103 with expf and 107 with
-// one access in flight besides, 76 with exp_neg's first line alone; 2046 rows
-// 66 us backward (402 MB).
+// one access in flight besides, 76 with exp_neg's first line alone (2046 rows
+// that the product has just left in the last-level cache 50, 40 with that); 2046
+// rows 66 us backward (402 MB).
 //
 // zk_ce_labels and zk_ce_finish are what precedes and follows the chunks, one
 // workgroup each: checked row labels, the number of valid rows and the initial

@@ -54,9 +54,11 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
 // storing a round's tiles takes.  Constants
 // in us, fitted to 372 products timed on an MI355X in every tile (32 to 4095
 // tokens by the widths of the layers and heads from 1536 to 49152, forward,
-// input- and weight-gradient layouts, weights not in any cache): over those
-// products the choice is on average 0.3 % and at most 15 % slower than the
-// best tile.  Examples, us on 256 / 128 / 128x2 / 64 / 64x128 tiles:
+// input- and weight-gradient layouts, weights not in any cache).  The choice by
+// these constants alone was on average 0.3 % and at most 15 % slower than the
+// best tile; that was without the 128 x 256 tile and `store`, fitted later to
+// products of their own, and without the two terms for weight gradients below,
+// which on purpose name a tile that is not the fastest by itself.  Examples, us on 256 / 128 / 128x2 / 64 / 64x128 tiles:
 //   128 x 2048 x 2048 NT       42 / 26 / 21 / 11.5 / 16      (64)
 //   512 x 4096 x 11008 dX     198 / 121 / 100 / 104 / 76     (64x128)
 //   2048 x 2048 x 5632 NT     105 / 67 / 57 / 85 / 81        (128x2)
@@ -111,7 +113,8 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     us = c[i].launch + (us > stores ? us : stores);
     // a K-major A is a weight gradient, which runs beside the input-gradient
     // chain: the share of the chip it holds counts more than its own time
-    // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone)
+    // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone; the
+    // line between 0.15 and 1 rests on that stage)
     if (a_km && n < cus) us *= 0.15 + 0.85 * static_cast<double>(n) / cus;
     // and one of two rounds of 256 x 256 or more stays on those unless a smaller
     // tile is clearly ahead: twice the operand reads and a stream of short
@@ -121,7 +124,7 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     // us, of the 14336-wide grouped-query layer, 1527 tokens, 2382 / 2350.  Below
     // two rounds the smaller tile's own time decides (1B grouped-query layer, 1024
     // tokens, 680 against 705 us), as it does more than 8 % ahead (7B, 512 tokens,
-    // 908 against 925).
+    // 908 against 925 with 20 % or no small tiles at all).
     if (a_km && i > 0 && tiles256 >= 2 * cus) us *= 1.08;
     if (i == 0 || us < best_us) {
       best = c[i].t;
@@ -134,8 +137,9 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
 
 // Splitting the reduction over workgroups (gemm_split.hip): `parts` ranges of
 // split_k on tiles of at most one workgroup per CU, when the estimate of the
-// rule above for tiles and parts, plus the sum over the parts (5 us with its
-// launch, and 8 bytes an output and part at 3.5 TB/s), is 11 us below that of
+// rule above for tiles and parts, plus the partial sums (5 us for the second
+// launch, and 8 bytes an output and part, stored by one and read by the other, at
+// 3.5 TB/s), is 11 us below that of
 // the best single pass: a layer whose products are that short is bound by the
 // host, whom the workspace and the second launch cost 7 us (a forward of the
 // 2048-wide layer at 128 tokens: 112 us, 121 with its down product split, 22

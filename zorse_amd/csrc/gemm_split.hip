@@ -5,7 +5,9 @@
 //
 // Bound: a CU takes in its tiles' operands at about 55 GB/s, so a product with
 // 32 tiles runs at an eighth of what 256 workgroups load; the partial sums cost
-// 8 bytes an output and part, and the sum's launch 3 us.
+// 8 bytes an output and part.  The second launch takes 3.8 us for 64 x 4096 in 8
+// parts, 5.0 for 256 x 4096 in 4, 9.7 for 1024 x 2688 in 5 and 10.9 for 2046 x
+// 1536 in 5 (63 MB read, 5.8 TB/s), with no gap before it.
 #include "gemm_ring.h"
 
 namespace zk {

@@ -186,7 +186,9 @@ _side_streams: dict = {}
 
 # A layer backward with less work than this keeps them in order too: its
 # kernels are shorter than the host takes to enqueue them, and the three
-# cross-stream waits cost the host 15 us each.  Forward + backward, side
+# cross-stream waits cost the host 15 us each -- also with set_wgrad_stream(True),
+# which sets what larger ones do.  The line lies where one host (the times are
+# its Python's) broke even.  Forward + backward, side
 # stream / in order: tiny shape at 256 tokens (0.5e11) 620 / 470 us, at 512
 # (1.0e11) 460 / 397, at 1024 (2.1e11) 647 / 623, at 2048 (4.2e11) 935 / 994;
 # 1B grouped-query at 512 (1.2e11) 620 / 485, at 1024 (2.5e11) 744 / 772; 7B at
@@ -195,8 +197,9 @@ SIDE_STREAM_FLOPS = 2.2e11
 
 
 def set_wgrad_stream(enable: bool) -> bool:
-    """Run the weight-gradient GEMMs on a side stream (True) or in order on the
-    compute stream; returns the previous setting."""
+    """Run the o and down weight-gradient GEMMs on a side stream, for layer
+    backwards of at least SIDE_STREAM_FLOPS (True), or all in order on the
+    compute stream (False); returns the previous setting."""
     global _wgrad_side
     prev, _wgrad_side = _wgrad_side, bool(enable)
     return prev
@@ -238,8 +241,10 @@ class _WeightGrads:
 # writes g, u and z in one pass) for 2-byte types; otherwise the GEMM and a
 # separate SwiGLU pass.  On by default: in the 7B stage it measured equal to
 # the GEMM plus the SwiGLU pass; ZORSE_FUSED_MLP=0 or set_fused_gate_up(False)
-# turns it off (the separate pass computes SiLU with the IEEE exp and
-# division, the fused epilogue with the hardware exp2 and reciprocal).
+# turns it off.  The separate pass and every masked or small tile's epilogue
+# compute SiLU with the IEEE exp and division, the 256 x 256 tile on its grid with
+# the hardware exp2 and reciprocal -- so which of the two a product's z has
+# depends on the tile its shape gets (kernels.GEMM_TILES).
 _fused_gate_up = os.environ.get("ZORSE_FUSED_MLP", "1") != "0"
 
 
