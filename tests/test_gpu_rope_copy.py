@@ -25,3 +25,14 @@ def test_rope_copy(dev, B, S, Hq, Hkv, d, dtype, inter, off):
     K.rope_(qr, kr, cos, sin, interleaved=inter)
     assert torch.equal(qo, qr) and torch.equal(ko, kr) and torch.equal(buf, before)
     assert qo.is_contiguous() and ko.is_contiguous()
+
+
+@pytest.mark.parametrize("shape", [(0, 4, 2, 64), (2, 0, 2, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rope_copy_refuses_empty_tensors(dev, shape, dtype):
+    """As rope_ does, whatever the kernel: no position to rotate is an error."""
+    from zorse_amd import kernels as K
+    q = torch.zeros(shape, device=dev, dtype=dtype)
+    cos = torch.ones(4, shape[3] // 2, device=dev)
+    with pytest.raises(RuntimeError, match="zk_rope"):
+        K.rope_copy(q, q, cos, cos)

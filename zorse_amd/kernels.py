@@ -492,7 +492,8 @@ def rope_copy(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Te
               interleaved: bool = False):
     """Rotated contiguous copies of q [B,S,Hq,d] and k [B,S,Hkv,d], positions
     0 .. S-1: in one pass (zk_rope_copy) for head dims 64 and 128 of 2-byte
-    types with 16-byte aligned rows, else copies rotated in place."""
+    types with 16-byte aligned rows, else copies rotated in place (which refuses
+    empty tensors)."""
     dev = _require_gpu(q, k, cos, sin)
     if q.dim() == 4 and k.dim() == 4 and q.dtype in _LOWP and k.dtype == q.dtype:
         B, S, Hq, d = q.shape
@@ -500,7 +501,7 @@ def rope_copy(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Te
         if k.shape[:2] == (B, S) and k.shape[3] == d and d in (64, 128) and qu == ku == 1 \
                 and (qb | qs | qh | kb | ks | kh) % 8 == 0 \
                 and (q.data_ptr() | k.data_ptr() | cos.data_ptr() | sin.data_ptr()) % 16 == 0 \
-                and 0 < Hq and 0 < k.shape[2] and Hq + k.shape[2] < 65536 and B < 65536 \
+                and q.numel() and k.numel() and Hq + k.shape[2] < 65536 and B < 65536 \
                 and cos.shape == sin.shape == (cos.shape[0], d // 2) and cos.shape[0] >= S \
                 and cos.dtype == sin.dtype == torch.float32 \
                 and cos.is_contiguous() and sin.is_contiguous():
