@@ -26,3 +26,15 @@ def test_in_order_and_side_stream_agree(monkeypatch, tokens, strided):
         got.append((out.detach(), xr.grad, fr.grad))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("missing", [8, 128 + 8])
+def test_flat_parameter_too_short(missing):
+    """A flat parameter that ends inside the norm weights is the kernels'
+    ValueError about the weight's shape."""
+    import zorse_amd.layer as L
+    spec = L.LayerSpec(hidden=128, heads=2, kv_heads=1, head_dim=64, ffn=256)
+    flat = torch.zeros(spec.numel - missing, device="cuda", dtype=torch.bfloat16)
+    x = torch.zeros(1, 16, 128, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="weight shape"):
+        L.DecoderLayerFunction.apply(x, flat, spec, None)

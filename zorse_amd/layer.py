@@ -101,7 +101,8 @@ class FlatViews:
                 setattr(self, name, flat.as_strided(shape, strides, base + off))
         else:  # strided, or too short for its layer: view and the kernels' checks say so
             for name, shape, _, off in spec.view_specs:
-                setattr(self, name, flat[off:off + math.prod(shape)].view(shape))
+                part = flat[off:off + math.prod(shape)]
+                setattr(self, name, part if len(shape) == 1 else part.view(shape))
 
 
 # Every projection product runs on the hand-written GEMMs (zk_gemm) with the
