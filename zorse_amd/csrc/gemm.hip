@@ -114,8 +114,11 @@ static gemm::Tile pick_tile(int64_t M, int64_t N, int64_t K, bool a_km, bool b_k
     // a K-major A is a weight gradient, which runs beside the input-gradient
     // chain: the share of the chip it holds counts more than its own time
     // (a stage of 2048-wide layers 4.29 ms this way, 4.37 by time alone; the
-    // line between 0.15 and 1 rests on that stage)
-    if (a_km && n < cus) us *= 0.15 + 0.85 * static_cast<double>(n) / cus;
+    // line between 0.15 and 1 rests on that stage).  Layers of fewer tokens, K,
+    // mostly run it in order, where its own time counts: 2048 x 2048 x 48 on 128 x
+    // 128 tiles 7.3 us, on 256 x 256, which the share would name, 14.2; x 512 9.5 and
+    // 16.9; a 2B layer of 512 tokens 513, with the share 530.
+    if (a_km && n < cus && K >= 1024) us *= 0.15 + 0.85 * static_cast<double>(n) / cus;
     // and one of two rounds of 256 x 256 or more stays on those unless a smaller
     // tile is clearly ahead: twice the operand reads and a stream of short
     // workgroups slow the chain beside it.  5120 x 13824 x 2048: 495 us on 128 x
