@@ -444,8 +444,8 @@ int zk_ce_labels(const int64_t* labels, int64_t rows, int64_t vocab, int64_t ign
                  int64_t* row_label, float* run_max, float* run_sum, float* target_logit,
                  int64_t* stats, int64_t* host_stats, zk_stream_t stream);
 /* After the last: lse per row and loss = sum of (lse - target_logit) over the
- * labelled rows / max(stats[0], 1). */
-int zk_ce_finish(const int64_t* row_label, int64_t rows, const float* run_max,
+ * labelled rows / max(stats[0], 1).  run_max is scratch afterwards. */
+int zk_ce_finish(const int64_t* row_label, int64_t rows, float* run_max,
                  const float* run_sum, const float* target_logit, const int64_t* stats,
                  float* lse, float* loss, zk_stream_t stream);
 

@@ -20,7 +20,7 @@
 // rows 66 us backward (402 MB).
 //
 // zk_ce_labels and zk_ce_finish are what precedes and follows the chunks, one
-// workgroup each: checked row labels, the number of valid rows and the initial
+// workgroup each up to kOneGroup rows: checked row labels, the number of valid rows and the initial
 // accumulators; the rows' log-sum-exp and the mean loss.  As tensor operations
 // they were 30 launches of 2 to 5 us and two waits of the host for the device (a
 // head of 2046 tokens, 1536 wide, 49152 columns: 1098 us against 931).  One wait
@@ -175,13 +175,20 @@ __device__ __forceinline__ U block_sum_1024(U x, U* red) {
   return t;
 }
 
+// One workgroup moves 80 GB/s: 262144 rows took 94 us for the labels, 11 this way.
+// More rows than the two ways take alike go to a workgroup per kGroupRows and a
+// second launch for the totals (integer counts; float sums in the groups' order).
+constexpr int64_t kOneGroup = 16384, kGroupRows = 4096;
+
 __global__ __launch_bounds__(1024) void ce_labels_kernel(
     const int64_t* __restrict__ labels, int64_t rows, int64_t vocab, int64_t ignore,
     int64_t* __restrict__ row_label, float* __restrict__ run_max, float* __restrict__ run_sum,
     float* __restrict__ target, int64_t* __restrict__ stats, int64_t* __restrict__ host_stats) {
   __shared__ int red[16];
   int valid = 0, bad = 0;
-  for (int64_t i = threadIdx.x; i < rows; i += 1024) {
+  const int64_t first = blockIdx.x * kGroupRows;
+  const int64_t end = gridDim.x == 1 || first + kGroupRows > rows ? rows : first + kGroupRows;
+  for (int64_t i = first + threadIdx.x; i < end; i += 1024) {
     const int64_t l = labels[i];
     const bool skip = l == ignore;
     valid += !skip;
@@ -193,7 +200,10 @@ __global__ __launch_bounds__(1024) void ce_labels_kernel(
   }
   valid = block_sum_1024(valid, red);
   bad = block_sum_1024(bad, red);
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && gridDim.x > 1) {
+    atomicAdd(reinterpret_cast<unsigned long long*>(stats), static_cast<unsigned long long>(valid));
+    atomicAdd(reinterpret_cast<unsigned long long*>(stats + 1), static_cast<unsigned long long>(bad));
+  } else if (threadIdx.x == 0) {
     stats[0] = valid;
     stats[1] = bad;
     host_stats[0] = valid;
@@ -201,19 +211,49 @@ __global__ __launch_bounds__(1024) void ce_labels_kernel(
   }
 }
 
+// stats = {0, 0}, or its copy to the host.
+__global__ void ce_stats_kernel(int64_t* stats, int64_t* host_stats) {
+  if (host_stats == nullptr)
+    stats[threadIdx.x] = 0;
+  else
+    host_stats[threadIdx.x] = stats[threadIdx.x];
+}
+
+// A workgroup of several leaves its sum in run_max at its first row.
 __global__ __launch_bounds__(1024) void ce_finish_kernel(
-    const int64_t* __restrict__ row_label, int64_t rows, const float* __restrict__ run_max,
+    const int64_t* __restrict__ row_label, int64_t rows, float* run_max,
     const float* __restrict__ run_sum, const float* __restrict__ target,
     const int64_t* __restrict__ stats, float* __restrict__ lse, float* __restrict__ loss) {
   __shared__ float red[16];
   float sum = 0.f;
-  for (int64_t i = threadIdx.x; i < rows; i += 1024) {
+  const int64_t first = blockIdx.x * kGroupRows;
+  const int64_t end = gridDim.x == 1 || first + kGroupRows > rows ? rows : first + kGroupRows;
+  for (int64_t i = first + threadIdx.x; i < end; i += 1024) {
     const float l = run_max[i] + logf(run_sum[i]);
     lse[i] = l;
     if (row_label[i] >= 0) sum += l - target[i];
   }
+  sum = block_sum_1024(sum, red);  // (its barriers: every row is read)
+  if (threadIdx.x != 0) return;
+  if (gridDim.x > 1)
+    run_max[first] = sum;
+  else
+    *loss = sum / static_cast<float>(stats[0] > 1 ? stats[0] : 1);
+}
+
+__global__ __launch_bounds__(1024) void ce_mean_kernel(const float* __restrict__ run_max,
+                                                       int64_t groups,
+                                                       const int64_t* __restrict__ stats,
+                                                       float* __restrict__ loss) {
+  __shared__ float red[16];
+  float sum = 0.f;
+  for (int64_t i = threadIdx.x; i < groups; i += 1024) sum += run_max[i * kGroupRows];
   sum = block_sum_1024(sum, red);
   if (threadIdx.x == 0) *loss = sum / static_cast<float>(stats[0] > 1 ? stats[0] : 1);
+}
+
+static unsigned row_groups(int64_t rows) {
+  return rows <= kOneGroup ? 1 : static_cast<unsigned>((rows + kGroupRows - 1) / kGroupRows);
 }
 
 }  // namespace zk
@@ -228,20 +268,29 @@ extern "C" int zk_ce_labels(const int64_t* labels, int64_t rows, int64_t vocab, 
   ZK_REQUIRE(stats && host_stats &&
                  (rows == 0 || (labels && row_label && run_max && run_sum && target_logit)),
              ZK_EINVAL, "zk_ce_labels: null pointer");
-  hipLaunchKernelGGL(ce_labels_kernel, dim3(1), dim3(1024), 0, as_stream(stream), labels, rows,
-                     vocab, ignore_index, row_label, run_max, run_sum, target_logit, stats,
-                     host_stats);
+  hipStream_t s = as_stream(stream);
+  const unsigned groups = row_groups(rows);
+  int64_t* const none = nullptr;
+  if (groups > 1) hipLaunchKernelGGL(ce_stats_kernel, dim3(1), dim3(2), 0, s, stats, none);
+  hipLaunchKernelGGL(ce_labels_kernel, dim3(groups), dim3(1024), 0, s, labels, rows, vocab,
+                     ignore_index, row_label, run_max, run_sum, target_logit, stats, host_stats);
+  if (groups > 1) hipLaunchKernelGGL(ce_stats_kernel, dim3(1), dim3(2), 0, s, stats, host_stats);
   return launch_status("zk_ce_labels");
 }
 
-extern "C" int zk_ce_finish(const int64_t* row_label, int64_t rows, const float* run_max,
+extern "C" int zk_ce_finish(const int64_t* row_label, int64_t rows, float* run_max,
                             const float* run_sum, const float* target_logit,
                             const int64_t* stats, float* lse, float* loss, zk_stream_t stream) {
   ZK_REQUIRE(rows >= 0 && rows <= 0x7fffffff, ZK_EINVAL, "zk_ce_finish: bad shape");
   ZK_REQUIRE(stats && loss && (rows == 0 || (row_label && run_max && run_sum && target_logit && lse)),
              ZK_EINVAL, "zk_ce_finish: null pointer");
-  hipLaunchKernelGGL(ce_finish_kernel, dim3(1), dim3(1024), 0, as_stream(stream), row_label, rows,
-                     run_max, run_sum, target_logit, stats, lse, loss);
+  hipStream_t s = as_stream(stream);
+  const unsigned groups = row_groups(rows);
+  hipLaunchKernelGGL(ce_finish_kernel, dim3(groups), dim3(1024), 0, s, row_label, rows, run_max,
+                     run_sum, target_logit, stats, lse, loss);
+  if (groups > 1)
+    hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(1024), 0, s, run_max,
+                       static_cast<int64_t>(groups), stats, loss);
   return launch_status("zk_ce_finish");
 }
 
