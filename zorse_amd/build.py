@@ -47,8 +47,8 @@ HIPCC_FLAGS = [
 # of them between AGPRs per pass; the NT forms do better with the default).
 _KMAJOR = ["-Wno-inline-asm", "-mllvm", "-greedy-reverse-local-assignment=1"]
 FILE_FLAGS = {"rope.hip": ["-fno-slp-vectorize"], "gemm.hip": ["-Wno-inline-asm"],
-              "gemm_ring.hip": ["-Wno-inline-asm"], "gemm_split.hip": ["-Wno-inline-asm"], "gemm_f32.hip": ["-Wno-inline-asm"],
-              "gemm_kmajor.hip": _KMAJOR,
+              "gemm_ring.hip": ["-Wno-inline-asm"], "gemm_split.hip": ["-Wno-inline-asm"],
+              "gemm_f32.hip": ["-Wno-inline-asm"], "gemm_kmajor.hip": _KMAJOR,
               "gemm_ring_kmajor.hip": _KMAJOR}
 
 

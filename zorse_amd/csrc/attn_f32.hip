@@ -221,8 +221,8 @@ __device__ __forceinline__ int64_t group_id() {
   return static_cast<int64_t>(blockIdx.y) * kGridX + blockIdx.x;
 }
 dim3 group_grid(int64_t n) {
-  return n <= kGridX ? dim3(static_cast<unsigned>(n))
-                     : dim3(static_cast<unsigned>(kGridX), static_cast<unsigned>((n + kGridX - 1) / kGridX));
+  if (n <= kGridX) return dim3(static_cast<unsigned>(n));
+  return dim3(static_cast<unsigned>(kGridX), static_cast<unsigned>((n + kGridX - 1) / kGridX));
 }
 
 template <int D, bool kVec>

@@ -201,8 +201,9 @@ __global__ __launch_bounds__(1024) void ce_labels_kernel(
   valid = block_sum_1024(valid, red);
   bad = block_sum_1024(bad, red);
   if (threadIdx.x == 0 && gridDim.x > 1) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(stats), static_cast<unsigned long long>(valid));
-    atomicAdd(reinterpret_cast<unsigned long long*>(stats + 1), static_cast<unsigned long long>(bad));
+    unsigned long long* const total = reinterpret_cast<unsigned long long*>(stats);
+    atomicAdd(total, static_cast<unsigned long long>(valid));
+    atomicAdd(total + 1, static_cast<unsigned long long>(bad));
   } else if (threadIdx.x == 0) {
     stats[0] = valid;
     stats[1] = bad;

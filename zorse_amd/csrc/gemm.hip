@@ -58,7 +58,8 @@ static bool masked_takes(int64_t M, int64_t N, int64_t K, int64_t lda, int a_km,
 // these constants alone was on average 0.3 % and at most 15 % slower than the
 // best tile; that was without the 128 x 256 tile and `store`, fitted later to
 // products of their own, and without the two terms for weight gradients below,
-// which on purpose name a tile that is not the fastest by itself.  Examples, us on 256 / 128 / 128x2 / 64 / 64x128 tiles:
+// which on purpose name a tile that is not the fastest by itself.  Examples, us
+// on 256 / 128 / 128x2 / 64 / 64x128 tiles:
 //   128 x 2048 x 2048 NT       42 / 26 / 21 / 11.5 / 16      (64)
 //   512 x 4096 x 11008 dX     198 / 121 / 100 / 104 / 76     (64x128)
 //   2048 x 2048 x 5632 NT     105 / 67 / 57 / 85 / 81        (128x2)
@@ -533,8 +534,8 @@ extern "C" int zk_gemm_swiglu(const void* x, int64_t ld_x, const void* w_gate,
     if (rc != ZK_OK) return rc;
     rc = zk_gemm(x, ld_x, 0, w_up, ld_w, 0, u_out, ld_gu, nullptr, 0, M, F, K, dtype, stream);
     if (rc != ZK_OK) return rc;
-    return zt != nullptr ? zk_swiglu_fwd_t(g_out, u_out, ld_gu, z, ld_z, zt, ld_zt, M, F, dtype, stream)
-                         : zk_swiglu_fwd(g_out, u_out, ld_gu, z, ld_z, M, F, dtype, stream);
+    if (zt == nullptr) return zk_swiglu_fwd(g_out, u_out, ld_gu, z, ld_z, M, F, dtype, stream);
+    return zk_swiglu_fwd_t(g_out, u_out, ld_gu, z, ld_z, zt, ld_zt, M, F, dtype, stream);
   }
   gemm::GemmArgs ga{};
   ga.a = x;

@@ -1,9 +1,10 @@
-// The small-tile MFMA GEMM for bf16 / fp16 and fp32, any M, N and K:
+// The small-tile MFMA GEMM for bf16 / fp16 and fp32, M, N and K off every grid
+// but the 8 elements of a load or store (masked_takes in gemm.hip):
 //
 //   C[M, N] = op(A) op(B)^T (+ R[M, N])
 //
-// with the operand layouts and rounding of gemm_kernels.h.  It takes what the 256 x 256 pipeline is too
-// coarse for: few tokens, widths off the 256 grid, token counts off every
+// with the operand layouts and rounding of gemm_kernels.h.  It takes what the
+// 256 x 256 pipeline is too coarse for: few tokens, widths off the 256 grid, token counts off every
 // grid, and products whose large tiles would leave CUs idle.
 //
 // Workgroup = 4 waves in a 2 x 2 arrangement over a tile of 32 MB x 32 NB,
@@ -154,7 +155,8 @@ __device__ __forceinline__ typename RingOp<T>::vec kmaj_operand_n(const T* tile,
 template <typename T, int EPI, bool AKM, bool BKM, int MB, int NB, int RB, int WPE, int KS>
 __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void gemm_ring_kernel(GemmArgs args) {
-  static_assert(EPI == 0 || (EPI == 3 && !AKM) || (!AKM && !BKM), "the SwiGLU and RoPE epilogues take NT operands");
+  static_assert(EPI == 0 || (EPI == 3 && !AKM) || (!AKM && !BKM),
+                "the SwiGLU and RoPE epilogues take NT operands");
   constexpr int TBM = 32 * MB, TBN = 32 * NB, WR = 16 * MB, WC = 16 * NB;
   typedef RingOp<T> Mm;
   typedef typename Mm::vec V8;
@@ -205,7 +207,7 @@ void gemm_ring_kernel(GemmArgs args) {
   TA ta;
   TB tb;
   ta.init(lda);
-  static_assert(EPI != 1 || TB::NI % 2 == 0, "gate and up rows are loaded by instructions of their own");
+  static_assert(EPI != 1 || TB::NI % 2 == 0, "gate and up rows: instructions of their own");
   tb.init(ldb);
   const uint32_t lds_a = lds_addr(As), lds_b = lds_addr(Bs);
   f32x4 acc[MB][NB];

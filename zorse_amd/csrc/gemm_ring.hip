@@ -9,9 +9,9 @@ namespace {
 template <typename T, int EPI>
 void launch_t(Tile t, const GemmArgs& ga, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(tile_count(t, ga.M, ga.N)));
-#define ZK_RING(MB, NB, RB, WPE, KS)                                                            \
-  hipLaunchKernelGGL((gemm_ring_kernel<T, EPI, false, false, MB, NB, RB, WPE, KS>), grid, dim3(256 * KS), 0, \
-                     s, ga)
+#define ZK_RING(MB, NB, RB, WPE, KS)                                                       \
+  hipLaunchKernelGGL((gemm_ring_kernel<T, EPI, false, false, MB, NB, RB, WPE, KS>), grid, \
+                     dim3(256 * KS), 0, s, ga)
   if (t == k64)
     ZK_RING(2, 2, 4, 2, 1);
   else if (t == k64x128)

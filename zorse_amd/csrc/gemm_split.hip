@@ -20,9 +20,11 @@ void launch_t(Tile t, int parts, const GemmArgs& ga, hipStream_t s) {
   if (t == k256)
     hipLaunchKernelGGL((gemm_tiled_kernel<T, 3, false, BKM, true>), grid, dim3(256), 0, s, ga);
   else if (t == k128x2)
-    hipLaunchKernelGGL((gemm_ring_kernel<T, 3, false, BKM, 4, 4, 4, 2, 2>), grid, dim3(512), 0, s, ga);
+    hipLaunchKernelGGL((gemm_ring_kernel<T, 3, false, BKM, 4, 4, 4, 2, 2>), grid, dim3(512), 0, s,
+                       ga);
   else
-    hipLaunchKernelGGL((gemm_ring_kernel<T, 3, false, BKM, 2, 4, 4, 2, 2>), grid, dim3(512), 0, s, ga);
+    hipLaunchKernelGGL((gemm_ring_kernel<T, 3, false, BKM, 2, 4, 4, 2, 2>), grid, dim3(512), 0, s,
+                       ga);
 }
 
 // Four columns a thread; N is a multiple of 8 and rows 16-byte aligned.
@@ -58,9 +60,15 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
 
 void launch_split(bool bf16_, bool b_kmajor, Tile t, int parts, const GemmArgs& ga, hipStream_t s) {
   if (bf16_) {
-    if (b_kmajor) launch_t<bf16, true>(t, parts, ga, s); else launch_t<bf16, false>(t, parts, ga, s);
+    if (b_kmajor)
+      launch_t<bf16, true>(t, parts, ga, s);
+    else
+      launch_t<bf16, false>(t, parts, ga, s);
   } else {
-    if (b_kmajor) launch_t<f16, true>(t, parts, ga, s); else launch_t<f16, false>(t, parts, ga, s);
+    if (b_kmajor)
+      launch_t<f16, true>(t, parts, ga, s);
+    else
+      launch_t<f16, false>(t, parts, ga, s);
   }
 }
 
