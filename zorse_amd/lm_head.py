@@ -122,8 +122,8 @@ class LMHeadCrossEntropyFunction(torch.autograd.Function):
 # Default chunking: the whole vocabulary in one chunk (logits kept for the
 # backward) while the [tokens, vocab] logits take at most this many bytes,
 # else chunks of 8192 columns.  Measured at 4096 tokens, hidden 4096, vocab
-# 49152 (403 MB of bf16 logits), fwd + bwd: 3.85 ms in one chunk, 5.11 ms in
-# 8192-column chunks, 5.40 ms for F.linear + F.cross_entropy.
+# 49152 (403 MB of bf16 logits), fwd + bwd: 3.77 ms in one chunk, 5.04 ms in
+# 8192-column chunks, 5.38 ms for F.linear + F.cross_entropy.
 SINGLE_CHUNK_BYTES = 1 << 30
 
 
